@@ -6,16 +6,16 @@
 //       - sum_{near pairs} sum_{j in patch} K(x_i,y_j) s_j (subtraction, :1156-1193)
 // with s_j = sigma_over_j * whtsover_j and K the combined kernel (alpha S + beta D).
 //
-// The FMM is replaced by a tiled all-pairs sum: 256 targets per workgroup, source tiles
-// staged in LDS.  Two modes:
-//   ADDSUB : all sources, then an explicit subtraction kernel (the reference's algebra);
-//   MASKED : sources of the target's near patches are skipped inside the tiled sum
+// The FMM is replaced by an all-pairs sum, one density on the vector units (k_farsum) and
+// blocks of densities on the matrix cores (k_farsum_mfma).  Two modes:
+//   ADDSUB : all sources, then the near patches' contributions subtracted (the reference's
+//            algebra);
+//   MASKED : sources of the target's near patches are skipped inside the sum
 //            (algebraically identical, no cancellation; used for FP32).
 // Sources are sorted by patch, so the near-patch test is a moving pointer into the
 // target's sorted near list.  Sources with |x-y| <= thresh are skipped in every sum
 // (get_fmm_thresh, src/common/get_fmm_thresh.f:81).
-// Laplace runs through the same code with k = 0 and real densities (the kernel then
-// reduces exactly to (beta d/r^3 + alpha/r)/(4 pi)).
+// Laplace densities may be complex too: a real kernel applied to both parts.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -39,375 +39,426 @@ struct V2 {
   T x, y;
 };
 
-// sigma_over = I * sigma per patch; strengths q = alpha*s, m = beta*s, s = sigma_over*w.
+// Source geometry record: x, y, z, nx, ny, nz (FP32: padded to 32 bytes).
 template <typename T>
+constexpr int GEO = sizeof(T) == 8 ? 6 : 8;
+
+// Right-hand sides of a group on the matrix cores.
+constexpr int MG = 16;
+
+// Strengths of the far sum: sigma_over = I * sigma per patch, s = phase * sigma_over * w,
+// one complex value per oversampled node and right-hand side, stored by groups of nr
+// right-hand sides: group g, node i, right-hand side r of the group at (g nptso + i) nr + r.
+// Right-hand sides from nrhs to the end of the last group are zero.
+// A thread takes RB right-hand sides of one node (grid y).
+template <typename T, int RB>
 __global__ void k_oversample(int64_t nptso, const int* __restrict__ opatch, const int64_t* __restrict__ ixyzs,
                              const int64_t* __restrict__ ixyzso, const int64_t* __restrict__ ioff,
                              const int* __restrict__ np_of, const double* __restrict__ imat,
                              const V2<T>* __restrict__ sigma, int nrhs, int64_t ldsig,
-                             const T* __restrict__ wover, double ar, double ai, double br, double bi,
-                             V2<T>* __restrict__ qstr, V2<T>* __restrict__ mstr, int64_t ldstr) {
+                             const T* __restrict__ wover, double pr, double pi, int nr, V2<T>* __restrict__ str) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= nptso) return;
+  const int r0 = blockIdx.y * RB;
   const int ip = opatch[i];
   const int p = np_of[ip];
   const int64_t li = i - (ixyzso[ip] - 1);
   const double* row = imat + ioff[ip] + li * p;
   const int64_t s0 = ixyzs[ip] - 1;
   const double w = (double)wover[i];
-  for (int r = 0; r < nrhs; r++) {
-    const V2<T>* sg = sigma + r * ldsig + s0;
-    double sr = 0.0, si = 0.0;
-    for (int l = 0; l < p; l++) {
-      sr = fma(row[l], (double)sg[l].x, sr);
-      si = fma(row[l], (double)sg[l].y, si);
+  double sr[RB], si[RB];
+  const V2<T>* sg[RB];
+#pragma unroll
+  for (int r = 0; r < RB; r++) {
+    sr[r] = si[r] = 0.0;
+    sg[r] = sigma + (int64_t)(r0 + r < nrhs ? r0 + r : 0) * ldsig + s0;
+  }
+  for (int l = 0; l < p; l++) {
+    const double c = row[l];
+#pragma unroll
+    for (int r = 0; r < RB; r++) {
+      const V2<T> v = sg[r][l];
+      sr[r] = fma(c, (double)v.x, sr[r]);
+      si[r] = fma(c, (double)v.y, si[r]);
     }
-    sr *= w;
-    si *= w;
-    qstr[r * ldstr + i] = {(T)(ar * sr - ai * si), (T)(ar * si + ai * sr)};
-    mstr[r * ldstr + i] = {(T)(br * sr - bi * si), (T)(br * si + bi * sr)};
+  }
+  const int g = r0 / nr;
+  V2<T>* o = str + ((int64_t)g * nptso + i) * nr + (r0 - g * nr);
+#pragma unroll
+  for (int r = 0; r < RB; r++) {
+    const double a = sr[r] * w, b = si[r] * w;
+    const bool live = r0 + r < nrhs;
+    o[r] = {live ? (T)(pr * a - pi * b) : (T)0, live ? (T)(pr * b + pi * a) : (T)0};
   }
 }
 
-// 16-byte LDS word of T values (4 floats or 2 doubles)
+// ---- kernel values of the far sum
+// The combined kernel is K = (alpha + beta t (1 - ikr)) e^{ikr} / (4 pi r), t = (x - y).n / r^2.
+// The plan factors it as phase * (a + t' (1 - ikr)) e^{ikr} / r with |a| <= 1 and the source
+// normals scaled (apply_plan_scale): one complex strength per node instead of a charge and a
+// dipole, and G = a + t' (1 - ikr) takes two fused multiply-adds.
+// KIND 0: k = 0 (Laplace): a real kernel, no sine and cosine.  KIND 1: real wavenumber.  KIND
+// 2: complex wavenumber, or (FP32) phases beyond the hardware sine's range, which are
+// reduced to one revolution first; otherwise the FP32 phase k r / (2 pi) goes to the hardware
+// sine and cosine directly (they take revolutions, valid below 256, which the plan checks
+// against its bounding box): with KIND 1 the FP32 coordinates are stored in units of the
+// wavelength (scaled before they are rounded to FP32), so that r is the phase.
 template <typename T>
-struct Word16;
-template <>
-struct Word16<float> {
-  using type = float4;
-  static __device__ __forceinline__ float4 pack(const float* v) { return make_float4(v[0], v[1], v[2], v[3]); }
-  static __device__ __forceinline__ void unpack(const float4 w, float* v) {
-    v[0] = w.x; v[1] = w.y; v[2] = w.z; v[3] = w.w;
-  }
-};
-template <>
-struct Word16<double> {
-  using type = double2;
-  static __device__ __forceinline__ double2 pack(const double* v) { return make_double2(v[0], v[1]); }
-  static __device__ __forceinline__ void unpack(const double2 w, double* v) {
-    v[0] = w.x; v[1] = w.y;
-  }
+struct FarPar {
+  T ar, ai;    // a
+  T kr, ki;    // wavenumber
+  T khi, klo;  // FP64: k / pi as a sum of two doubles; FP32, KIND 2: khi = k / (2 pi)
 };
 
-// e^{ikr}/r and the dipole factor; T = double or float.  GEN: complex wavenumber, or (FP32)
-// phases beyond the hardware sine's range, reduced to one revolution first; otherwise the
-// FP32 phase k r / (2 pi) = r * krev goes to the hardware sine and cosine directly
-// (valid for |k r| / (2 pi) < 256, which the plan checks against its bounding box).
-template <typename T, bool GEN>
-__device__ __forceinline__ void pair_kernel(T dx, T dy, T dz, T nx, T ny, T nz, T kr, T krev, T ki, T& er, T& ei,
-                                            T& tdr, T& tdi, T& r2out) {
-  const T r2 = dx * dx + dy * dy + dz * dz;
-  r2out = r2;
-  T rinv, r;
-  if constexpr (sizeof(T) == 4) {
-    rinv = __frsqrt_rn(r2);
-    r = r2 * rinv;
-  } else {
-    rinv = rsqrt_nr(r2);
-    r = r2 * rinv;
-  }
-  const T d = dx * nx + dy * ny + dz * nz;
-  T s, c;
-  if constexpr (sizeof(T) == 4) {
-    T rev = r * krev;
-    if constexpr (GEN) rev -= rintf(rev);
-    s = __builtin_amdgcn_sinf(rev);
-    c = __builtin_amdgcn_cosf(rev);
-  } else {
-    (void)krev;
-    sincos_red(kr * r, s, c);
-  }
-  T mag = rinv;
-  if constexpr (GEN) {
-    if constexpr (sizeof(T) == 4) mag *= __expf(-ki * r);
-    else mag *= exp(-ki * r);
-  }
-  er = c * mag;
-  ei = s * mag;
-  // dipole factor t (1 - i k r), t = d / r^2, k = kr + i ki: (1 + ki r) - i kr r, and
-  // t kr r = kr d / r
+// 1 / sqrt(x)
+__device__ __forceinline__ float far_rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
+__device__ __forceinline__ double far_rsqrt(double x) { return rsqrt_halley(x); }
+
+// From r^2, 1/r and d = (x - y).n': G and (c, s, q) with e^{ikr} / r = (c + i s) q.  A pair to
+// be skipped passes rinv = 0: r is then 0, every factor finite and q zero, so that its
+// contribution is an exact zero.
+template <typename T, int KIND>
+__device__ __forceinline__ void pair_factors(T r2, T rinv, T d, const FarPar<T>& P, T& gr, T& gi, T& c, T& s, T& q) {
   const T u = d * rinv;
-  const T t = u * rinv;
-  tdr = GEN ? t * ((T)1 + ki * r) : t;
-  tdi = -kr * u;
+  q = rinv;
+  if constexpr (KIND == 0) {
+    gr = fma(u, rinv, P.ar);
+    gi = (T)0;
+    c = (T)1;
+    s = (T)0;
+  } else {
+    const T r = r2 * rinv;
+    if constexpr (sizeof(T) == 4) {
+      T rev = r;
+      if constexpr (KIND == 2) {
+        rev *= P.khi;
+        rev -= rintf(rev);
+      }
+      s = __builtin_amdgcn_sinf(rev);
+      c = __builtin_amdgcn_cosf(rev);
+    } else {
+      bool neg;
+      sincos_turns(r, P.khi, P.klo, s, c, neg);
+      q = neg ? -rinv : rinv;
+    }
+    if constexpr (KIND == 2) {
+      T mag;
+      if constexpr (sizeof(T) == 4) mag = __expf(-P.ki * r);
+      else mag = exp(-P.ki * r);
+      q *= mag;
+      gr = fma(u * rinv, fma(P.ki, r, (T)1), P.ar);
+    } else {
+      gr = fma(u, rinv, P.ar);
+    }
+    gi = fma(-P.kr, u, P.ai);
+  }
 }
 
-// Far-sum pair factors with 1/r left to the caller: (c, s) = e^{i kr r} (times e^{-ki r}
-// when GEN), the dipole factor t (1 - i k r) = (tdr, tdi) with t = d / r^2, from r^2, d =
-// (x - y).n and rinv = 1/r.  A pair to be skipped passes rinv = 0: r is then 0 and every
-// factor stays finite, so its contribution (factors x rinv) is an exact zero.
-template <typename T, bool GEN>
-__device__ __forceinline__ void pair_factors(T r2, T rinv, T d, T kr, T krev, T ki, T& c, T& s, T& tdr, T& tdi) {
-  const T r = r2 * rinv;
-  if constexpr (sizeof(T) == 4) {
-    T rev = r * krev;
-    if constexpr (GEN) rev -= rintf(rev);
-    s = __builtin_amdgcn_sinf(rev);
-    c = __builtin_amdgcn_cosf(rev);
+// The complex kernel value from the factors.
+template <typename T, int KIND>
+__device__ __forceinline__ void pair_value(T gr, T gi, T c, T s, T q, T& kr, T& ki) {
+  if constexpr (KIND == 0) {
+    kr = gr * q;
+    ki = (T)0;
   } else {
-    (void)krev;
-    sincos_red(kr * r, s, c);
+    const T cq = c * q, sq = s * q;
+    kr = gr * cq - gi * sq;
+    ki = gr * sq + gi * cq;
   }
-  if constexpr (GEN) {
-    T mag;
-    if constexpr (sizeof(T) == 4) mag = __expf(-ki * r);
-    else mag = exp(-ki * r);
-    c *= mag;
-    s *= mag;
-  }
-  const T u = d * rinv;
-  const T t = u * rinv;
-  tdr = GEN ? t * ((T)1 + ki * r) : t;
-  tdi = -kr * u;
 }
 
-// Tiled far sum.  pot[i] (+)= sum_j [q_j + m_j * t_ij (1-ikr)] e^{ikr}/r / (4 pi)
-// MASK: skip sources whose patch is in the target's sorted near list.  Sources are sorted
-// by patch, so each thread keeps the source interval [ea, eb) of the next near patch
-// (patch p owns sources ixyzso[p]-1 .. ixyzso[p+1]-2) and moves it forward when the tile
-// passes eb; the pair loop itself has no branches (a skipped pair adds an exact zero).
-template <typename T, bool MASK, bool GEN, int NRHS>
-__global__ void __launch_bounds__(TPB) k_farsum(int64_t ntarg, const T* __restrict__ tx, const T* __restrict__ ty,
-                                                const T* __restrict__ tz, int64_t nsrc,
-                                                const T* __restrict__ sx, const T* __restrict__ sy,
-                                                const T* __restrict__ sz, const T* __restrict__ snx,
-                                                const T* __restrict__ sny, const T* __restrict__ snz,
-                                                const int64_t* __restrict__ ixyzso, const V2<T>* __restrict__ qstr,
-                                                const V2<T>* __restrict__ mstr, int64_t ldstr,
-                                                const int64_t* __restrict__ row_ptr,
-                                                const int* __restrict__ near_sorted, T kr, T krev, T ki, T thresh2,
-                                                int64_t chunk, V2<T>* __restrict__ part, int64_t ldpart) {
-  // One LDS record per source of the tile: x, y, z, nx, ny, nz, then (q, m) of each
-  // right-hand side, padded to whole 16-byte words, so that a pair's operands are a few
-  // 16-byte reads at immediate offsets from one address (all lanes read the same record).
-  using W16 = typename Word16<T>::type;
-  constexpr int PER = 16 / (int)sizeof(T);            // values per 16-byte word
-  constexpr int NV = 6 + 4 * NRHS;                    // values per source
-  constexpr int REC = (NV + PER - 1) / PER;           // 16-byte words per source
-  __shared__ W16 tile[TPB * REC];
-  // blockIdx.z selects a group of NRHS right-hand sides: the geometry and e^{ikr} of a
-  // pair are computed once per group
+// The sources of a target's near patches, in source order: sources are sorted by patch and
+// the near list of each target too, so [ea, eb) is the interval of the next near patch
+// (patch p owns sources ixyzso[p]-1 .. ixyzso[p+1]-2), moved on by seek(j) to the first
+// that ends after source j.
+struct NearCursor {
+  static constexpr int NONE = 0x7fffffff;
+  const int* list;
+  const int64_t* ixyzso;
+  int64_t ptr = 0, end = 0;
+  int ea = NONE, eb = NONE;
+  __device__ __forceinline__ void seek(int j) {
+    ea = NONE;
+    eb = NONE;
+    while (ptr < end) {
+      const int p = list[ptr];
+      const int e = (int)(ixyzso[p + 1] - 1);
+      if (e > j) {
+        ea = (int)(ixyzso[p] - 1);
+        eb = e;
+        break;
+      }
+      ptr++;
+    }
+  }
+};
+
+// Far sum on the vector units, one target per lane, one wavefront per workgroup:
+// part[i] = sum over the sources of split blockIdx.y of K(x_i, y_j) s_j, for the NRHS
+// right-hand sides of group blockIdx.z (the kernel value is computed once per group).
+// Every lane works on the same source, whose geometry and strengths are wave-uniform: they
+// come by scalar loads into scalar registers, and one operand of each vector instruction
+// may be one of those, so that no LDS, barrier or vector register is spent on them.
+// Bound by vector instruction issue: a pair takes 58 instructions in FP64 with a real
+// wavenumber (76 with a charge and a dipole strength per source, sincos_red and a Newton
+// step more; 262 against 330 cycles of a SIMD per 64 pairs; the add/subtract apply of 344064
+// points 412 -> 337 ms, of 25920 points 4.44 -> 3.55 ms), 20 for Laplace (which ran the
+// Helmholtz kernel with k = 0: 106 against 330 cycles) and 26 in FP32 (91 against 103
+// cycles: 1.95 -> 1.85 ms for 43008 points), three of them hardware functions of 10 cycles.
+// MASK: sources of the target's near patches are skipped; tiles of STILE sources that hold
+// none for any lane of the wavefront (nearly all) run without a test.
+// !MASK: sources within thresh of the target are skipped: each pair is compared, and only
+// if a lane of a block of UB sources finds one is the block summed again with the test.
+constexpr int STILE = 32;
+template <typename T, bool MASK, int KIND, int NRHS>
+__global__ void __launch_bounds__(64) k_farsum(int ntarg, const T* __restrict__ tx, const T* __restrict__ ty,
+                                               const T* __restrict__ tz, int nsrc, const T* __restrict__ geo,
+                                               const int64_t* __restrict__ ixyzso, const V2<T>* __restrict__ str,
+                                               const int64_t* __restrict__ row_ptr, const int* __restrict__ near_sorted,
+                                               FarPar<T> P, T thresh2, int chunk, int nrhs,
+                                               V2<T>* __restrict__ part, int64_t ldpart) {
   const int64_t rg = blockIdx.z;
-  qstr += rg * NRHS * ldstr;
-  mstr += rg * NRHS * ldstr;
-  const int64_t i = blockIdx.x * (int64_t)TPB + threadIdx.x;
+  str += rg * NRHS * nsrc;
+  const int i = blockIdx.x * 64 + threadIdx.x;
   const bool act = i < ntarg;
   const T x = act ? tx[i] : (T)0, y = act ? ty[i] : (T)0, z = act ? tz[i] : (T)0;
   T accr[NRHS], acci[NRHS];
 #pragma unroll
   for (int r = 0; r < NRHS; r++) { accr[r] = 0; acci[r] = 0; }
-  const int64_t jbeg = blockIdx.y * chunk;
-  const int64_t jend = jbeg + chunk < nsrc ? jbeg + chunk : nsrc;
-  constexpr int64_t NONE = INT64_MAX;
-  int64_t nptr = 0, nend = 0, ea = NONE, eb = NONE;
-  // first near patch of the target whose sources end after j
-  auto advance = [&](int64_t j) {
-    ea = NONE;
-    eb = NONE;
-    while (nptr < nend) {
-      const int p = near_sorted[nptr];
-      const int64_t e = ixyzso[p + 1] - 1;
-      if (e > j) {
-        ea = ixyzso[p] - 1;
-        eb = e;
-        break;
-      }
-      nptr++;
-    }
-  };
-  if (MASK && act && jbeg < jend) {
-    nptr = row_ptr[i] - 1;
-    nend = row_ptr[i + 1] - 1;
-    advance(jbeg);
-  }
-  for (int64_t base = jbeg; base < jend; base += TPB) {
-    const int64_t j = base + threadIdx.x;
-    if (j < jend) {
-      T v[REC * PER];
-      v[0] = sx[j]; v[1] = sy[j]; v[2] = sz[j];
-      v[3] = snx[j]; v[4] = sny[j]; v[5] = snz[j];
+  const int jbeg = blockIdx.y * chunk;
+  const int jend = jbeg + chunk < nsrc ? jbeg + chunk : nsrc;
+  // source j: r^2 and, unless skip, its contribution
+  auto pair = [&](int j, auto test) -> T {
+    const T* g = geo + (int64_t)j * GEO<T>;
+    const T dx = x - g[0], dy = y - g[1], dz = z - g[2];
+    const T r2 = dx * dx + dy * dy + dz * dz;
+    const T d = dx * g[3] + dy * g[4] + dz * g[5];
+    T rinv = far_rsqrt(r2);
+    if constexpr (!std::is_same<decltype(test), std::nullptr_t>::value) rinv = test(r2) ? rinv : (T)0;
+    T gr, gi, c, s, q;
+    pair_factors<T, KIND>(r2, rinv, d, P, gr, gi, c, s, q);
+    const V2<T>* v = str + (int64_t)j * NRHS;
+    if constexpr (NRHS == 1 && KIND != 0) {
+      const T ir = v[0].x * gr - v[0].y * gi, ii = v[0].x * gi + v[0].y * gr;
+      accr[0] = fma(ir * c - ii * s, q, accr[0]);
+      acci[0] = fma(ir * s + ii * c, q, acci[0]);
+    } else {
+      T vr, vi;
+      pair_value<T, KIND>(gr, gi, c, s, q, vr, vi);
 #pragma unroll
       for (int r = 0; r < NRHS; r++) {
-        const V2<T> q = qstr[r * ldstr + j], m = mstr[r * ldstr + j];
-        v[6 + 4 * r] = q.x; v[7 + 4 * r] = q.y; v[8 + 4 * r] = m.x; v[9 + 4 * r] = m.y;
-      }
-#pragma unroll
-      for (int e = NV; e < REC * PER; e++) v[e] = (T)0;
-#pragma unroll
-      for (int w = 0; w < REC; w++) tile[threadIdx.x * REC + w] = Word16<T>::pack(v + w * PER);
-    }
-    __syncthreads();
-    const int cnt = jend - base < TPB ? (int)(jend - base) : TPB;
-    // FULL: no source of the tile belongs to a near patch of any target of the wavefront
-    // (the next near interval of every lane starts at or after the tile's end), so every
-    // pair is summed and the per-pair test and selects drop out
-    auto pairs = [&](auto full_tag) {
-      constexpr bool FULL = decltype(full_tag)::value;
-#pragma unroll 2
-      for (int k = 0; k < cnt; k++) {
-        const int64_t jk = base + k;
-        if (MASK && !FULL && jk >= eb) advance(jk);
-        T v[REC * PER];
-#pragma unroll
-        for (int w = 0; w < REC; w++) Word16<T>::unpack(tile[k * REC + w], v + w * PER);
-        const T dx = x - v[0], dy = y - v[1], dz = z - v[2];
-        const T r2 = dx * dx + dy * dy + dz * dz;
-        T rinv;
-        if constexpr (sizeof(T) == 4) rinv = __frsqrt_rn(r2);
-        else rinv = rsqrt_nr(r2);
-        // with the mask, sources within thresh of the target belong to its near patches
-        if (!FULL) rinv = (MASK ? jk < ea : r2 > thresh2) ? rinv : (T)0;
-        const T d = dx * v[3] + dy * v[4] + dz * v[5];
-        T c, sn, tdr, tdi;
-        pair_factors<T, GEN>(r2, rinv, d, kr, krev, ki, c, sn, tdr, tdi);
-#pragma unroll
-        for (int r = 0; r < NRHS; r++) {
-          const V2<T> q = {v[6 + 4 * r], v[7 + 4 * r]}, m = {v[8 + 4 * r], v[9 + 4 * r]};
-          // inner = q + m*(tdr + i tdi); contribution = inner * (c + i sn) / r
-          const T ir = q.x + m.x * tdr - m.y * tdi;
-          const T ii = q.y + m.x * tdi + m.y * tdr;
-          const T zr = ir * c - ii * sn, zi = ir * sn + ii * c;
-          accr[r] += zr * rinv;
-          acci[r] += zi * rinv;
+        if constexpr (KIND == 0) {
+          accr[r] = fma(vr, v[r].x, accr[r]);
+          acci[r] = fma(vr, v[r].y, acci[r]);
+        } else {
+          accr[r] = fma(vr, v[r].x, fma(-vi, v[r].y, accr[r]));
+          acci[r] = fma(vr, v[r].y, fma(vi, v[r].x, acci[r]));
         }
       }
-    };
-    // (FP64 with several right-hand sides keeps the one loop: the second copy would cost
-    // it occupancy)
-    constexpr bool TRY_FULL = MASK && (sizeof(T) == 4 || NRHS == 1);
-    bool full = false;
-    if (TRY_FULL) {
-      if (base >= eb) advance(base);  // the state the first pair of the tile would reach
-      full = __all(ea >= base + cnt) != 0;  // wave-uniform
     }
-    if (full)
-      pairs(std::true_type{});
-    else
-      pairs(std::false_type{});
-    __syncthreads();
+    return r2;
+  };
+  if constexpr (MASK) {
+    constexpr int UN = sizeof(T) == 8 ? 2 : 1;  // FP64: 262 against 295 cycles per 64 pairs; FP32: 98 against 95
+    NearCursor nc{near_sorted, ixyzso};
+    if (act && jbeg < jend) {
+      nc.ptr = row_ptr[i] - 1;
+      nc.end = row_ptr[i + 1] - 1;
+      nc.seek(jbeg);
+    }
+    for (int base = jbeg; base < jend; base += STILE) {
+      const int cnt = jend - base < STILE ? jend - base : STILE;
+      if (base >= nc.eb) nc.seek(base);
+      if (__all(nc.ea >= base + cnt)) {
+#pragma unroll UN
+        for (int k = 0; k < cnt; k++) pair(base + k, nullptr);
+      } else {
+#pragma unroll 1
+        for (int k = 0; k < cnt; k++) {
+          const int j = base + k;
+          if (j >= nc.eb) nc.seek(j);
+          pair(j, [&](T) { return j < nc.ea; });
+        }
+      }
+    }
+  } else {
+    constexpr int UB = 4;
+    int j = jbeg;
+    for (; j + UB <= jend; j += UB) {
+      T sr[NRHS], si[NRHS];
+#pragma unroll
+      for (int r = 0; r < NRHS; r++) { sr[r] = accr[r]; si[r] = acci[r]; }
+      bool close = false;
+#pragma unroll
+      for (int k = 0; k < UB; k++) close |= !(pair(j + k, nullptr) > thresh2);
+      if (__any(close)) {
+#pragma unroll
+        for (int r = 0; r < NRHS; r++) { accr[r] = sr[r]; acci[r] = si[r]; }
+#pragma unroll 1
+        for (int k = 0; k < UB; k++) pair(j + k, [&](T r2) { return r2 > thresh2; });
+      }
+    }
+    for (; j < jend; j++) pair(j, [&](T r2) { return r2 > thresh2; });
   }
   if (act) {
 #pragma unroll
-    for (int r = 0; r < NRHS; r++) part[(int64_t)blockIdx.y * ldpart + (rg * NRHS + r) * ntarg + i] = {accr[r], acci[r]};
+    for (int r = 0; r < NRHS; r++)
+      if (rg * NRHS + r < nrhs)
+        part[(int64_t)blockIdx.y * ldpart + (rg * NRHS + r) * ntarg + i] = {accr[r], acci[r]};
   }
 }
 
-// Far sum of 16 right-hand sides on the matrix cores (FP32, near patches masked): with
-// G = e^{ikr}/r and H = t (1 - ikr) e^{ikr}/r for a pair (target, source), the group's
-// potentials are the complex products pot = G q + H m of the target x source kernel
-// matrices with the source x 16 strength matrices.  A wavefront takes 16 targets; in a
-// step of 4 sources lane l evaluates the pair (target l % 16, source l / 16) once, and
-// v_mfma_f32_16x16x4f32 multiplies 16 x 4 kernel blocks by 4 x 16 strength blocks (lane
-// l supplies source l / 16, right-hand side l % 16).  Each complex product takes three
-// real ones (Gauss): a1 = Re G Re q + Re H Re m, a2 = Im G Im q + Im H Im m,
-// a3 = (Re G + Im G)(Re q + Im q) + (Re H + Im H)(Re m + Im m), so Re pot = a1 - a2 and
-// Im pot = a3 - a1 - a2: six matrix products per step instead of eight.  Accumulator
-// element r of lane l is target 4 (l / 16) + r, right-hand side l % 16.
-// The workgroup stages FT sources at a time in LDS: geometry (x, y, z, nx, ny, nz) and
-// the (q, m) of the 16 right-hand sides of each source.
-constexpr int FT = 64;         // sources per LDS tile (18 KB of LDS per workgroup with FW = 4)
-constexpr int FW = 4;          // wavefronts per workgroup (16 targets each)
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-template <bool GEN>
-__global__ void __launch_bounds__(64 * FW) k_farsum_mfma(int64_t ntarg, const float* __restrict__ tx,
-                                                        const float* __restrict__ ty, const float* __restrict__ tz,
-                                                        int64_t nsrc, const float* __restrict__ sx,
-                                                        const float* __restrict__ sy, const float* __restrict__ sz,
-                                                        const float* __restrict__ snx, const float* __restrict__ sny,
-                                                        const float* __restrict__ snz,
-                                                        const int64_t* __restrict__ ixyzso,
-                                                        const V2<float>* __restrict__ qstr,
-                                                        const V2<float>* __restrict__ mstr, int64_t ldstr,
-                                                        const int64_t* __restrict__ row_ptr,
-                                                        const int* __restrict__ near_sorted, float kr, float krev,
-                                                        float ki, int64_t chunk, V2<float>* __restrict__ part,
-                                                        int64_t ldpart) {
-  __shared__ float4 geo[FT * 2];   // x y z nx | ny nz - -
-  __shared__ float4 str[FT * 16];  // (q re, q im, m re, m im) of source j, right-hand side r at j * 16 + r
+// Far sum of a group of 16 right-hand sides on the matrix cores: the group's potentials are
+// the complex product pot = K S of the target x source kernel matrix with the source x 16
+// strength matrix.  A wavefront takes MT tiles of 16 targets; in a step of 4 sources lane l
+// evaluates the pairs (target l % 16 of each tile, source l / 16) once on the vector units,
+// and the 16x16x4 product of the matrix cores multiplies the 16 x 4 kernel blocks by the 4 x
+// 16 strength blocks (lane l supplies source l / 16, right-hand side l % 16).  The complex
+// product takes three real ones (Gauss): a1 = Re K Re s, a2 = Im K Im s, a3 = (Re K + Im K)
+// (Re s + Im s), so Re pot = a1 - a2 and Im pot = a3 - a1 - a2.  Laplace: two, K being real.
+// The workgroup stages FT sources at a time in LDS, geometry and strengths; MT tiles share
+// each LDS read.
+// Bound by issue: on this chip FP32 and FP64 matrix instructions do not overlap with vector
+// ones of the same SIMD (measured: the times of wavefronts of either kind add up), so that the
+// products' 3 x 32 cycles (FP32; 3 x 64 in FP64) and the kernel values of 64 pairs add.  One
+// complex kernel matrix takes half the products of separate charge and dipole matrices: 209
+// against 337 cycles per 64 pairs in FP32 (the 16-density apply of 86016 points 27.1 -> 16.7
+// ms), 466 in FP64 for 16 densities, where groups of 4 on the vector units took 400 each.
+// Tiles of 128 sources, 1, 3 or 4 target tiles and an unrolled loop were all 1 to 15% slower.
+template <typename T>
+struct Mfma16;
+template <>
+struct Mfma16<float> {
+  typedef float V __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ V mul(float a, float b, V c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  // target of the tile in accumulator element r of lane l (its right-hand side is l % 16)
+  static __device__ __forceinline__ int row(int l, int r) { return 4 * (l >> 4) + r; }
+};
+template <>
+struct Mfma16<double> {
+  typedef double V __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ V mul(double a, double b, V c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int l, int r) { return (l >> 4) + 4 * r; }
+};
+
+constexpr int FT = 64;  // sources per LDS tile
+constexpr int FW = 4;   // wavefronts per workgroup
+template <typename T>
+constexpr int MT = 2;  // tiles of 16 targets per wavefront
+template <typename T, bool MASK, int KIND>
+__global__ void __launch_bounds__(64 * FW) k_farsum_mfma(int ntarg, const T* __restrict__ tx, const T* __restrict__ ty,
+                                                         const T* __restrict__ tz, int nsrc, const T* __restrict__ geo,
+                                                         const int64_t* __restrict__ ixyzso,
+                                                         const V2<T>* __restrict__ str,
+                                                         const int64_t* __restrict__ row_ptr,
+                                                         const int* __restrict__ near_sorted, FarPar<T> P, T thresh2,
+                                                         int chunk, int nrhs, V2<T>* __restrict__ part,
+                                                         int64_t ldpart) {
+  using M = Mfma16<T>;
+  using V = typename M::V;
+  constexpr int NT = MT<T>, G = GEO<T>;
+  __shared__ __align__(16) T lgeo[FT * G];
+  __shared__ __align__(16) V2<T> lstr[FT * MG];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int rg = blockIdx.z;
-  qstr += (int64_t)rg * 16 * ldstr;
-  mstr += (int64_t)rg * 16 * ldstr;
-  const int64_t t0 = (blockIdx.x * (int64_t)FW + wv) * 16;
-  const int64_t i = t0 + (lane & 15);  // this lane's target
-  const bool act = i < ntarg;
-  const float x = act ? tx[i] : 0.0f, y = act ? ty[i] : 0.0f, z = act ? tz[i] : 0.0f;
+  const int64_t rg = blockIdx.z;
+  str += rg * MG * nsrc;
+  const int t0 = (blockIdx.x * FW + wv) * (16 * NT);
   const int ks = lane >> 4;  // this lane's source within a step of 4
-  f32x4 a1 = {0.0f, 0.0f, 0.0f, 0.0f}, a2 = {0.0f, 0.0f, 0.0f, 0.0f}, a3 = {0.0f, 0.0f, 0.0f, 0.0f};
-  const int64_t jbeg = blockIdx.y * chunk;
-  const int64_t jend = jbeg + chunk < nsrc ? jbeg + chunk : nsrc;
-  constexpr int64_t NONE = INT64_MAX;
-  int64_t nptr = 0, nend = 0, ea = NONE, eb = NONE;
-  auto advance = [&](int64_t j) {
-    ea = NONE;
-    eb = NONE;
-    while (nptr < nend) {
-      const int p = near_sorted[nptr];
-      const int64_t e = ixyzso[p + 1] - 1;
-      if (e > j) {
-        ea = ixyzso[p] - 1;
-        eb = e;
-        break;
-      }
-      nptr++;
-    }
-  };
-  if (act && jbeg < jend) {
-    nptr = row_ptr[i] - 1;
-    nend = row_ptr[i + 1] - 1;
-    advance(jbeg);
-  }
-  for (int64_t base = jbeg; base < jend; base += FT) {
-    const int cnt = jend - base < FT ? (int)(jend - base) : FT;
-    __syncthreads();
-    for (int e = threadIdx.x; e < FT; e += 64 * FW) {
-      const int64_t j = base + e;
-      const bool ok = e < cnt;
-      geo[2 * e] = ok ? make_float4(sx[j], sy[j], sz[j], snx[j]) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      geo[2 * e + 1] = ok ? make_float4(sny[j], snz[j], 0.0f, 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
-    // strengths: consecutive threads read consecutive sources of one right-hand side
-    for (int e = threadIdx.x; e < FT * 16; e += 64 * FW) {
-      const int jl = e % FT, r = e / FT;
-      float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      if (jl < cnt) {
-        const V2<float> q = qstr[r * ldstr + base + jl], m = mstr[r * ldstr + base + jl];
-        v = make_float4(q.x, q.y, m.x, m.y);
-      }
-      str[jl * 16 + r] = v;
-    }
-    __syncthreads();
-    // sources past the tile's count carry zero strengths (and are masked below)
-    for (int k = 0; k < cnt; k += 4) {
-      const int jl = k + ks;
-      const int64_t jk = base + jl;
-      if (jk >= eb) advance(jk);
-      const float4 g0 = geo[2 * jl], g1 = geo[2 * jl + 1];
-      const float dx = x - g0.x, dy = y - g0.y, dz = z - g0.z;
-      const float r2 = dx * dx + dy * dy + dz * dz;
-      float rinv = __frsqrt_rn(r2);
-      rinv = (act && jl < cnt && jk < ea) ? rinv : 0.0f;
-      const float d = dx * g0.w + dy * g1.x + dz * g1.y;
-      float c, sn, tdr, tdi;
-      pair_factors<float, GEN>(r2, rinv, d, kr, krev, ki, c, sn, tdr, tdi);
-      const float gr = c * rinv, gi = sn * rinv;
-      const float hr = tdr * gr - tdi * gi, hi = tdr * gi + tdi * gr;
-      const float4 sv = str[(k + ks) * 16 + (lane & 15)];  // source k + l / 16, right-hand side l % 16
-      a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(gr, sv.x, a1, 0, 0, 0);
-      a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(hr, sv.z, a1, 0, 0, 0);
-      a2 = __builtin_amdgcn_mfma_f32_16x16x4f32(gi, sv.y, a2, 0, 0, 0);
-      a2 = __builtin_amdgcn_mfma_f32_16x16x4f32(hi, sv.w, a2, 0, 0, 0);
-      a3 = __builtin_amdgcn_mfma_f32_16x16x4f32(gr + gi, sv.x + sv.y, a3, 0, 0, 0);
-      a3 = __builtin_amdgcn_mfma_f32_16x16x4f32(hr + hi, sv.z + sv.w, a3, 0, 0, 0);
-    }
-  }
-  // accumulator element r of lane l: target 4 (l / 16) + r, right-hand side l % 16
-  const int rhs = lane & 15;
+  T x[NT], y[NT], z[NT];
+  V a1[NT], a2[NT], a3[NT];
+  const int jbeg = blockIdx.y * chunk;
+  const int jend = jbeg + chunk < nsrc ? jbeg + chunk : nsrc;
+  NearCursor nc[NT];
+  bool act[NT];
 #pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const int64_t it = t0 + 4 * (lane >> 4) + r;
-    if (it < ntarg)
-      part[(int64_t)blockIdx.y * ldpart + (int64_t)(rg * 16 + rhs) * ntarg + it] = {a1[r] - a2[r], a3[r] - a1[r] - a2[r]};
+  for (int t = 0; t < NT; t++) {
+    const int i = t0 + 16 * t + (lane & 15);
+    act[t] = i < ntarg;
+    x[t] = act[t] ? tx[i] : (T)0;
+    y[t] = act[t] ? ty[i] : (T)0;
+    z[t] = act[t] ? tz[i] : (T)0;
+    a1[t] = a2[t] = a3[t] = V{(T)0, (T)0, (T)0, (T)0};
+    nc[t] = NearCursor{near_sorted, ixyzso};
+    if (MASK && act[t] && jbeg < jend) {
+      nc[t].ptr = row_ptr[i] - 1;
+      nc[t].end = row_ptr[i + 1] - 1;
+      nc[t].seek(jbeg);
+    }
+  }
+  for (int base = jbeg; base < jend; base += FT) {
+    const int cnt = jend - base < FT ? jend - base : FT;
+    __syncthreads();
+    // sources past the tile's count: zero geometry and strengths (and skipped below)
+    for (int e = threadIdx.x; e < FT * G; e += 64 * FW) lgeo[e] = e < cnt * G ? geo[(int64_t)base * G + e] : (T)0;
+    for (int e = threadIdx.x; e < FT * MG; e += 64 * FW)
+      lstr[e] = e < cnt * MG ? str[(int64_t)base * MG + e] : V2<T>{(T)0, (T)0};
+    __syncthreads();
+    // FULL: no source of the tile is skipped for any target of the wavefront
+    auto step = [&](int k, auto full_tag) {
+      constexpr bool FULL = decltype(full_tag)::value;
+      const int jl = k + ks, j = base + jl;
+      const T* g = lgeo + jl * G;
+      const T gx = g[0], gy = g[1], gz = g[2], nx = g[3], ny = g[4], nz = g[5];
+      const V2<T> sv = lstr[jl * MG + (lane & 15)];  // source k + l / 16, right-hand side l % 16
+      const T ss = sv.x + sv.y;
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        const T dx = x[t] - gx, dy = y[t] - gy, dz = z[t] - gz;
+        const T r2 = dx * dx + dy * dy + dz * dz;
+        const T d = dx * nx + dy * ny + dz * nz;
+        T rinv = far_rsqrt(r2);
+        if constexpr (!FULL) {
+          if (MASK && j >= nc[t].eb) nc[t].seek(j);
+          rinv = (act[t] && jl < cnt && (MASK ? j < nc[t].ea : r2 > thresh2)) ? rinv : (T)0;
+        }
+        T gr, gi, c, s, q, vr, vi;
+        pair_factors<T, KIND>(r2, rinv, d, P, gr, gi, c, s, q);
+        pair_value<T, KIND>(gr, gi, c, s, q, vr, vi);
+        a1[t] = M::mul(vr, sv.x, a1[t]);
+        if constexpr (KIND == 0) {
+          a2[t] = M::mul(vr, sv.y, a2[t]);
+        } else {
+          a2[t] = M::mul(vi, sv.y, a2[t]);
+          a3[t] = M::mul(vr + vi, ss, a3[t]);
+        }
+      }
+    };
+    bool full = MASK && cnt == FT;
+    if constexpr (MASK) {
+      bool mine = true;
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        if (base >= nc[t].eb) nc[t].seek(base);
+        mine = mine && act[t] && nc[t].ea >= base + cnt;
+      }
+      full = full && __all(mine);
+    }
+    if (full) {
+#pragma unroll 1
+      for (int k = 0; k < FT; k += 4) step(k, std::true_type{});
+    } else {
+#pragma unroll 1
+      for (int k = 0; k < cnt; k += 4) step(k, std::false_type{});
+    }
+  }
+  const int r = (int)rg * MG + (lane & 15);
+  if (r < nrhs) {
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int it = t0 + 16 * t + M::row(lane, e);
+        if (it < ntarg) {
+          V2<T> v;
+          if constexpr (KIND == 0) v = {a1[t][e], a2[t][e]};
+          else v = {a1[t][e] - a2[t][e], a3[t][e] - a1[t][e] - a2[t][e]};
+          part[(int64_t)blockIdx.y * ldpart + (int64_t)r * ntarg + it] = v;
+        }
+      }
   }
 }
 
@@ -427,42 +478,65 @@ __global__ void k_farsum_reduce(int64_t ntarg, int nrhs, int nsplit, const V2<T>
   pot[r * ldpot + i] = {(T)(sr * (T)OVER4PI), (T)(si * (T)OVER4PI)};
 }
 
-// Near subtraction (ADDSUB mode): one wavefront per target, lanes over the oversampled
-// points of each near patch.
-__global__ void k_near_sub(int64_t ntarg, const double* __restrict__ tx, const double* __restrict__ ty,
-                           const double* __restrict__ tz, const double* __restrict__ sx,
-                           const double* __restrict__ sy, const double* __restrict__ sz,
-                           const double* __restrict__ snx, const double* __restrict__ sny,
-                           const double* __restrict__ snz, const V2<double>* __restrict__ qstr,
-                           const V2<double>* __restrict__ mstr, int64_t ldstr, int nrhs,
-                           const int64_t* __restrict__ row_ptr, const int64_t* __restrict__ col_ind,
-                           const int64_t* __restrict__ ixyzso, double kr, double ki, double thresh2,
-                           V2<double>* __restrict__ pot, int64_t ldpot) {
-  const int64_t i = blockIdx.x * (int64_t)(blockDim.x / 64) + threadIdx.x / 64;
+// What the near subtraction (add/subtract form) needs: targets, sources and strengths.
+struct SubArgs {
+  const double *tx, *ty, *tz, *geo;
+  const V2<double>* str;
+  int64_t nptso;
+  int nr;  // right-hand sides per strength group
+  const int64_t *col_ind, *ixyzso;
+  FarPar<double> P;
+  double thresh2;
+};
+
+// Smooth-rule contributions of target i's near patches (CSR entries j0..j1), subtracted from
+// the lane's sums of right-hand sides rb .. rb + RB - 1.  Four patches at a time, 16 lanes
+// each: a patch's 15 to 45 oversampled nodes fill 16 lanes better than 64 (one patch at a
+// time on all lanes took 24 us for 1920 and 182 us for 25920 targets).
+template <int RB>
+__device__ __forceinline__ void near_sub(const SubArgs& S, int64_t i, int64_t j0, int64_t j1, int rb, int nrhs,
+                                         double (&ar)[RB], double (&ai)[RB]) {
   const int lane = threadIdx.x % 64;
-  if (i >= ntarg) return;
-  const double x = tx[i], y = ty[i], z = tz[i];
-  for (int r = 0; r < nrhs; r++) {
-    double sr = 0.0, si = 0.0;
-    for (int64_t jj = row_ptr[i] - 1; jj < row_ptr[i + 1] - 1; jj++) {
-      const int64_t ip = col_ind[jj] - 1;
-      for (int64_t j = ixyzso[ip] - 1 + lane; j < ixyzso[ip + 1] - 1; j += 64) {
-        double er, ei, tdr, tdi, r2;
-        pair_kernel<double, true>(x - sx[j], y - sy[j], z - sz[j], snx[j], sny[j], snz[j], kr, 0.0, ki, er, ei, tdr,
-                                  tdi, r2);
-        if (r2 <= thresh2) continue;
-        const V2<double> q = qstr[r * ldstr + j], m = mstr[r * ldstr + j];
-        const double ir = q.x + m.x * tdr - m.y * tdi;
-        const double ii = q.y + m.x * tdi + m.y * tdr;
-        sr += ir * er - ii * ei;
-        si += ir * ei + ii * er;
+  const double x = S.tx[i], y = S.ty[i], z = S.tz[i];
+  for (int64_t jj = j0 + (lane >> 4); jj < j1; jj += 4) {
+    const int64_t ip = S.col_ind[jj] - 1;
+    const int64_t e = S.ixyzso[ip + 1] - 1;
+    for (int64_t j = S.ixyzso[ip] - 1 + (lane & 15); j < e; j += 16) {
+      const double* g = S.geo + 6 * j;
+      const double dx = x - g[0], dy = y - g[1], dz = z - g[2];
+      const double r2 = dx * dx + dy * dy + dz * dz;
+      const double d = dx * g[3] + dy * g[4] + dz * g[5];
+      const double rinv = r2 > S.thresh2 ? far_rsqrt(r2) : 0.0;
+      double gr, gi, c, s, q, vr, vi;
+      if (S.P.ki != 0.0) pair_factors<double, 2>(r2, rinv, d, S.P, gr, gi, c, s, q);
+      else if (S.P.kr != 0.0) pair_factors<double, 1>(r2, rinv, d, S.P, gr, gi, c, s, q);
+      else pair_factors<double, 0>(r2, rinv, d, S.P, gr, gi, c, s, q), gi = S.P.ai;
+      pair_value<double, 1>(gr, gi, c, s, -OVER4PI * q, vr, vi);
+#pragma unroll
+      for (int r = 0; r < RB; r++) {
+        if (rb + r < nrhs) {
+          const int g_ = (rb + r) / S.nr;
+          const V2<double> v = S.str[((int64_t)g_ * S.nptso + j) * S.nr + (rb + r - g_ * S.nr)];
+          ar[r] = fma(vr, v.x, fma(-vi, v.y, ar[r]));
+          ai[r] = fma(vr, v.y, fma(vi, v.x, ai[r]));
+        }
       }
     }
-    sr = wave_sum(sr);
-    si = wave_sum(si);
-    if (lane == 0) {
-      pot[r * ldpot + i].x -= sr * OVER4PI;
-      pot[r * ldpot + i].y -= si * OVER4PI;
+  }
+}
+
+// Near subtraction alone (after the general CSR kernel): one wavefront per target.
+__global__ void k_near_sub(int64_t ntarg, const int64_t* __restrict__ row_ptr, SubArgs S, int nrhs,
+                           V2<double>* __restrict__ pot, int64_t ldpot) {
+  const int64_t i = blockIdx.x * (int64_t)(blockDim.x / 64) + threadIdx.x / 64;
+  if (i >= ntarg) return;
+  for (int r = 0; r < nrhs; r++) {
+    double ar[1] = {0.0}, ai[1] = {0.0};
+    near_sub<1>(S, i, row_ptr[i] - 1, row_ptr[i + 1] - 1, r, nrhs, ar, ai);
+    const double sr = wave_sum(ar[0]), si = wave_sum(ai[0]);
+    if (threadIdx.x % 64 == 0) {
+      pot[r * ldpot + i].x += sr;
+      pot[r * ldpot + i].y += si;
     }
   }
 }
@@ -492,17 +566,20 @@ __global__ void k_csr_gen(int64_t ntarg, const int64_t* __restrict__ row_ptr, co
   }
 }
 
-// Far-sum reduction fused with the CSR near correction for all right-hand sides (uniform
-// patch size p): one wavefront per target row, lanes over the row's contiguous wnear
-// segment; every wnear element is loaded once per group of RB right-hand sides.
+// Far-sum reduction fused with the CSR near correction and, with SUB (FP64 add/subtract
+// form), the near subtraction, for all right-hand sides (uniform patch size p): one
+// wavefront per target row, lanes over the row's contiguous wnear segment; every wnear
+// element is loaded once per group of RB right-hand sides.  One launch instead of three for
+// a small problem (1920 points: the whole apply 83 -> 37 us, with the far sum's 53 us cut by
+// its finer source splits).
 //   pot[r][i] = (sum over source splits of part[r][i]) / (4 pi) + sum_e wnear_e sigma_r(src_e)
 // PC > 0: the patch size as a compile-time constant (the orders 1..10), else p_rt.
-template <typename T, typename TW, int RB, int PC>
+template <typename T, typename TW, int RB, int PC, bool SUB>
 __global__ void k_reduce_csr(int64_t ntarg, int nrhs, int nsplit, const V2<T>* __restrict__ part, int64_t ldpart,
                              const int64_t* __restrict__ row_ptr, const int* __restrict__ csr_src,
                              const int64_t* __restrict__ iquad, int p_rt,
                              const V2<TW>* __restrict__ wnear, const V2<T>* __restrict__ sigma, int64_t ldsig,
-                             V2<T>* __restrict__ pot, int64_t ldpot) {
+                             V2<T>* __restrict__ pot, int64_t ldpot, SubArgs S) {
   const int p = PC > 0 ? PC : p_rt;
   const int64_t i = blockIdx.x * (int64_t)(blockDim.x / 64) + threadIdx.x / 64;
   const int lane = threadIdx.x % 64;
@@ -527,6 +604,18 @@ __global__ void k_reduce_csr(int64_t ntarg, int nrhs, int nsplit, const V2<T>* _
         }
       }
     }
+    if constexpr (SUB) near_sub<RB>(S, i, j0, j1, rb, nrhs, ar, ai);
+    // the source splits: with one right-hand side the lanes share them
+    T fr = 0, fi = 0;
+    if constexpr (RB == 1) {
+      for (int sp = lane; sp < nsplit; sp += 64) {
+        const V2<T> v = part[(int64_t)sp * ldpart + rb * ntarg + i];
+        fr += v.x;
+        fi += v.y;
+      }
+      fr = wave_sum(fr);
+      fi = wave_sum(fi);
+    }
     double mr = 0.0, mi = 0.0;
 #pragma unroll
     for (int r = 0; r < RB; r++) {
@@ -535,11 +624,12 @@ __global__ void k_reduce_csr(int64_t ntarg, int nrhs, int nsplit, const V2<T>* _
     }
     const int r = rb + lane;
     if (lane < RB && r < nrhs) {
-      T fr = 0, fi = 0;
-      for (int sp = 0; sp < nsplit; sp++) {
-        const V2<T> v = part[(int64_t)sp * ldpart + r * ntarg + i];
-        fr += v.x;
-        fi += v.y;
+      if constexpr (RB > 1) {
+        for (int sp = 0; sp < nsplit; sp++) {
+          const V2<T> v = part[(int64_t)sp * ldpart + r * ntarg + i];
+          fr += v.x;
+          fi += v.y;
+        }
       }
       pot[r * ldpot + i] = {(T)(fr * (T)OVER4PI + (T)mr), (T)(fi * (T)OVER4PI + (T)mi)};
     }
@@ -581,14 +671,33 @@ __global__ void k_fill(int64_t n, T* __restrict__ a, T v) {
   if (i < n) a[i] = v;
 }
 
-__global__ void k_split_src(int64_t n, const double* __restrict__ s12, double* __restrict__ x, double* __restrict__ y,
-                            double* __restrict__ z, double* __restrict__ nx, double* __restrict__ ny,
-                            double* __restrict__ nz, int64_t stride) {
+// Source geometry records (normals scaled by ns; FP32 coordinates by unit32) from rows x y z
+// du dv n of 12 doubles
+__global__ void k_geo(int64_t n, const double* __restrict__ s12, double ns, double unit32,
+                      double* __restrict__ g64, float* __restrict__ g32) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const double* s = s12 + stride * i;
-  x[i] = s[0]; y[i] = s[1]; z[i] = s[2];
-  if (nx) { nx[i] = s[9]; ny[i] = s[10]; nz[i] = s[11]; }
+  const double* s = s12 + 12 * i;
+  const double v[6] = {s[0], s[1], s[2], ns * s[9], ns * s[10], ns * s[11]};
+  for (int m = 0; m < 6; m++) {
+    g64[GEO<double> * i + m] = v[m];
+    g32[GEO<float> * i + m] = (float)(m < 3 ? unit32 * v[m] : v[m]);
+  }
+  g32[GEO<float> * i + 6] = g32[GEO<float> * i + 7] = 0.0f;
+}
+
+struct Targets {
+  double* t64[3];
+  float* t32[3];
+};
+__global__ void k_split_targ(int64_t n, const double* __restrict__ t, int64_t stride, double unit32, Targets T) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  for (int m = 0; m < 3; m++) {
+    const double v = t[stride * i + m];
+    T.t64[m][i] = v;
+    T.t32[m][i] = (float)(unit32 * v);
+  }
 }
 
 template <typename A, typename B>
@@ -613,6 +722,11 @@ T* dal(size_t n) {
   if (hipMalloc(&p, (n ? n : 1) * sizeof(T)) != hipSuccess) return nullptr;
   return (T*)p;
 }
+
+// Workgroups of one wavefront that fill the chip twice (256 CUs x 4 SIMDs x 8 wavefronts)
+constexpr int64_t FAR_FILL = 16384;
+// Far-sum partials (splits x targets) up to which the CSR kernel sums them itself
+constexpr int64_t SPLIT_INLINE = (int64_t)1 << 19;
 
 inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
@@ -639,6 +753,25 @@ static T* own(ApplyPlan* P, size_t n) {
   return p;
 }
 
+// The far sum's kernel: alpha + beta t (1 - ikr) = (phase mu) (a + ns t (1 - ikr)) with mu the
+// power of two above |alpha| and |beta|, phase = beta / |beta| (1 without a double layer),
+// a = alpha / (phase mu) and ns = |beta| / mu: |a|, ns <= 1 in any units of alpha and beta,
+// and for beta = 1 (the usual double layer) no factor is rounded.
+static void apply_plan_scale(ApplyPlan* P) {
+  const double ar = P->alpha[0], ai = P->helm ? P->alpha[1] : 0.0;
+  const double br = P->beta[0], bi = P->helm ? P->beta[1] : 0.0;
+  const double bm = std::hypot(br, bi), m = std::max(std::hypot(ar, ai), bm);
+  int e = 0;
+  (void)std::frexp(m, &e);
+  const double mu = std::ldexp(1.0, e);
+  const double pr = bm > 0.0 ? br / bm : 1.0, pi = bm > 0.0 ? bi / bm : 0.0;
+  P->far_phase[0] = m > 0.0 ? pr * mu : 0.0;
+  P->far_phase[1] = m > 0.0 ? pi * mu : 0.0;
+  P->far_a[0] = (ar * pr + ai * pi) / mu;
+  P->far_a[1] = (ai * pr - ar * pi) / mu;
+  P->far_ns = bm / mu;
+}
+
 int apply_plan_build(ApplyPlan* P, const ApplyPlanInput& in, hipStream_t s) {
   P->npatches = in.npatches;
   P->npts = in.npts;
@@ -649,6 +782,7 @@ int apply_plan_build(ApplyPlan* P, const ApplyPlanInput& in, hipStream_t s) {
   P->zk[0] = in.zk[0]; P->zk[1] = in.zk[1];
   P->alpha[0] = in.alpha[0]; P->alpha[1] = in.alpha[1];
   P->beta[0] = in.beta[0]; P->beta[1] = in.beta[1];
+  apply_plan_scale(P);
   const int64_t npat = in.npatches, N = P->ntarg, NO = in.nptso;
   const double* tsrc = in.targs ? in.targs : in.srcvals;  // target coordinates
   const int64_t tstride = in.targs ? in.ndtarg : 12;
@@ -712,6 +846,11 @@ int apply_plan_build(ApplyPlan* P, const ApplyPlanInput& in, hipStream_t s) {
   const double diag = std::sqrt((mx[0] - mn[0]) * (mx[0] - mn[0]) + (mx[1] - mn[1]) * (mx[1] - mn[1]) +
                                 (mx[2] - mn[2]) * (mx[2] - mn[2]));
   P->phase_small = !in.helm || std::fabs(in.zk[0]) * diag * 0.15915494309189533577 < 200.0;
+  // FP32 coordinates in wavelengths where the phase is r itself (KIND 1); units so long or so
+  // short that FP32 powers of r could leave its range keep the caller's (KIND 2)
+  const double rev = in.zk[0] * 0.15915494309189533577;
+  P->wave32 = in.helm && in.zk[1] == 0.0 && P->phase_small && rev > 1e-6 && rev < 1e6;
+  P->unit32 = P->wave32 ? rev : 1.0;
   // the FP64 kernel evaluations take sin/cos of k r for |k r| <= SINCOS_RED_MAX
   if (in.helm && std::fabs(in.zk[0]) * diag > SINCOS_RED_MAX) {
     fprintf(stderr, "fmm3dbie_amd: |Re k| x surface diameter = %g exceeds %g\n", std::fabs(in.zk[0]) * diag,
@@ -734,10 +873,8 @@ int apply_plan_build(ApplyPlan* P, const ApplyPlanInput& in, hipStream_t s) {
   P->imat = own<double>(P, imat_all.size());
   P->wover = own<double>(P, NO);
   P->wover32 = own<float>(P, NO);
-  for (int c = 0; c < 6; c++) {
-    P->src64[c] = own<double>(P, NO);
-    P->src32[c] = own<float>(P, NO);
-  }
+  P->geo64 = own<double>(P, GEO<double> * NO);
+  P->geo32 = own<float>(P, GEO<float> * NO);
   for (int c = 0; c < 3; c++) {
     P->trg64[c] = own<double>(P, N);
     P->trg32[c] = own<float>(P, N);
@@ -782,16 +919,11 @@ int apply_plan_build(ApplyPlan* P, const ApplyPlanInput& in, hipStream_t s) {
     (void)hipFree(tmp);
   }
   if (nq > 0) k_convert<double, float><<<nblk(2 * nq, 256), 256, 0, s>>>(2 * nq, P->wnear64, P->wnear32);
-  if (NO > 0)
-    k_split_src<<<nblk(NO, 256), 256, 0, s>>>(NO, d_srcover, P->src64[0], P->src64[1], P->src64[2], P->src64[3],
-                                              P->src64[4], P->src64[5], 12);
+  if (NO > 0) k_geo<<<nblk(NO, 256), 256, 0, s>>>(NO, d_srcover, P->far_ns, P->unit32, P->geo64, P->geo32);
   if (N > 0)
-    k_split_src<<<nblk(N, 256), 256, 0, s>>>(N, d_srcvals, P->trg64[0], P->trg64[1], P->trg64[2], nullptr, nullptr,
-                                            nullptr, tstride);
-  if (NO > 0)
-    for (int c = 0; c < 6; c++) k_convert<double, float><<<nblk(NO, 256), 256, 0, s>>>(NO, P->src64[c], P->src32[c]);
-  if (N > 0)
-    for (int c = 0; c < 3; c++) k_convert<double, float><<<nblk(N, 256), 256, 0, s>>>(N, P->trg64[c], P->trg32[c]);
+    k_split_targ<<<nblk(N, 256), 256, 0, s>>>(N, d_srcvals, tstride, P->unit32,
+                                              Targets{{P->trg64[0], P->trg64[1], P->trg64[2]},
+                                                      {P->trg32[0], P->trg32[1], P->trg32[2]}});
   if (NO > 0) k_convert<double, float><<<nblk(NO, 256), 256, 0, s>>>(NO, P->wover, P->wover32);
   ACHK(hipGetLastError());
   ACHK(hipStreamSynchronize(s));
@@ -801,182 +933,231 @@ int apply_plan_build(ApplyPlan* P, const ApplyPlanInput& in, hipStream_t s) {
   return 0;
 }
 
+// Right-hand sides in whole groups of grp
+static int padded_rhs(int nrhs, int grp) { return (nrhs + grp - 1) / grp * grp; }
+// ... and the most that a block of nrhs takes with any group
+static int padded_rhs(int nrhs) { return nrhs == 1 ? 1 : padded_rhs(nrhs, MG); }
+
 static int ensure_ws(ApplyPlan* P, int nrhs) {
   if (P->ws_cap >= nrhs) return 0;
-  if (P->q64) { (void)hipFree(P->q64); (void)hipFree(P->m64); (void)hipFree(P->q32); (void)hipFree(P->m32); }
-  if (P->part64) { (void)hipFree(P->part64); (void)hipFree(P->part32); }
-  if (P->sig64c) (void)hipFree(P->sig64c);
-  if (P->pot64c) (void)hipFree(P->pot64c);
-  const size_t NO = P->nptso;
-  P->q64 = dal<double>(2 * NO * nrhs);
-  P->m64 = dal<double>(2 * NO * nrhs);
-  P->q32 = dal<float>(2 * NO * nrhs);
-  P->m32 = dal<float>(2 * NO * nrhs);
+  apply_plan_free_ws(P);
+  const size_t ns = (size_t)P->nptso * padded_rhs(nrhs);
+  P->str64 = dal<double>(2 * ns);
+  P->str32 = dal<float>(2 * ns);
   P->sig64c = dal<double>(2 * (size_t)P->npts);
   P->pot64c = dal<double>(2 * (size_t)P->ntarg);
   // partial far sums: nsplit x nrhs x npts with nsplit x nrhs <= far_split_cap x 64
   const size_t npart = (size_t)P->far_split_cap * 64 * P->ntarg;
   P->part64 = dal<double>(2 * npart);
   P->part32 = dal<float>(2 * npart);
-  if (!P->q64 || !P->m64 || !P->q32 || !P->m32 || !P->sig64c || !P->pot64c || !P->part64 || !P->part32) return -2;
+  if (!P->str64 || !P->str32 || !P->sig64c || !P->pot64c || !P->part64 || !P->part32) return -2;
   P->ws_cap = nrhs;
   return 0;
 }
 
 void apply_plan_free_ws(ApplyPlan* P) {
-  void* ps[] = {P->q64, P->m64, P->q32, P->m32, P->sig64c, P->pot64c, P->part64, P->part32};
+  void* ps[] = {P->str64, P->sig64c, P->pot64c, P->part64, P->str32, P->part32};
   for (void* p : ps)
     if (p) (void)hipFree(p);
-  P->q64 = P->m64 = P->sig64c = P->pot64c = P->part64 = nullptr;
-  P->q32 = P->m32 = P->part32 = nullptr;
+  P->str64 = P->sig64c = P->pot64c = P->part64 = nullptr;
+  P->str32 = P->part32 = nullptr;
   P->ws_cap = 0;
 }
 
-// Far sum of nrhs right-hand sides in groups of NRHS (grid z), then the reduction over
-// source splits fused with the CSR correction (uniform p) or followed by the general CSR
-// kernel.  The split count keeps the grid at >= wg_target workgroups, within the partial
-// buffer (far_split_cap x 64 x npts).
-template <typename T, int NRHS>
-static int launch_far(ApplyPlan* P, bool mask, int64_t wg_target, const V2<T>* q, const V2<T>* m, int64_t ldstr,
-                      int nrhs, V2<T>* part, int64_t part_cap, int64_t* nsplit_out, hipStream_t s) {
-  const T* const* src;
-  const T* const* trg;
+template <typename T>
+static FarPar<T> far_par(const ApplyPlan* P) {
+  const double zr = P->helm ? P->zk[0] : 0.0, zi = P->helm ? P->zk[1] : 0.0;
+  FarPar<T> F;
+  F.ar = (T)P->far_a[0];
+  F.ai = (T)P->far_a[1];
+  F.kr = (T)zr;
+  F.ki = (T)zi;
   if constexpr (sizeof(T) == 8) {
-    src = (const T* const*)P->src64;
-    trg = (const T* const*)P->trg64;
+    double hi, lo;
+    half_turns(zr, hi, lo);
+    F.khi = hi;
+    F.klo = lo;
   } else {
-    src = (const T* const*)P->src32;
-    trg = (const T* const*)P->trg32;
+    F.khi = (T)(zr * 0.15915494309189533577);  // k / (2 pi)
+    F.klo = (T)0;
+    // in wavelengths: a + t (1 - ikr) and 1 / r, each over the unit, the rest in the strengths
+    F.ar = (T)(P->far_a[0] / P->unit32);
+    F.ai = (T)(P->far_a[1] / P->unit32);
+    if (P->wave32) F.kr = (T)6.283185307179586;
   }
-  const T kr = (T)(P->helm ? P->zk[0] : 0.0), ki = (T)(P->helm ? P->zk[1] : 0.0);
-  const T krev = (T)(P->helm ? P->zk[0] * 0.15915494309189533577 : 0.0);  // k / (2 pi)
+  return F;
+}
+
+// Kernel form (FarPar's KIND) of a plan in precision T
+template <typename T>
+static int far_kind(const ApplyPlan* P) {
+  if (!P->helm) return 0;
+  return P->zk[1] != 0.0 || (sizeof(T) == 4 && !P->wave32) ? 2 : 1;
+}
+
+template <typename T>
+static const T* const* targets_of(const ApplyPlan* P) {
+  if constexpr (sizeof(T) == 8) return (const T* const*)P->trg64;
+  else return (const T* const*)P->trg32;
+}
+template <typename T>
+static const T* sources_of(const ApplyPlan* P) {
+  if constexpr (sizeof(T) == 8) return P->geo64;
+  else return P->geo32;
+}
+
+// Source splits and sources per split (a multiple of tile) of a far sum whose launch has g
+// workgroups per split: up to wg_target workgroups, within the partial buffer, and no
+// split below 256 sources (its partial sums would cost more than the balance gains)
+// unless the launch would leave slots empty (fewer than `fill` workgroups).
+static int64_t split_sources(int64_t nsrc, int tile, int64_t g, int64_t wg_target, int64_t fill, int64_t cap,
+                             int64_t* chunk) {
+  const int64_t ntiles = (nsrc + tile - 1) / tile;
+  int64_t nsplit = (wg_target + g - 1) / g;
+  const int64_t need = (fill + g - 1) / g;
+  nsplit = std::min(nsplit, std::max((nsrc + 255) / 256, need));
+  nsplit = std::max<int64_t>(1, std::min({nsplit, cap, ntiles}));
+  *chunk = ((ntiles + nsplit - 1) / nsplit) * tile;
+  return (nsrc + *chunk - 1) / *chunk;
+}
+
+// Far sum of nrhs right-hand sides in groups of NRHS (grid z).
+template <typename T, int NRHS>
+static int launch_far(ApplyPlan* P, bool mask, int64_t wg_target, const V2<T>* str, int nrhs, V2<T>* part,
+                      int64_t part_cap, int64_t* nsplit_out, hipStream_t s) {
+  const T* const* trg = targets_of<T>(P);
+  const unsigned g = nblk(P->ntarg, 64);
+  const int ngrp = (nrhs + NRHS - 1) / NRHS;
+  int64_t chunk;
+  const int64_t nsplit = split_sources(P->nptso, STILE, (int64_t)g * ngrp, 4 * wg_target, FAR_FILL,
+                                       part_cap / ((int64_t)nrhs * P->ntarg), &chunk);
+  const dim3 grid(g, (unsigned)nsplit, (unsigned)ngrp);
   const T th2 = (T)(P->thresh * P->thresh);
-  const unsigned g = nblk(P->ntarg, TPB);
-  const int ngrp = nrhs / NRHS;
-  const int64_t ntiles = (P->nptso + TPB - 1) / TPB;
-  int64_t nsplit = (wg_target + (int64_t)g * ngrp - 1) / ((int64_t)g * ngrp);
-  // splits that fit the partial buffer (part_cap complex values)
-  const int64_t cap = part_cap / ((int64_t)nrhs * (P->ntarg > 0 ? P->ntarg : 1));
-  if (nsplit > cap) nsplit = cap;
-  if (nsplit > ntiles) nsplit = ntiles;
-  if (nsplit < 1) nsplit = 1;
-  const int64_t chunk = ((ntiles + nsplit - 1) / nsplit) * TPB;
-  nsplit = (P->nptso + chunk - 1) / chunk;
-  const int64_t ldpart = (int64_t)nrhs * P->ntarg;
-  dim3 grid(g, (unsigned)nsplit, (unsigned)ngrp);
-#define FMM_FAR(MK, CKV)                                                                                       \
-  k_farsum<T, MK, CKV, NRHS><<<grid, TPB, 0, s>>>(P->ntarg, trg[0], trg[1], trg[2], P->nptso, src[0], src[1], src[2], \
-                                                  src[3], src[4], src[5], P->ixyzso, q, m, ldstr, P->row_ptr,       \
-                                                  P->near_sorted, kr, krev, ki, th2, chunk, part, ldpart)
-  const bool ck = ki != (T)0 || (sizeof(T) == 4 && !P->phase_small);
-  if (mask) {
-    if (ck) FMM_FAR(true, true);
-    else FMM_FAR(true, false);
-  } else {
-    if (ck) FMM_FAR(false, true);
-    else FMM_FAR(false, false);
+#define FMM_FAR(MK, KD)                                                                                     \
+  k_farsum<T, MK, KD, NRHS><<<grid, 64, 0, s>>>((int)P->ntarg, trg[0], trg[1], trg[2], (int)P->nptso,       \
+                                                sources_of<T>(P), P->ixyzso, str, P->row_ptr, P->near_sorted, \
+                                                far_par<T>(P), th2, (int)chunk, nrhs, part, (int64_t)nrhs * P->ntarg)
+  const int kind = far_kind<T>(P);
+  if (mask || sizeof(T) == 4) {
+    if (kind == 0) FMM_FAR(true, 0);
+    else if (kind == 1) FMM_FAR(true, 1);
+    else FMM_FAR(true, 2);
+  } else if constexpr (sizeof(T) == 8) {
+    if (kind == 0) FMM_FAR(false, 0);
+    else if (kind == 1) FMM_FAR(false, 1);
+    else FMM_FAR(false, 2);
   }
 #undef FMM_FAR
   *nsplit_out = nsplit;
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// The matrix-core far sum: 16 right-hand sides of one group per launch column, FP32,
-// near patches masked; 64 targets per workgroup, the source range split as for k_farsum.
-static int launch_far_mfma(ApplyPlan* P, int64_t wg_target, const V2<float>* q, const V2<float>* m,
-                           int64_t ldstr, int nrhs, V2<float>* part, int64_t part_cap, int64_t* nsplit_out,
-                           hipStream_t s) {
-  const float* const* src = (const float* const*)P->src32;
-  const float* const* trg = (const float* const*)P->trg32;
-  const float kr = (float)(P->helm ? P->zk[0] : 0.0), ki = (float)(P->helm ? P->zk[1] : 0.0);
-  const float krev = (float)(P->helm ? P->zk[0] * 0.15915494309189533577 : 0.0);  // k / (2 pi)
-  const unsigned g = nblk(P->ntarg, 16 * FW);
-  const int ngrp = nrhs / 16;
-  const int64_t ntiles = (P->nptso + FT - 1) / FT;
-  int64_t nsplit = (wg_target + (int64_t)g * ngrp - 1) / ((int64_t)g * ngrp);
-  const int64_t cap = part_cap / ((int64_t)nrhs * (P->ntarg > 0 ? P->ntarg : 1));
-  if (nsplit > cap) nsplit = cap;
-  if (nsplit > ntiles) nsplit = ntiles;
-  if (nsplit < 1) nsplit = 1;
-  const int64_t chunk = ((ntiles + nsplit - 1) / nsplit) * FT;
-  nsplit = (P->nptso + chunk - 1) / chunk;
-  const int64_t ldpart = (int64_t)nrhs * P->ntarg;
-  dim3 grid(g, (unsigned)nsplit, (unsigned)ngrp);
-#define FMM_FARM(CKV)                                                                                          \
-  k_farsum_mfma<CKV><<<grid, 64 * FW, 0, s>>>(P->ntarg, trg[0], trg[1], trg[2], P->nptso, src[0], src[1], src[2], \
-                                             src[3], src[4], src[5], P->ixyzso, q, m, ldstr, P->row_ptr,         \
-                                             P->near_sorted, kr, krev, ki, chunk, part, ldpart)
-  if (ki != 0.0f || !P->phase_small) FMM_FARM(true);
-  else FMM_FARM(false);
+// The matrix-core far sum: groups of 16 right-hand sides, the last one padded with zeros.
+template <typename T>
+static int launch_far_mfma(ApplyPlan* P, bool mask, int64_t wg_target, const V2<T>* str, int nrhs, V2<T>* part,
+                           int64_t part_cap, int64_t* nsplit_out, hipStream_t s) {
+  const T* const* trg = targets_of<T>(P);
+  const unsigned g = nblk(P->ntarg, 16 * FW * MT<T>);
+  const int ngrp = (nrhs + MG - 1) / MG;
+  int64_t chunk;
+  const int64_t nsplit = split_sources(P->nptso, FT, (int64_t)g * ngrp, wg_target, FAR_FILL / FW,
+                                       part_cap / ((int64_t)nrhs * P->ntarg), &chunk);
+  const dim3 grid(g, (unsigned)nsplit, (unsigned)ngrp);
+  const T th2 = (T)(P->thresh * P->thresh);
+#define FMM_FARM(MK, KD)                                                                                       \
+  k_farsum_mfma<T, MK, KD><<<grid, 64 * FW, 0, s>>>((int)P->ntarg, trg[0], trg[1], trg[2], (int)P->nptso,      \
+                                                   sources_of<T>(P), P->ixyzso, str, P->row_ptr,               \
+                                                   P->near_sorted, far_par<T>(P), th2, (int)chunk, nrhs, part, \
+                                                   (int64_t)nrhs * P->ntarg)
+  const int kind = far_kind<T>(P);
+  if (mask || sizeof(T) == 4) {
+    if (kind == 0) FMM_FARM(true, 0);
+    else if (kind == 1) FMM_FARM(true, 1);
+    else FMM_FARM(true, 2);
+  } else if constexpr (sizeof(T) == 8) {
+    if (kind == 0) FMM_FARM(false, 0);
+    else if (kind == 1) FMM_FARM(false, 1);
+    else FMM_FARM(false, 2);
+  }
 #undef FMM_FARM
   *nsplit_out = nsplit;
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-template <typename T>
-static int far_group(const ApplyPlan* P, int nrhs, int prec, int64_t* wg) {
+// Right-hand sides per far-sum group: tuned, or by default the smallest of 1, 2, 4, 8 that
+// holds the block, and 16 (matrix cores) beyond; a last group is padded with zeros.  Measured
+// in cycles of a SIMD per 64 pairs (43008 x 70000 pairs, Helmholtz): FP64 262 / 280 / 316 for
+// 1, 2 and 4 densities and 466 for 16; FP32 98 / 110 / 140 and 217.  str_cap: strengths
+// (complex values) that fit the buffer of the call; a padded block that does not falls back
+// to a group that divides nrhs.
+static int far_group(const ApplyPlan* P, int nrhs, int prec, int64_t str_cap, int64_t* wg) {
   const auto it = P->tuned.find(prec * 1000 + nrhs);
-  if (it != P->tuned.end()) {
-    *wg = it->second.second;
-    return it->second.first;
+  *wg = it != P->tuned.end() ? it->second.second : P->far_wg_target;
+  int grp = it != P->tuned.end() ? it->second.first : 1;
+  if (it == P->tuned.end())
+    while (grp < nrhs && grp < MG) grp *= 2;
+  while (P->nptso * padded_rhs(nrhs, grp) > str_cap || grp > MG) {
+    grp /= 2;
+    while (nrhs % grp != 0) grp /= 2;
   }
-  *wg = P->far_wg_target;
-  if (sizeof(T) == 4 && nrhs % 16 == 0) return 16;  // the matrix-core far sum
-  const int pref = sizeof(T) == 8 ? 4 : 8;
-  for (int gsz = pref; gsz > 1; gsz >>= 1)
-    if (nrhs % gsz == 0) return gsz;
-  return 1;
+  return grp;
 }
 
 template <typename T>
-static int dispatch_far(ApplyPlan* P, bool mask, int grp, int64_t wg, const V2<T>* q, const V2<T>* m, int64_t ldstr,
-                        int nrhs, V2<T>* part, int64_t part_cap, int64_t* nsplit, hipStream_t s) {
+static int dispatch_far(ApplyPlan* P, bool mask, int grp, int64_t wg, const V2<T>* str, int nrhs, V2<T>* part,
+                        int64_t part_cap, int64_t* nsplit, hipStream_t s) {
   switch (grp) {
-    case 1: return launch_far<T, 1>(P, mask, wg, q, m, ldstr, nrhs, part, part_cap, nsplit, s);
-    case 2: return launch_far<T, 2>(P, mask, wg, q, m, ldstr, nrhs, part, part_cap, nsplit, s);
-    case 4: return launch_far<T, 4>(P, mask, wg, q, m, ldstr, nrhs, part, part_cap, nsplit, s);
-    case 8: return launch_far<T, 8>(P, mask, wg, q, m, ldstr, nrhs, part, part_cap, nsplit, s);
-    case 16:
-      if constexpr (sizeof(T) == 4) {
-        if (mask) return launch_far_mfma(P, wg, q, m, ldstr, nrhs, part, part_cap, nsplit, s);
-        return launch_far<T, 16>(P, mask, wg, q, m, ldstr, nrhs, part, part_cap, nsplit, s);
-      }
-      return -6;
+    case 1: return launch_far<T, 1>(P, mask, wg, str, nrhs, part, part_cap, nsplit, s);
+    case 2: return launch_far<T, 2>(P, mask, wg, str, nrhs, part, part_cap, nsplit, s);
+    case 4: return launch_far<T, 4>(P, mask, wg, str, nrhs, part, part_cap, nsplit, s);
+    case 8: return launch_far<T, 8>(P, mask, wg, str, nrhs, part, part_cap, nsplit, s);
+    case MG: return launch_far_mfma<T>(P, mask, wg, str, nrhs, part, part_cap, nsplit, s);
     default: return -6;
   }
 }
 
-// pot = far (+ CSR) for all right-hand sides
+// pot = far (+ CSR, and with sub the near subtraction) for all right-hand sides
 template <typename T>
-static int far_and_csr(ApplyPlan* P, int prec, bool mask, const V2<T>* q, const V2<T>* m, const V2<T>* sg,
+static int far_and_csr(ApplyPlan* P, bool mask, bool sub, int grp, int64_t wg, const V2<T>* str, const V2<T>* sg,
                        V2<T>* pt, int nrhs, V2<T>* part, int64_t part_cap, hipStream_t s, hipEvent_t ev_far) {
   const int64_t N = P->ntarg, NO = P->nptso, NS = P->npts;
   const V2<T>* wn = (const V2<T>*)(sizeof(T) == 8 ? (void*)P->wnear64 : (void*)P->wnear32);
   int64_t nsplit = 0;
   if (N == 0) return 0;
   if (NO > 0) {
-    int64_t wg;
-    const int grp = far_group<T>(P, nrhs, prec, &wg);
-    const int rc = dispatch_far<T>(P, mask, grp, wg, q, m, NO, nrhs, part, part_cap, &nsplit, s);
+    const int rc = dispatch_far<T>(P, mask, grp, wg, str, nrhs, part, part_cap, &nsplit, s);
     if (rc) return rc;
   }
   if (ev_far) ACHK(hipEventRecord(ev_far, s));
-  if (nsplit > 4) {
-    // many source splits: one coalesced pass over the partials before the per-target CSR
+  SubArgs S = {};
+  if constexpr (sizeof(T) == 8)
+    S = {P->trg64[0], P->trg64[1], P->trg64[2], P->geo64, str, NO, grp, P->col_ind, P->ixyzso, far_par<double>(P),
+         P->thresh * P->thresh};
+  // many source splits: one coalesced pass over the partials first; the partials of one
+  // right-hand side of a small problem are summed by the lanes of the CSR kernel instead
+  // (a launch less; their strided reads stay in L2)
+  if (nsplit > 4 && !(nrhs == 1 && P->uniform_p > 0 && nsplit * N <= SPLIT_INLINE)) {
     k_split_sum<T><<<dim3((unsigned)((N + 63) / 64), (unsigned)nrhs), 256, 0, s>>>(N, (int)nsplit, part,
                                                                                   (int64_t)nrhs * N);
     nsplit = 1;
   }
   if (P->uniform_p > 0) {
-#define FMM_CSR(PC)                                                                                             \
-  if (nrhs == 1)                                                                                               \
-    k_reduce_csr<T, T, 1, PC><<<nblk(N, 4), 256, 0, s>>>(N, nrhs, (int)nsplit, part, (int64_t)nrhs * N,         \
-                                                         P->row_ptr, P->csr_src, P->iquad, P->uniform_p, wn, sg, \
-                                                         NS, pt, N);                                             \
-  else                                                                                                         \
-    k_reduce_csr<T, T, 8, PC><<<nblk(N, 4), 256, 0, s>>>(N, nrhs, (int)nsplit, part, (int64_t)nrhs * N,         \
-                                                         P->row_ptr, P->csr_src, P->iquad, P->uniform_p, wn, sg, \
-                                                         NS, pt, N)
+#define FMM_CSR1(RB, PC, SB)                                                                                    \
+  k_reduce_csr<T, T, RB, PC, SB><<<nblk(N, 4), 256, 0, s>>>(N, nrhs, (int)nsplit, part, (int64_t)nrhs * N,       \
+                                                            P->row_ptr, P->csr_src, P->iquad, P->uniform_p, wn, \
+                                                            sg, NS, pt, N, S)
+#define FMM_CSR(PC)                                        \
+  do {                                                     \
+    if constexpr (sizeof(T) == 8) {                        \
+      if (sub) {                                           \
+        if (nrhs == 1) FMM_CSR1(1, PC, true);              \
+        else FMM_CSR1(8, PC, true);                        \
+        break;                                             \
+      }                                                    \
+    }                                                      \
+    if (nrhs == 1) FMM_CSR1(1, PC, false);                 \
+    else FMM_CSR1(8, PC, false);                           \
+  } while (0)
     switch (P->uniform_p) {
       case 3: FMM_CSR(3); break;
       case 6: FMM_CSR(6); break;
@@ -991,6 +1172,7 @@ static int far_and_csr(ApplyPlan* P, int prec, bool mask, const V2<T>* q, const 
       default: FMM_CSR(0);
     }
 #undef FMM_CSR
+#undef FMM_CSR1
   } else {
     if (nsplit > 0)
       k_farsum_reduce<T><<<dim3(nblk(N, 256), nrhs), 256, 0, s>>>(N, nrhs, (int)nsplit, part, (int64_t)nrhs * N, pt,
@@ -999,75 +1181,69 @@ static int far_and_csr(ApplyPlan* P, int prec, bool mask, const V2<T>* q, const 
       k_fill<T><<<nblk(2 * N * nrhs, 256), 256, 0, s>>>(2 * N * nrhs, (T*)pt, (T)0);
     k_csr_gen<T, T><<<nblk(N, 256), 256, 0, s>>>(N, P->row_ptr, P->col_ind, P->iquad, P->ixyzs, wn, sg, NS, nrhs,
                                                  pt, N);
+    if constexpr (sizeof(T) == 8)
+      if (sub) k_near_sub<<<nblk(N, 4), 256, 0, s>>>(N, P->row_ptr, S, nrhs, pt, N);
   }
   ACHK(hipGetLastError());
   return 0;
 }
 
-// Work buffers of one apply in the precision of the call: charge and dipole strengths
-// at the oversampled nodes (nptso x nrhs complex each) and the far-sum partials
-// (part_cap complex values, at least ntarg x nrhs: one source split).
+// Work buffers of one apply in the precision of the call: strengths at the oversampled nodes
+// (str_cap complex values, at least nptso x nrhs) and the far-sum partials (part_cap complex
+// values, at least ntarg x nrhs: one source split).
 struct ApplyWs {
-  void *q, *m, *part;
-  int64_t part_cap;
+  void *str, *part;
+  int64_t str_cap, part_cap;
 };
 
+template <typename T>
+static void oversample(ApplyPlan* P, const V2<T>* sigma, int nrhs, int grp, V2<T>* str, hipStream_t s) {
+  const int64_t NO = P->nptso;
+  const int nr = padded_rhs(nrhs, grp);
+  const T* wover;
+  if constexpr (sizeof(T) == 8) wover = P->wover;
+  else wover = P->wover32;
+  const double scale = sizeof(T) == 4 ? P->unit32 * P->unit32 : 1.0;
+#define FMM_OVER(RB)                                                                                             \
+  k_oversample<T, RB><<<dim3(nblk(NO, 256), (unsigned)(nr / RB)), 256, 0, s>>>(                                  \
+      NO, P->opatch, P->ixyzs, P->ixyzso, P->ioff, P->np_of, P->imat, sigma, nrhs, P->npts, wover,               \
+      scale * P->far_phase[0], scale * P->far_phase[1], grp, str)
+  if (grp % 4 == 0) FMM_OVER(4);
+  else if (grp == 2) FMM_OVER(2);
+  else FMM_OVER(1);
+#undef FMM_OVER
+}
+
 // sigma/pot: complex (interleaved) device arrays of length npts * nrhs, leading dim npts
+template <typename T>
+static int apply_run_t(ApplyPlan* P, bool mask, const void* sigma, void* pot, int nrhs, hipStream_t s,
+                       const ApplyWs& W, hipEvent_t* ev) {
+  int64_t wg;
+  const int grp = far_group(P, nrhs, sizeof(T) * 8, W.str_cap, &wg);
+  if (P->nptso > 0) oversample<T>(P, (const V2<T>*)sigma, nrhs, grp, (V2<T>*)W.str, s);
+  if (ev) ACHK(hipEventRecord(ev[1], s));
+  return far_and_csr<T>(P, mask, !mask, grp, wg, (const V2<T>*)W.str, (const V2<T>*)sigma, (V2<T>*)pot, nrhs,
+                        (V2<T>*)W.part, W.part_cap, s, ev ? ev[2] : nullptr);
+}
+
 static int apply_run_ws(ApplyPlan* P, int prec, int mode, const void* sigma, void* pot, int nrhs, hipStream_t s,
                         ApplyTimes* tm, const ApplyWs& W) {
-  const int64_t N = P->npts, NT = P->ntarg, NO = P->nptso;
-  const double ar = P->alpha[0], ai = P->helm ? P->alpha[1] : 0.0;
-  const double br = P->beta[0], bi = P->helm ? P->beta[1] : 0.0;
-  hipEvent_t ev[5];
+  hipEvent_t ev[4];
   if (tm)
     for (auto& e : ev) ACHK(hipEventCreate(&e));
   if (tm) ACHK(hipEventRecord(ev[0], s));
-  int rc = 0;
-  if (prec == 64) {
-    const V2<double>* sg = (const V2<double>*)sigma;
-    V2<double>* pt = (V2<double>*)pot;
-    if (NO > 0)
-      k_oversample<double><<<nblk(NO, 256), 256, 0, s>>>(NO, P->opatch, P->ixyzs, P->ixyzso, P->ioff, P->np_of, P->imat,
-                                                       sg, nrhs, N, P->wover, ar, ai, br, bi,
-                                                       (V2<double>*)W.q, (V2<double>*)W.m, NO);
-    if (tm) ACHK(hipEventRecord(ev[1], s));
-    const bool mask = mode == APPLY_MASKED;
-    auto* q = (const V2<double>*)W.q;
-    auto* m = (const V2<double>*)W.m;
-    rc = far_and_csr<double>(P, 64, mask, q, m, sg, pt, nrhs, (V2<double>*)W.part, W.part_cap, s,
-                             tm ? ev[2] : nullptr);
-    if (tm) ACHK(hipEventRecord(ev[3], s));
-    if (!rc && !mask) {
-      const double kr = P->helm ? P->zk[0] : 0.0, ki = P->helm ? P->zk[1] : 0.0;
-      if (NT > 0)
-        k_near_sub<<<nblk(NT, 4), 256, 0, s>>>(NT, P->trg64[0], P->trg64[1], P->trg64[2], P->src64[0], P->src64[1],
-                                               P->src64[2], P->src64[3], P->src64[4], P->src64[5], q, m, NO, nrhs,
-                                               P->row_ptr, P->col_ind, P->ixyzso, kr, ki, P->thresh * P->thresh, pt,
-                                               NT);
-    }
-    if (tm) ACHK(hipEventRecord(ev[4], s));
-  } else {
-    const V2<float>* sg = (const V2<float>*)sigma;
-    V2<float>* pt = (V2<float>*)pot;
-    if (NO > 0)
-      k_oversample<float><<<nblk(NO, 256), 256, 0, s>>>(NO, P->opatch, P->ixyzs, P->ixyzso, P->ioff, P->np_of, P->imat,
-                                                      sg, nrhs, N, P->wover32, ar, ai, br, bi, (V2<float>*)W.q,
-                                                      (V2<float>*)W.m, NO);
-    if (tm) ACHK(hipEventRecord(ev[1], s));
-    rc = far_and_csr<float>(P, 32, true, (const V2<float>*)W.q, (const V2<float>*)W.m, sg, pt, nrhs,
-                            (V2<float>*)W.part, W.part_cap, s, tm ? ev[2] : nullptr);
-    if (tm) ACHK(hipEventRecord(ev[3], s));
-    if (tm) ACHK(hipEventRecord(ev[4], s));
-  }
+  const int rc = prec == 64 ? apply_run_t<double>(P, mode == APPLY_MASKED, sigma, pot, nrhs, s, W, tm ? ev : nullptr)
+                            : apply_run_t<float>(P, true, sigma, pot, nrhs, s, W, tm ? ev : nullptr);
+  if (tm) ACHK(hipEventRecord(ev[3], s));
   if (rc) return rc;
   ACHK(hipGetLastError());
   if (tm) {
-    ACHK(hipEventSynchronize(ev[4]));
+    ACHK(hipEventSynchronize(ev[3]));
     float ms;
     (void)hipEventElapsedTime(&ms, ev[0], ev[1]); tm->ms_over = ms;
     (void)hipEventElapsedTime(&ms, ev[1], ev[2]); tm->ms_far = ms;
     (void)hipEventElapsedTime(&ms, ev[2], ev[3]); tm->ms_csr = ms;
-    (void)hipEventElapsedTime(&ms, ev[3], ev[4]); tm->ms_sub = ms;
+    tm->ms_sub = 0.0;  // within ms_csr: one kernel
     for (auto& e : ev) (void)hipEventDestroy(e);
   }
   return 0;
@@ -1083,9 +1259,9 @@ static int check_prec_nrhs(int prec, int nrhs) {
 }
 
 static ApplyWs plan_ws(const ApplyPlan* P, int prec) {
-  const int64_t cap = (int64_t)P->far_split_cap * 64 * P->ntarg;
-  if (prec == 64) return {P->q64, P->m64, P->part64, cap};
-  return {P->q32, P->m32, P->part32, cap};
+  const int64_t cap = (int64_t)P->far_split_cap * 64 * P->ntarg, str = P->nptso * padded_rhs(P->ws_cap);
+  if (prec == 64) return {P->str64, P->part64, str, cap};
+  return {P->str32, P->part32, str, cap};
 }
 
 // sigma/pot: complex (interleaved) device arrays of length npts * nrhs, leading dim npts;
@@ -1143,52 +1319,48 @@ int apply_plan_run_noalloc(ApplyPlan* P, int prec, int mode, const void* sigma, 
   }
   unsigned char* base = (unsigned char*)scratch_address();
   if (!base) return -1;
+  // strengths in the first two blocks, partials in the rest
   ApplyWs W;
-  W.q = base;
-  W.m = base + strength;
+  W.str = base;
+  W.str_cap = (int64_t)(2 * strength / cs);
   W.part = base + 2 * strength;
   W.part_cap = (int64_t)((APPLY_SCRATCH_BYTES - 2 * strength) / cs);
   return apply_run_ws(P, prec, mode, sigma, pot, nrhs, s, nullptr, W);
 }
 
-// Autotuner of the far-sum launch shape for (prec, nrhs): every right-hand-side group
-// size that divides nrhs (1..8 in FP64, 1..16 in FP32) and workgroup targets of 1024,
-// 4096, 8192, 16384, 32768 are timed (one warm-up launch, then one launch each) on unit
-// densities; the fastest is kept
-// in the plan and used by every later apply with the same (prec, nrhs).
+// Autotuner of the far-sum launch shape for (prec, nrhs): every right-hand-side group size
+// that divides nrhs (1..16; in FP64 blocks of 16 and more leave out the group of one, 16 times
+// the kernel values of the matrix cores) and workgroup targets of 4096, 8192, 16384, 32768
+// are timed (one warm-up launch, then one launch each) on unit densities; the fastest is
+// kept in the plan and used by every later apply with the same (prec, nrhs).
 int apply_plan_tune(ApplyPlan* P, int prec, int nrhs, hipStream_t s, double* report, int nreport) {
   if (nrhs < 1 || nrhs > 64 || (prec != 32 && prec != 64)) return -6;
   if (ensure_ws(P, nrhs) != 0) return -2;
   if (P->ntarg == 0 || P->nptso == 0) return 0;
-  const int64_t NO = P->nptso;
-  if (prec == 64) {
-    k_fill<double><<<nblk(2 * NO * nrhs, 256), 256, 0, s>>>(2 * NO * nrhs, P->q64, 1.0);
-    k_fill<double><<<nblk(2 * NO * nrhs, 256), 256, 0, s>>>(2 * NO * nrhs, P->m64, 1.0);
-  } else {
-    k_fill<float><<<nblk(2 * NO * nrhs, 256), 256, 0, s>>>(2 * NO * nrhs, P->q32, 1.0f);
-    k_fill<float><<<nblk(2 * NO * nrhs, 256), 256, 0, s>>>(2 * NO * nrhs, P->m32, 1.0f);
-  }
+  const int64_t nval = 2 * P->nptso * padded_rhs(nrhs);
+  if (prec == 64) k_fill<double><<<nblk(nval, 256), 256, 0, s>>>(nval, P->str64, 1.0);
+  else k_fill<float><<<nblk(nval, 256), 256, 0, s>>>(nval, P->str32, 1.0f);
   auto far = [&](int gsz, int64_t wg) {
     int64_t nsplit;
     const int64_t cap = (int64_t)P->far_split_cap * 64 * P->ntarg;
-    return prec == 64 ? dispatch_far<double>(P, true, gsz, wg, (const V2<double>*)P->q64, (const V2<double>*)P->m64,
-                                             NO, nrhs, (V2<double>*)P->part64, cap, &nsplit, s)
-                      : dispatch_far<float>(P, true, gsz, wg, (const V2<float>*)P->q32, (const V2<float>*)P->m32, NO,
-                                            nrhs, (V2<float>*)P->part32, cap, &nsplit, s);
+    return prec == 64 ? dispatch_far<double>(P, true, gsz, wg, (const V2<double>*)P->str64, nrhs,
+                                             (V2<double>*)P->part64, cap, &nsplit, s)
+                      : dispatch_far<float>(P, true, gsz, wg, (const V2<float>*)P->str32, nrhs,
+                                            (V2<float>*)P->part32, cap, &nsplit, s);
   };
   hipEvent_t e0, e1;
   ACHK(hipEventCreate(&e0));
   ACHK(hipEventCreate(&e1));
-  const int groups[5] = {1, 2, 4, 8, 16};
+  const int groups[5] = {1, 2, 4, 8, MG};
   const int64_t wgs[4] = {4096, 8192, 16384, 32768};
   float best = 1e30f;
   int bg = 1, nrep = 0;
   int64_t bw = P->far_wg_target;
   // one warm-up launch, then one timed launch per shape
-  int rc = far(1, P->far_wg_target);
+  int rc = far(nrhs % MG == 0 ? MG : 1, P->far_wg_target);
   if (rc) return rc;
   for (int gsz : groups) {
-    if (nrhs % gsz != 0 || (prec == 64 && gsz > 8)) continue;
+    if (nrhs % gsz != 0 || (prec == 64 && gsz == 1 && nrhs % MG == 0)) continue;
     for (int64_t wg : wgs) {
       ACHK(hipEventRecord(e0, s));
       rc = far(gsz, wg);

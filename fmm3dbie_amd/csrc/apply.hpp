@@ -33,8 +33,12 @@ struct ApplyPlan {
   int64_t npatches = 0, npts = 0, nptso = 0, nnz = 0, nquad = 0;
   int64_t ntarg = 0;  // targets (rows of the near list); npts for the on-surface operator
   double zk[2] = {0, 0}, alpha[2] = {0, 0}, beta[2] = {0, 0};
+  // alpha + beta t (1 - ikr) = far_phase (far_a + far_ns t (1 - ikr)), t the dipole factor
+  double far_phase[2] = {0, 0}, far_a[2] = {0, 0}, far_ns = 0;
   double thresh = 0;
   bool phase_small = true;  // FP32 phases within the hardware sine's range (no reduction)
+  double unit32 = 1.0;      // FP32 coordinates are unit32 times the caller's
+  bool wave32 = false;      // ... in wavelengths: r is the phase in revolutions
   int uniform_p = 0;
   int64_t *ixyzs = nullptr, *ixyzso = nullptr, *row_ptr = nullptr, *col_ind = nullptr, *iquad = nullptr,
           *ioff = nullptr;
@@ -43,16 +47,16 @@ struct ApplyPlan {
   double* imat = nullptr;
   double* wover = nullptr;
   float* wover32 = nullptr;
-  double* src64[6] = {};
-  float* src32[6] = {};
+  double* geo64 = nullptr;  // source records x y z nx ny nz, normals scaled by far_ns
+  float* geo32 = nullptr;   // the same padded to 8 floats
   double* trg64[3] = {};
   float* trg32[3] = {};
   double* wnear64 = nullptr;  // complex128 (Laplace weights with zero imaginary part)
   float* wnear32 = nullptr;   // complex64 copy for the mixed-precision path
   // workspace
   int ws_cap = 0;
-  double *q64 = nullptr, *m64 = nullptr, *sig64c = nullptr, *pot64c = nullptr, *part64 = nullptr;
-  float *q32 = nullptr, *m32 = nullptr, *part32 = nullptr;
+  double *str64 = nullptr, *sig64c = nullptr, *pot64c = nullptr, *part64 = nullptr;
+  float *str32 = nullptr, *part32 = nullptr;
   // far-sum launch shape: target workgroups x source splits >= far_wg_target (many short
   // workgroups, ~128 per CU, balance the 256 CUs better than one long round; the partial
   // sums of the splits are added by one coalesced pass)

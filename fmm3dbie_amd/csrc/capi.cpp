@@ -690,7 +690,7 @@ void* fmm3dbie_apply_plan_create(int helm, int64_t npatches, const int64_t* nord
 }
 
 // prec 64 (complex128) or 32 (complex64); mode 0 add/subtract, 1 masked (prec 32 is
-// always masked); times (optional, 4 doubles): oversample, far, csr, subtract ms.
+// always masked); times (optional, 4 doubles): oversample, far, csr + subtraction ms, 0.
 int fmm3dbie_apply_plan_apply(void* plan, int prec, int mode, const void* sigma, void* pot, int nrhs, void* stream,
                               double* times) {
   if (!plan) return -12;

@@ -105,6 +105,14 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
   return fma(0.5 * y, e, y);
 }
 
+// 1/sqrt(x) for x > 0: hardware estimate y refined by one third-order step, y + y e (1/2 +
+// 3/8 e) with e = 1 - x y^2 (relative error 5/16 e^3 before rounding).
+__device__ __forceinline__ double rsqrt_halley(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * y), y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
 // Kernel parameters: Helmholtz zk, alpha, beta (complex) or Laplace alpha, beta (real
 // parts used).  u = alpha*S + beta*D.
 struct KPar {

@@ -325,7 +325,8 @@ void *fmm3dbie_apply_plan_create(int helm, int64_t npatches, const int64_t *nord
                                  const double *whtsover, void *stream);
 /* prec 64: complex128 sigma/pot; prec 32: complex64 (near patches masked in the tiled
  * sum).  mode 0: add/subtract as the reference; 1: masked.  nrhs <= 64 columns of
- * length npts.  times (optional, 4 doubles): oversample, far, csr, subtract ms. */
+ * length npts.  times (optional, 4 doubles): oversample, far, csr and subtraction (one
+ * kernel) ms, 0. */
 int fmm3dbie_apply_plan_apply(void *plan, int prec, int mode, const void *sigma, void *pot, int nrhs,
                               void *stream, double *times);
 /* No reference counterpart: fmm3dbie_apply_plan_apply for callers that cannot allocate
@@ -344,8 +345,8 @@ size_t fmm3dbie_apply_scratch_bytes(void);
 int fmm3dbie_apply_plan_info(void *plan, int64_t *out4);
 void fmm3dbie_apply_plan_destroy(void *plan);
 /* Autotuner of the all-pairs far-sum launch (no reference counterpart): times every
- * right-hand-side group size dividing nrhs (FP64 1..8, FP32 1..16) and four workgroup
- * targets (4096..32768), keeps the fastest for later applies with the same (prec, nrhs); report gets
+ * right-hand-side group size dividing nrhs (1..16; FP64 blocks of a multiple of 16: 2..16)
+ * and four workgroup targets (4096..32768), keeps the fastest for later applies with the same (prec, nrhs); report gets
  * (group, workgroup target, ms) triples (nreport doubles).  Returns the number timed. */
 int fmm3dbie_apply_plan_tune(void *plan, int prec, int nrhs, void *stream, double *report, int nreport);
 

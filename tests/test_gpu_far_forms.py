@@ -1,0 +1,80 @@
+"""GPU tests of the far sum's forms: every size of a block of right-hand sides (vector groups,
+padded groups, matrix cores), kernel (Laplace, real and complex wavenumber, no double or no
+single layer, alpha and beta of any size and phase), precision and near-correction mode,
+against one 64-bit sum in plain torch."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _sum64(g, P, helm, pars, sig):
+    """All oversampled sources except those of near patches (near weights zero), (nrhs, npts)
+    in 64 bits (the add/subtract form is the same sum), and the sums of |K| |s| over those
+    sources and over all sources, which bound the rounding of either form."""
+    import torch
+    from fmm3dbie_amd import basis
+    no = int(g["norders"][0])
+    p = len(basis.rv_nodes(no)[1])
+    um = basis.rv_umat(no)
+    nrhs = len(sig)
+    over = np.zeros((nrhs, len(P["whtsover"])), complex)
+    for ip, nv in enumerate(P["novers"]):
+        uv, _ = basis.rv_nodes(int(nv))
+        im = np.stack([basis.koorn_pols(u, v, no) for u, v in uv]) @ um
+        a, b = P["ixyzso"][ip] - 1, P["ixyzso"][ip + 1] - 1
+        over[:, a:b] = sig[:, ip * p:(ip + 1) * p] @ im.T
+    over *= P["whtsover"]
+    t = torch.as_tensor
+    d = t(g["srcvals"][:, None, :3] - P["srcover"][None, :, :3])
+    r = d.square().sum(-1).sqrt()
+    ri = torch.where(r > 1e-14, 1 / r, torch.zeros_like(r))
+    dn = (d * t(P["srcover"][None, :, 9:12])).sum(-1) * ri * ri
+    zk, a, b = (pars if helm else (0.0, pars[0], pars[1]))
+    zk = complex(zk)
+    ker = (a + b * dn * (1 - 1j * zk * r)) * torch.exp(1j * zk * r) * ri / (4 * np.pi)
+    patch = np.repeat(np.arange(len(P["novers"])), np.diff(P["ixyzso"]))
+    near = np.zeros((len(r), len(P["novers"])), bool)
+    rows = np.repeat(np.arange(len(r)), np.diff(P["row_ptr"]))
+    near[rows, P["col_ind"] - 1] = True
+    far = torch.where(t(near[:, patch]), 0, ker)
+    size = [(t(over).abs() @ k.abs().T).numpy() for k in (far, ker)]
+    return (t(over) @ far.T).numpy(), size[0], size[1]
+
+
+# helm, (k, alpha, beta); the sphere's points are ragged: 27 targets of the last wavefront at
+# order 3 (12 patches of 10 points), 52 at order 4
+CASES = [(False, (0.7, -1.3), 3), (False, (1.0, 0.0), 4), (False, (0.0, 2.0), 3),
+         (True, (5.0, 5.0j, 1.0), 4), (True, (2.0, 0.0, 1.0), 3), (True, (3.0, 1.0 - 2.0j, 0.0), 4),
+         (True, (1.5, 3e4 + 1e3j, -2e-3 + 1e-3j), 3), (True, (0.0, 1.0 + 0.5j, 1.0j), 3),
+         (True, (2.0 + 0.7j, 1.0, 1.0), 4), (True, (-4.0, 1.0, 1.0), 3)]
+
+
+@pytest.mark.parametrize("helm,pars,norder", CASES)
+def test_far_sum_forms_match_a_64_bit_sum(cuda, helm, pars, norder):
+    import torch
+    from fmm3dbie_amd import geometry as G, layer, problem
+    g = G.get_sphere_npat(1.0, 2 if norder == 3 else 1, (0, 0, 0), norder)
+    pars = np.array(pars)
+    P = problem.setup(g, 1e-6, helm, pars)
+    w = np.zeros(P["nquad"], complex if helm else float)
+    plan = layer.ApplyPlan(g, helm, pars, P["row_ptr"], P["col_ind"], P["iquad"], w, P["novers"], P["ixyzso"],
+                           P["srcover"], P["whtsover"])
+    rng = np.random.default_rng(3)
+    N = len(g["srcvals"])
+    S = rng.standard_normal((33, N)) + 1j * rng.standard_normal((33, N))
+    ref, size_far, size_all = _sum64(g, P, helm, pars, S)
+    # A kernel value has a relative error of a few roundings (1/r three, its powers, the dipole
+    # factor, the phase k r <= 10), a sum of n terms up to sqrt(n) more (n <= 500 here): 30
+    # roundings of the sum of |K| |s|, over all sources where the near part is added and
+    # subtracted again
+    for nrhs in (1, 2, 3, 4, 5, 7, 8, 9, 16, 17, 33):
+        s = torch.as_tensor(S[:nrhs], device=cuda)
+        s = s[0] if nrhs == 1 else s
+        for prec, mode, unit, size in ((64, 1, 2.0 ** -53, size_far), (64, 0, 2.0 ** -53, size_all),
+                                       (32, 1, 2.0 ** -24, size_far)):
+            sp = s if prec == 64 else s.to(torch.complex64)
+            out = np.atleast_2d(plan.apply(sp.contiguous(), prec, mode).cpu().numpy())
+            err = np.linalg.norm(out - ref[:nrhs]) / np.linalg.norm(size[:nrhs])
+            assert err < 30 * unit, (nrhs, prec, mode, err / unit)
+    plan.close()
