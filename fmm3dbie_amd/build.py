@@ -45,9 +45,11 @@ def build(verbose=True):
     # the persistent quadrature kernels, which costs a wave per SIMD of occupancy; without
     # it they are rematerialised at their use (measured: adaptive, self and fixed-rule
     # kernels 14-24% faster, the far sum unchanged).
+    # Matrix products accumulate in VGPRs: in accumulation registers the compiler copied the
+    # accumulators out and in again around every step of a loop with branches (64 moves beside
+    # the 4 products of a step of the fixed-rule kernel).
     cmd = [HIPCC, "--offload-arch=" + ARCH, "-fgpu-rdc", "--hip-link", "-mllvm", "-disable-machine-licm",
-           "-shared", "-fPIC", "-o",
-           str(tmp)] + [str(o) for o in objs]
+           "-mllvm", "-amdgpu-mfma-vgpr-form", "-shared", "-fPIC", "-o", str(tmp)] + [str(o) for o in objs]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed: %s\n%s\n%s" % (" ".join(cmd), r.stdout, r.stderr))

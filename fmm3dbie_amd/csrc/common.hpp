@@ -91,26 +91,39 @@ __device__ __forceinline__ void koorn_eval(double u, double v, double* P) {
 
 
 // ---- FP64 elementary functions for the kernel evaluations ------------------------
-// sin/cos: sincos_red (trig.hpp), valid for |k r| <= 1.6e6, with no large-argument path:
-// the device library's sincos evaluates a large-argument reduction beside the small one
-// and selects, which made it most of a node evaluation's instructions.
-// 1/sqrt(x) for x > 0: hardware estimate refined by two Newton steps.
-__device__ __forceinline__ double rsqrt_nr(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  double t = x * y;
-  double e = fma(-t, y, 1.0);
-  y = fma(0.5 * y, e, y);
-  t = x * y;
-  e = fma(-t, y, 1.0);
-  return fma(0.5 * y, e, y);
-}
-
+// sin/cos: trig.hpp, valid for |k r| <= 1.6e6, with no large-argument path: the device
+// library's sincos evaluates a large-argument reduction beside the small one and selects,
+// which made it most of a node evaluation's instructions.
 // 1/sqrt(x) for x > 0: hardware estimate y refined by one third-order step, y + y e (1/2 +
-// 3/8 e) with e = 1 - x y^2 (relative error 5/16 e^3 before rounding).
+// 3/8 e) with e = 1 - x y^2 (relative error 5/16 e^3 before rounding).  The estimate's largest
+// relative error over 4e6 mantissas is 5.2e-8, the result's 1.9e-16, that of two Newton steps
+// (three instructions more).
 __device__ __forceinline__ double rsqrt_halley(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   const double e = fma(-(x * y), y, 1.0);
   return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+// sin x and cos x of the quadrature kernels, |x| <= SINCOS_RED_MAX: x = n pi + y (three-part
+// reduction as in sincos_red), then sincos_half_pi(y) and the sign of n's parity.  Near a
+// patch k r is small: where it is within pi/2 in every lane of the wavefront, n is zero and
+// the reduction and the signs are jumped over (20 instructions instead of 34 with
+// sincos_red); the bits of a lane's result do not depend on the other lanes.
+__device__ __forceinline__ void sincos_near(double x, double& s, double& c) {
+  const bool reduce = !__all(fabs(x) <= 1.5707963267948966);
+  double y = x, n = 0.0;
+  if (reduce) {
+    n = rint(x * 0x1.45f306dc9c883p-2);  // 1/pi
+    y = fma(-n, 0x1.921fb54442d18p+1, x);
+    y = fma(-n, 0x1.1a62633145c07p-53, y);
+    y = fma(-n, -0x1.f1976b7ed8fbcp-109, y);
+  }
+  sincos_half_pi(y, s, c);
+  if (reduce) {
+    const bool odd = (int)n & 1;
+    s = odd ? -s : s;
+    c = odd ? -c : c;
+  }
 }
 
 // Kernel parameters: Helmholtz zk, alpha, beta (complex) or Laplace alpha, beta (real
@@ -124,11 +137,11 @@ struct KPar {
 __device__ __forceinline__ void helm_comb(double dx, double dy, double dz, double nx, double ny,
                                           double nz, const KPar& kp, double& vr, double& vi) {
   const double r2 = dx * dx + dy * dy + dz * dz;
-  const double rinv = rsqrt_nr(r2);
+  const double rinv = rsqrt_halley(r2);
   const double r = r2 * rinv;
   const double d = dx * nx + dy * ny + dz * nz;
   double s, c;
-  sincos_red(kp.zkr * r, s, c);
+  sincos_near(kp.zkr * r, s, c);
   double er = c, ei = s;
   if (kp.zki != 0.0) {
     const double dec = exp(-kp.zki * r);
@@ -149,7 +162,7 @@ __device__ __forceinline__ void helm_comb(double dx, double dy, double dz, doubl
 __device__ __forceinline__ double lap_comb(double dx, double dy, double dz, double nx, double ny,
                                            double nz, const KPar& kp) {
   const double r2 = dx * dx + dy * dy + dz * dz;
-  const double rinv = rsqrt_nr(r2);
+  const double rinv = rsqrt_halley(r2);
   const double d = dx * nx + dy * ny + dz * nz;
   return (kp.br * d * rinv * rinv * rinv + kp.ar * rinv) * OVER4PI;
 }
@@ -178,10 +191,8 @@ __device__ __forceinline__ double geom_eval(const double* __restrict__ sc, const
 
 // Basis into an LDS staging row, then geometry from that row:
 //   row[l] = P_l(u,v) (koornf_pols ordering),  g[m] = sum_l sc[9l+m] * row[l].
-// With the coefficients in global memory (scalar loads) the geometry loop is kept rolled
-// so the 9*NP reads stay next to their use instead of being hoisted into registers; with
-// the coefficients staged in LDS (SC_LDS) it is unrolled by 3, which overlaps the reads
-// of three basis functions.
+// The coefficients are in global memory and come by scalar loads; the loop over l is unrolled
+// by UN, which decides how many loads are in flight (a rolled loop waits for each).
 template <int N>
 __device__ __forceinline__ void koorn_row(double u, double v, double* row) {
   const double z = 2.0 * u + v - 1.0, y = 1.0 - v, x = 1.0 - 2.0 * v;
@@ -211,71 +222,24 @@ __device__ __forceinline__ void koorn_row(double u, double v, double* row) {
   }
 }
 
-template <int NP, bool SC_LDS>
+template <int NP, int UN>
 __device__ __forceinline__ void geom_from_row(const double* __restrict__ sc, const double* __restrict__ row,
                                               double* g) {
 #pragma unroll
   for (int m = 0; m < 9; m++) g[m] = 0.0;
-  if (SC_LDS) {
-#pragma unroll 3
-    for (int l = 0; l < NP; l++) {
-      const double p = row[l];
+#pragma unroll UN
+  for (int l = 0; l < NP; l++) {
+    const double p = row[l];
 #pragma unroll
-      for (int m = 0; m < 9; m++) g[m] = fma(sc[9 * l + m], p, g[m]);
-    }
-  } else {
-#pragma unroll 1
-    for (int l = 0; l < NP; l++) {
-      const double p = row[l];
-#pragma unroll
-      for (int m = 0; m < 9; m++) g[m] = fma(sc[9 * l + m], p, g[m]);
-    }
+    for (int m = 0; m < 9; m++) g[m] = fma(sc[9 * l + m], p, g[m]);
   }
 }
 
-// Basis into an LDS staging row and geometry from the same values as they are generated
-// (no read-back of the row): g[m] = sum_l sc[9l+m] P_l(u,v), summed in generation order.
-template <int N>
-__device__ __forceinline__ void koorn_geom_fused(double u, double v, const double* __restrict__ sc, double* g,
-                                                 double* row) {
-  const double z = 2.0 * u + v - 1.0, y = 1.0 - v, x = 1.0 - 2.0 * v;
-  const double y2 = y * y;
-#pragma unroll
-  for (int m = 0; m < 9; m++) g[m] = 0.0;
-  double lkm1 = 0.0, lk = 1.0;
-#pragma unroll
-  for (int k = 0; k <= N; k++) {
-    if (k == 1) { lkm1 = 1.0; lk = z; }
-    if (k >= 2) {
-      const double ln = kTab.la[k - 1] * z * lk + kTab.lb[k - 1] * lkm1 * y2;
-      lkm1 = lk;
-      lk = ln;
-    }
-    double jm1 = 0.0, j0 = 1.0;
-#pragma unroll
-    for (int m = 0; m <= N - k; m++) {
-      const int n = m + k;
-      const int idx = n * (n + 1) / 2 + k;
-      const double val = lk * j0 * kTab.rs[m][k];
-      row[idx] = val;
-#pragma unroll
-      for (int c = 0; c < 9; c++) g[c] = fma(sc[9 * idx + c], val, g[c]);
-      if (m + 1 <= N - k) {
-        double jn;
-        if (m == 0) jn = kTab.ja[k][1] * x + kTab.jb[k][1];
-        else jn = (kTab.ja[k][m + 1] * x + kTab.jb[k][m + 1]) * j0 + kTab.jc[k][m + 1] * jm1;
-        jm1 = j0;
-        j0 = jn;
-      }
-    }
-  }
-}
-
-template <int N, bool SC_LDS = false>
+template <int N, int UN = 1>
 __device__ __forceinline__ void koorn_geom_row(double u, double v, const double* __restrict__ sc, double* g,
                                                double* row) {
   koorn_row<N>(u, v, row);
-  geom_from_row<(N + 1) * (N + 2) / 2, SC_LDS>(sc, row, g);
+  geom_from_row<(N + 1) * (N + 2) / 2, UN>(sc, row, g);
 }
 
 // normal and area element from g[3..8]; returns |x_u x x_v|, writes unit normal to g[9..11]

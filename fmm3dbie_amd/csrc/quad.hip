@@ -13,18 +13,23 @@
 //                       + umat^T, ggq-quads.f:412).
 //   4. k_tree_cache_mfma : node geometry of the refinement tree's depths 0..3 or 0..4
 //                       per patch, 16 patches at a time on FP64 MFMA.
-//   5. k_adaptive     : persistent wavefronts pull (target, patch) pairs from a queue
-//                       and run the 1->4 refinement of triaadap_main
-//                       (triaintrouts.f:1269-1464) depth-first with a per-wave stack in
-//                       HBM; the nodes of a step's four children are evaluated up
-//                       to 64 at a time (55 at order 6 and above, where a rule of 28
-//                       to 55 nodes takes one chunk per child).  With learned order selection each pair runs
-//                       the XG rule of its predicted class.
+//   5. the 1->4 refinement of triaadap_main (triaintrouts.f:1269-1464) for every adaptive pair:
+//      k_adap_tile    : its first three levels, a triangle and 16 of its targets at a time,
+//                       moments on FP64 MFMA;
+//      k_adaptive     : persistent wavefronts pull the triangles refined there from a queue and
+//                       walk each one's subtree depth-first with a per-wave stack in HBM; the
+//                       nodes of a step's four children are evaluated up to 64 at a time (55 at
+//                       order 6 and above, where a rule of 28 to 55 nodes takes one chunk per
+//                       child);
+//      k_adap_comb,   : sums over the refined triangles, and the weights.
+//      k_adap_final
+//                       With learned order selection each pair runs the XG rule of its
+//                       predicted class (two batched levels for the others than the plain rule).
 //   6. k_self         : one wavefront per on-surface target; a polar/sinh product rule
 //                       on the three triangles meeting at the target replaces the GGQ
 //                       rule of zget_ggq_self_quad_pt (ggq-quads.f:933-1122).
-// Moments are formed by staging kernel values f_q and basis rows P_j(q) in LDS and
-// letting lane j sum column j, then weights = umat^T * moments.
+// Elsewhere moments are formed by staging kernel values f_q and basis rows P_j(q) in LDS and
+// letting lane j sum column j; weights = umat^T * moments.
 #include <hip/hip_runtime.h>
 
 #include <array>
@@ -50,6 +55,9 @@ namespace {
 constexpr int WAVE = 64;
 constexpr int STACK_CAP = 72;
 constexpr int NLMAX = 20;
+// ints between the counters of the 8 work-queue segments: a cache line each (in one line their
+// updates serialise: 41000 of them took 0.4 ms, half of a small generation)
+constexpr int QUEUE_STRIDE = 64;
 // The second stream is used on surfaces of up to SIDE_MAX_PATCHES patches: measured 7-8%
 // faster on cube spheres of 768-1728 patches of orders 4-6, equal on a 1536-patch order-6
 // torus, and 6-8% slower on a 12288-patch order-6 surface, where the adaptive kernel alone
@@ -380,7 +388,7 @@ __global__ void __launch_bounds__(256) k_fixed_mfma(int nf, const double* __rest
 #pragma unroll
       for (int ct = 0; ct < CT; ct++) {
         const int j = ia + 16 * ct;
-        const double bb = j < NP ? Bq[q * NP + j] : 0.0;
+        const double bb = Bq[q * NP + j];  // columns past NP: not used (the table is padded)
         acc[0][ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(fr, bb, acc[0][ct], 0, 0, 0);
         if (HELM) acc[NPART - 1][ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(fi, bb, acc[NPART - 1][ct], 0, 0, 0);
       }
@@ -600,16 +608,15 @@ void launch_tree_cache(int64_t npat, int ncn, const double* twq, const double* p
 
 // Rules of the adaptive integrator, one per class: the XG rule (kq nodes), the node
 // geometry of the cached tree for that rule (per patch) and its basis table, and the
-// deepest level a pair of the class may reach.  The work list is sorted by class;
-// seg[c] .. seg[c + 1] - 1 are the pairs of class c.  A plain generation has one class:
-// the reference's rule and level cap (NLMAX).
+// deepest level a pair of the class may reach.  A plain generation has one class: the
+// reference's rule and level cap (NLMAX).
 constexpr int MAX_RULES = 6;
 struct AdapRules {
-  int nrules;
+  int nrules, ndeep;     // rules; the first ndeep have three batched levels
+  int64_t b0[MAX_RULES]; // rule c's pairs of patch ip: bucket b0[c] + ip of the sorted list
   int kq[MAX_RULES];
   int lmax[MAX_RULES];
-  int npar[MAX_RULES];  // cached triangles whose children are cached too (1, 5 or 21)
-  int seg[MAX_RULES + 1];
+  int npar[MAX_RULES];  // cached triangles whose children are cached too (1, 5, 21 or 85)
   const double* xg[MAX_RULES];
   const double* cache[MAX_RULES];
   const double* ptab[MAX_RULES];
@@ -643,9 +650,8 @@ __device__ __forceinline__ Mom column_sum_rows(const double* pb, int r0, int r1)
   return lane < NP ? Mom{sr, HELM ? si : 0.0} : Mom{0.0, 0.0};
 }
 
-// Moments of the triangles of one refinement step (root: the patch triangle, m[0];
-// otherwise the four children of the triangle (x0, y0, dx, dy) at tree id tid, m[0..3]):
-// their ntri * kq nodes are spread over the lanes in chunks of at most chunk_rows(N)
+// Moments of the triangles of one refinement step (the four children of the triangle (x0,
+// y0, dx, dy) at tree id tid, m[0..3]): their 4 kq nodes are spread over the lanes in chunks of at most chunk_rows(N)
 // nodes, of equal size, so a small rule still fills the wavefront and the kernel
 // evaluations of all children are in flight together.  Children of a cached triangle
 // have consecutive tree ids, so a chunk's rows are one contiguous block of the basis
@@ -657,18 +663,16 @@ __device__ __forceinline__ Mom column_sum_rows(const double* pb, int r0, int r1)
 // coefficients sc in LDS.  CACHED selects the path at compile time (the caller tests the
 // step's tree id), so each path is scheduled without the other's registers.
 template <int N, bool HELM, bool CACHED>
-__device__ __forceinline__ void step_moments(double* pb, const double* sc, bool root, int tid, double x0, double y0, double dx, double dy, int kq,
+__device__ __forceinline__ void step_moments(double* pb, const double* sc, int tid, double x0, double y0, double dx, double dy, int kq,
                                              const double* __restrict__ xg, const double* __restrict__ cpatch,
                                              const double* __restrict__ ptab, const double* tg, const KPar& kp,
                                              Mom (&m)[4]) {
   constexpr int NP = (N + 1) * (N + 2) / 2;
   constexpr int PW = ptab_w(NP);
   const int lane = threadIdx.x;
-  const int ntri = root ? 1 : 4;
-  const int total = ntri * kq;
-  // cached: the root itself, or children of a cached triangle of depth <= 2
-  constexpr bool cached = CACHED;
-  const int t0 = root ? 0 : cached_child(tid, 0);  // first cached tree id of the step
+  const int total = 4 * kq;
+  constexpr bool cached = CACHED;  // children of a triangle whose children are cached
+  const int t0 = cached_child(tid, 0);  // first cached tree id of the step
   const double hx = 0.5 * dx, hy = 0.5 * dy, da = hx * hx;
 #pragma unroll
   for (int c = 0; c < 4; c++) m[c] = Mom{0.0, 0.0};
@@ -690,7 +694,7 @@ __device__ __forceinline__ void step_moments(double* pb, const double* sc, bool 
     }
     double2 fv = make_double2(0.0, 0.0);
     if (lane < nrows) {
-      const int c = ntri == 1 ? 0 : (n >= kq) + (n >= 2 * kq) + (n >= 3 * kq);
+      const int c = (n >= kq) + (n >= 2 * kq) + (n >= 3 * kq);
       const int q = n - c * kq;
       double g[12], w;
       if (cached) {
@@ -720,7 +724,7 @@ __device__ __forceinline__ void step_moments(double* pb, const double* sc, bool 
     if (lane < nrows) *reinterpret_cast<double2*>(pb + lane * PW) = fv;
     __syncthreads();
     // the rows of this chunk belong to triangles c0..c1 (wave-uniform)
-    const int c0 = ntri == 1 ? 0 : base / kq, c1 = ntri == 1 ? 0 : (base + nrows - 1) / kq;
+    const int c0 = base / kq, c1 = (base + nrows - 1) / kq;
 #pragma unroll
     for (int c = 0; c < 4; c++) {
       if (c < c0 || c > c1) continue;
@@ -775,19 +779,18 @@ __device__ __forceinline__ Mom column_sum_tri(const double* pb, int nr) {
 // step_moments, with the same chunks but per-lane child indices and per-lane row bounds in
 // the column sums, and 71.0 ms here).
 template <int N, bool HELM, bool CACHED>
-__device__ __forceinline__ void step_tris(double* pb, const double* sc, bool root, int tid, double x0, double y0,
+__device__ __forceinline__ void step_tris(double* pb, const double* sc, int tid, double x0, double y0,
                                           double dx, double dy, int kq, const double* __restrict__ xg,
                                           const double* __restrict__ cpatch, const double* __restrict__ ptab,
                                           const double* tg, const KPar& kp, Mom (&m)[4]) {
   constexpr int NP = (N + 1) * (N + 2) / 2;
   constexpr int PW = ptab_w(NP);
   const int lane = threadIdx.x;
-  const int ntri = root ? 1 : 4;
-  const int t0 = root ? 0 : cached_child(tid, 0);
+  const int t0 = cached_child(tid, 0);
   const double hx = 0.5 * dx, hy = 0.5 * dy, da = hx * hx;
 #pragma unroll
   for (int c = 0; c < 4; c++) m[c] = Mom{0.0, 0.0};
-  for (int c = 0; c < ntri; c++) {
+  for (int c = 0; c < 4; c++) {
     if (CACHED) {
       const double* blk = ptab + ((size_t)(t0 + c) * kq) * PW;
 #pragma unroll
@@ -827,42 +830,91 @@ __device__ __forceinline__ void step_tris(double* pb, const double* sc, bool roo
   }
 }
 
-// Adaptive integration (triaadap_main, triaintrouts.f:1269-1464): persistent wavefronts
-// pull (target, patch) pairs from a queue; each pair's refinement tree is walked depth
-// first from a per-wavefront stack (the leaf set is that of the reference's level-by-level
-// walk: every decision depends only on its own triangle).  A step evaluates the four
-// children of the popped triangle (step_tris: one chunk per child; step_moments: the
-// children's nodes in equal chunks) and refines iff max_j |sum_c M_c,j - M_j| >
-// epsp (triaintrouts.f:1435-1448); the children are pushed only when refined.  A pair of
-// a routed class whose tree needs leaves below the class's level cap (lmax < NLMAX) is
-// appended to fb_out
-// (the plain integrator takes it afterwards) and gets no weights here.  The list is read
-// from nlist or, when nlist_dev is set, from the device count (a second launch over the
-// pairs a first one sent back).
+// ------------------------------------------------------------------ 4c. batched levels
+// The first three levels of the adaptive integration (two for the rule classes of learned order
+// selection other than the plain one, whose tree caches end there), for all targets of a
+// patch at once.  Levels 0 and 1 test the same few triangles for most of a
+// patch's targets and level 2 the same 16 for many of them (the average set of targets that
+// test a triangle: 150 / 139 / 19 on the deformed sphere of order 6, 80 / 42 / 6 on the
+// sphere of order 4, and 3 or fewer from level 3 on), and these levels hold 75 to 90% of all
+// refinement tests.  A workgroup takes a triangle and 16 of the targets that test it; each of
+// its four wavefronts integrates one child triangle for the 16 targets as k_fixed_mfma does
+// (in a step of 4 nodes lane l evaluates the kernel for target l % 16 at node l / 16, and the
+// 16x16x4 products of the matrix cores sum the moments against the basis rows of the cached
+// tree's table), so that a node's geometry and basis values are read once for 16 targets
+// instead of copied to LDS for each of them.  The four children's moments meet in LDS, where
+// the refinement test is made.
+//
+// Measured against a wavefront per pair that walks the whole tree: near quadrature of the
+// deformed sphere with 344k points, order 6, 93.1 to 70.9 ms (levels 0 to 2 take 3.8, 9.8 and 7.2
+// ms, the subtrees below them 28); torus of 43k points 12.6 to 9.0; sphere of 26k points, order 4,
+// 3.54 to 2.71; Laplace, 2k points, 0.81 to 0.47.
+//
+// Tree bookkeeping: a refined triangle of a pair gets a slot, the moments of its four
+// children.  When a child's own test ends, its place in the slot takes the child's final
+// moments: the sum of its children at a leaf, or, for a refined child, the sum of its own slot
+// once that is final (k_adap_comb, after the deeper levels).  So every sum has a fixed order.
+// Slots come from a pool; a pair that finds it empty is integrated again by the plain
+// integrator from its root (cap below).
+struct AdapTiles {
+  // pairs (CSR index, target) by (rule class, patch): bucket b at boff[b] .. boff[b + 1] - 1.  The
+  // counters and lists below are per (rule, patch) of the pass (bk = rule npat + patch), whose pairs
+  // are those of bucket b0[rule] + patch
+  const int2* sorted;
+  const int* boff;
+  int npat;
+  const double *epsp, *umat;
+  double* slots;  // slot s: 4 moment vectors from s * 4
+  int cap;
+  int *nslot, *nitem, *nfb, *npast;  // slots handed out, items, pairs sent back (all, past the cap)
+  int* cnt1;                 // per bucket: pairs refined at the root
+  int2* list1;               // (place in sorted, slot) of them, bucket b from boff[b]
+  int* cnt2;                 // per bucket and root child q: pairs refined there
+  int4* list2;               // (place, slot, moment vector to fill), from 4 boff[b] + q n_b
+  int4* items;               // (place, slot, moment vector to fill, tree id + 65536 rule): refined
+                             // triangles of the last batched level
+  int* flag;                 // per place: sent back (null: no pair can be)
+  int2* fb;                  // pairs sent back
+  int *nref, *lev;           // optional statistics per CSR entry
+};
+
+// past: the pair's tree is deeper than its class's level cap (else: no slot left)
+__device__ __forceinline__ void adap_send_back(const AdapTiles& A, int e, bool past) {
+  if (atomicExch(A.flag + e, 1) != 0) return;
+  A.fb[atomicAdd(A.nfb, 1)] = A.sorted[e];
+  if (past) atomicAdd(A.npast, 1);
+}
+
+// Adaptive integration (triaadap_main, triaintrouts.f:1269-1464) below the batched levels:
+// persistent wavefronts pull items from a queue (a triangle that was refined, whose four
+// children are the first triangles to be tested) and walk each one's subtree depth first
+// from a per-wavefront stack (the leaf set is that of the reference's level-by-level walk:
+// every decision depends only on its own triangle).  A step evaluates the four children of
+// the popped triangle (step_tris: one chunk per child; step_moments: the children's nodes in
+// equal chunks) and refines iff max_j |sum_c M_c,j - M_j| > epsp (triaintrouts.f:1435-1448);
+// the children are pushed only when refined.  The subtree's moments go to the item's place in
+// its parent's slot.  A pair of a routed class whose tree needs leaves below the class's
+// level cap (lmax < NLMAX) is sent back.
 template <int N, bool HELM>
-__global__ void __launch_bounds__(64) k_adaptive(int nlist, const int* __restrict__ nlist_dev,
-                                                 const int2* __restrict__ list, AdapRules R,
-                                                 int2* __restrict__ fb_out, int* __restrict__ fb_cnt,
-                                                 int* __restrict__ qctr, const int64_t* __restrict__ col_ind,
+__global__ void __launch_bounds__(64) k_adaptive(AdapTiles A, AdapRules R, int* __restrict__ qctr,
+                                                 const int64_t* __restrict__ col_ind,
                                                  const int64_t* __restrict__ ixyzs,
                                                  const double* __restrict__ srccoefs, int64_t ndtarg,
                                                  const double* __restrict__ targs,
-                                                 const int64_t* __restrict__ iquad,
-                                                 const double* __restrict__ epsp_patch,
-                                                 const double* __restrict__ umat, KPar kp,
-                                                 double* __restrict__ stack_all, int* __restrict__ nref_out,
-                                                 int* __restrict__ lev_out, int* __restrict__ unc_out,
-                                                 int* __restrict__ overflow, double* __restrict__ wnear) {
+                                                 const double* __restrict__ epsp_patch, KPar kp,
+                                                 double* __restrict__ stack_all, int* __restrict__ unc_out,
+                                                 int* __restrict__ overflow) {
   constexpr int NP = (N + 1) * (N + 2) / 2;
+  constexpr int NC = HELM ? 2 : 1, VL = NP * NC;  // moment vector of a slot
   constexpr int ES = 6 + 2 * NP;  // stack entry: x0,y0,dx,dy,level,tree id, moments
   __shared__ __align__(16) double pb[chunk_blocks(N) * 128];
   const int lane = threadIdx.x;
   double* stack = stack_all + (size_t)blockIdx.x * STACK_CAP * ES;
-  const int nl = nlist_dev ? *nlist_dev : nlist;
-  // Work queue: the list (sorted by class, then patch) in 8 contiguous segments, one per
-  // XCD (workgroups are dispatched to the XCDs round-robin, so workgroup b starts on
-  // segment b % 8 and the patch geometry it reads stays in its XCD's L2), then the other
-  // segments once its own is drained.
+  const int nl = *A.nitem < A.cap ? *A.nitem : A.cap;
+  // Work queue: the items (nearly sorted by class and patch, as the batched levels run) in 8
+  // contiguous segments, one per XCD (workgroups are dispatched to the XCDs round-robin, so
+  // workgroup b starts on segment b % 8 and the patch geometry it reads stays in its XCD's
+  // L2), then the other segments once its own is drained.
   const int home = blockIdx.x & 7;
   int tried = 0;  // segments found empty (lane 0)
   for (;;) {
@@ -873,7 +925,11 @@ __global__ void __launch_bounds__(64) k_adaptive(int nlist, const int* __restric
       while (tried < 8) {
         const int sg = (home + tried) & 7;
         const int a = (int)((int64_t)nl * sg / 8), b = (int)((int64_t)nl * (sg + 1) / 8);
-        const int k = atomicAdd(qctr + sg, 1);
+        // (a drained segment is seen by a load: thousands of wavefronts leave through here, and
+        // their atomic updates of one address would queue up)
+        int* ctr = qctr + QUEUE_STRIDE * sg;
+        int k = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (a + k < b) k = atomicAdd(ctr, 1);
         if (a + k < b) {
           got = a + k;
           break;
@@ -883,13 +939,14 @@ __global__ void __launch_bounds__(64) k_adaptive(int nlist, const int* __restric
     }
     const int idx = __builtin_amdgcn_readfirstlane(got);
     if (idx < 0) break;
-    int cls = 0;
-    while (cls + 1 < R.nrules && idx >= R.seg[cls + 1]) cls++;
-    cls = __builtin_amdgcn_readfirstlane(cls);
+    const int4 item = A.items[idx];
+    if (item.y < 0) continue;  // a pair sent back
+    const int cls = __builtin_amdgcn_readfirstlane(item.w >> 16);
+    const int node = __builtin_amdgcn_readfirstlane(item.w & 0xffff);
     const int kq = R.kq[cls], lmax = R.lmax[cls];
     const double* xg = R.xg[cls];
     const double* ptab = R.ptab[cls];
-    const int2 jt = list[idx];
+    const int2 jt = A.sorted[item.x];
     const int64_t ip = col_ind[jt.x] - 1;
     // patch coefficients for the geometry below the cached tree, read with wave-uniform
     // (scalar) loads: in LDS they would cost the LDS of a wavefront per CU at order 6
@@ -902,10 +959,6 @@ __global__ void __launch_bounds__(64) k_adaptive(int nlist, const int* __restric
     Mom mc[4];
     // (at order 6 and above: at lower orders the second path costs a wavefront per SIMD)
     const bool per_tri = N >= 6 && kq <= chunk_rows(N) && 2 * kq > chunk_rows(N);
-    if (per_tri)
-      step_tris<N, HELM, true>(pb, lsc, true, 0, 0.0, 0.0, 1.0, 1.0, kq, xg, cpatch, ptab, tg, kp, mc);
-    else
-      step_moments<N, HELM, true>(pb, lsc, true, 0, 0.0, 0.0, 1.0, 1.0, kq, xg, cpatch, ptab, tg, kp, mc);
     // The triangle being tested is held in registers and the stack holds the others:
     // a refinement pushes children 0..2 and goes on with child 3 (the one the stack
     // order takes next).  At order 6 and above the entry on top of the stack is loaded at
@@ -914,10 +967,59 @@ __global__ void __launch_bounds__(64) k_adaptive(int nlist, const int* __restric
     constexpr bool PREFETCH = N >= 6;
     double cx0 = 0.0, cy0 = 0.0, cdx = 1.0, cdy = 1.0;
     int clevel = 0, ctid = 0;
-    Mom cpar = lane < NP ? mc[0] : Mom{0.0, 0.0};
+    Mom cpar{0.0, 0.0};
     int sp = 0, nref = 0, deep = 0, nunc = 0;
     bool aborted = false, have = true;
     Mom result{0.0, 0.0};
+    {
+      // the children of tree id node (1 + c of depth 1, or 5 + 4 c1 + c of depth 2): 0..2 to the
+      // stack, 3 to be tested first
+      auto child = [&](int c) {
+        const double hx = 0.5 * cdx, hy = 0.5 * cdy;
+        cx0 = (c & 1) ? cx0 + hx : cx0;
+        cy0 = (c & 2) ? cy0 + hy : cy0;
+        cdx = c == 3 ? -hx : hx;
+        cdy = c == 3 ? -hy : hy;
+      };
+      if (node < 5) {
+        child(node - 1);
+      } else {
+        child((node - 5) >> 2);
+        child((node - 5) & 3);
+      }
+      clevel = node < 5 ? 2 : 3;
+      const double* sl = A.slots + (size_t)item.y * 4 * VL;
+      const double bx = cx0, by = cy0, bdx = cdx, bdy = cdy;
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        cx0 = bx;
+        cy0 = by;
+        cdx = bdx;
+        cdy = bdy;
+        child(c);
+        if (lane < NP) {
+          cpar.re = sl[c * VL + NC * lane];
+          cpar.im = HELM ? sl[c * VL + NC * lane + NC - 1] : 0.0;
+        }
+        if (c == 3) break;
+        double* ne = stack + (size_t)c * ES;
+        if (lane == 0) {
+          ne[0] = cx0;
+          ne[1] = cy0;
+          ne[2] = cdx;
+          ne[3] = cdy;
+          ne[4] = (double)clevel;
+          ne[5] = (double)cached_child(node, c);
+        }
+        if (lane < NP) {
+          ne[6 + lane] = cpar.re;
+          ne[6 + NP + lane] = cpar.im;
+        }
+      }
+      sp = 3;
+      ctid = cached_child(node, 3);
+      __syncthreads();
+    }
     while (have) {
       double nx0 = 0.0, ny0 = 0.0, ndx = 0.0, ndy = 0.0, nlev = 0.0, ntid = 0.0;
       Mom tpar{0.0, 0.0};
@@ -936,13 +1038,13 @@ __global__ void __launch_bounds__(64) k_adaptive(int nlist, const int* __restric
       const Mom mpar = cpar;
       if (per_tri) {
         if (tid >= 0 && tid < npar)
-          step_tris<N, HELM, true>(pb, lsc, false, tid, x0, y0, dx, dy, kq, xg, cpatch, ptab, tg, kp, mc);
+          step_tris<N, HELM, true>(pb, lsc, tid, x0, y0, dx, dy, kq, xg, cpatch, ptab, tg, kp, mc);
         else
-          step_tris<N, HELM, false>(pb, lsc, false, tid, x0, y0, dx, dy, kq, xg, cpatch, ptab, tg, kp, mc);
+          step_tris<N, HELM, false>(pb, lsc, tid, x0, y0, dx, dy, kq, xg, cpatch, ptab, tg, kp, mc);
       } else if (tid >= 0 && tid < npar) {
-        step_moments<N, HELM, true>(pb, lsc, false, tid, x0, y0, dx, dy, kq, xg, cpatch, ptab, tg, kp, mc);
+        step_moments<N, HELM, true>(pb, lsc, tid, x0, y0, dx, dy, kq, xg, cpatch, ptab, tg, kp, mc);
       } else {
-        step_moments<N, HELM, false>(pb, lsc, false, tid, x0, y0, dx, dy, kq, xg, cpatch, ptab, tg, kp, mc);
+        step_moments<N, HELM, false>(pb, lsc, tid, x0, y0, dx, dy, kq, xg, cpatch, ptab, tg, kp, mc);
       }
       nref++;
       nunc += (tid < 0 || tid >= npar) ? 1 : 0;  // children below the cached tree
@@ -1019,15 +1121,270 @@ __global__ void __launch_bounds__(64) k_adaptive(int nlist, const int* __restric
     }
     __syncthreads();
     if (aborted) {
-      if (lane == 0 && fb_out) fb_out[atomicAdd(fb_cnt, 1)] = jt;
+      if (lane == 0) adap_send_back(A, item.x, true);
       continue;
     }
     if (lane == 0) {
-      if (nref_out) nref_out[jt.x] = nref;
-      if (lev_out) lev_out[jt.x] = deep;
-      if (unc_out) unc_out[jt.x] = nunc;
+      if (A.nref) atomicAdd(A.nref + jt.x, nref);
+      if (A.lev) atomicMax(A.lev + jt.x, deep);
+      if (unc_out) atomicAdd(unc_out + jt.x, nunc);
     }
-    store_weights<NP, HELM>(pb, result, umat, wnear, iquad[jt.x] - 1);
+    if (lane < NP) {
+      A.slots[(size_t)item.z * VL + NC * lane] = result.re;
+      if (HELM) A.slots[(size_t)item.z * VL + NC * lane + NC - 1] = result.im;
+    }
+  }
+}
+
+// Weights of up to 16 pairs: moments (interleaved re, im) of pair tt in mom[tt * VL], 16
+// threads per pair (sub).
+template <int NP, bool HELM>
+__device__ __forceinline__ void tile_weights(const double* mom, int tt, int sub, const double* __restrict__ umat,
+                                             double* __restrict__ wnear, int64_t q0) {
+  constexpr int NC = HELM ? 2 : 1, VL = NP * NC;
+  const double* m = mom + tt * VL;
+  for (int i = sub; i < NP; i += 16) {
+    double sr = 0.0, si = 0.0;
+#pragma unroll 4
+    for (int l = 0; l < NP; l++) {
+      const double u = umat[l + i * NP];
+      sr = fma(u, m[NC * l], sr);
+      if (HELM) si = fma(u, m[NC * l + 1], si);
+    }
+    if (HELM) *reinterpret_cast<double2*>(wnear + 2 * (q0 + i)) = make_double2(sr, si);
+    else wnear[q0 + i] = sr;
+  }
+}
+
+// Level LEV of the pairs of (rule, patch) blockIdx.x.  LEV 0: the root triangle of every pair (its own
+// moments are integrated first, the four wavefronts sharing its nodes).  LEV 1: root child
+// blockIdx.y of the pairs refined at the root.  LEV 2: child blockIdx.y % 4 of root child
+// blockIdx.y / 4 of the pairs refined there.  Sets longer than 16 are taken in tiles, blockIdx.z
+// apart.
+template <int N, bool HELM, int LEV>
+__global__ void __launch_bounds__(256) k_adap_tile(AdapTiles A, AdapRules R, int64_t ndtarg,
+                                                   const double* __restrict__ targs,
+                                                   const int64_t* __restrict__ iquad, KPar kp,
+                                                   double* __restrict__ wnear) {
+  constexpr int NP = (N + 1) * (N + 2) / 2, PW = ptab_w(NP);
+  constexpr int CT = (NP + 15) / 16, NC = HELM ? 2 : 1, VL = NP * NC;
+  __shared__ __align__(16) double lm[4 * 16 * VL];                 // children's moments: child, target
+  __shared__ __align__(16) double lp[LEV == 0 ? 16 * VL : 1];      // the root's; then final sums
+  __shared__ int refs[16], base[2];
+  const int bk = blockIdx.x, y = blockIdx.y;
+  const int cls = bk / A.npat, ip = bk - cls * A.npat;
+  const int64_t bs = R.b0[cls] + ip;
+  const int b0 = A.boff[bs], np = A.boff[bs + 1] - b0;
+  const int nset = LEV == 0 ? np : (LEV == 1 ? A.cnt1[bk] : A.cnt2[4 * bk + (y >> 2)]);
+  if (nset == 0) return;
+  const int t = LEV == 0 ? 0 : (LEV == 1 ? 1 + y : 5 + y);  // the tested triangle's tree id
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int ia = lane & 15, ka = lane >> 4;
+  const int tt = threadIdx.x >> 4, sub = threadIdx.x & 15;  // test stage: target, thread of 16
+  const int kq = R.kq[cls], lmax = R.lmax[cls];
+  const double* cp = R.cache[cls] + (size_t)ip * CACHE_STRIDE * cache_tris(R.npar[cls]) * kq;
+  const double* ptab = R.ptab[cls];
+  const double eps = A.epsp[ip];
+  // refined triangles of the last batched level go to the items
+  const bool last = LEV == 2 || (LEV == 1 && R.npar[cls] < 21);
+  // entry i of the set: place in sorted, and the vector of the parent's slot that holds the
+  // triangle's own moments (-1: a pair sent back)
+  auto entry = [&](int i, int& e, int& ref) {
+    e = b0 + i;
+    ref = 0;
+    if (LEV == 1) {
+      const int2 v = A.list1[b0 + i];
+      e = v.x;
+      ref = v.y < 0 ? -1 : 4 * v.y + y;
+    } else if (LEV == 2) {
+      const int4 v = A.list2[4 * (size_t)b0 + (size_t)(y >> 2) * np + i];
+      e = v.x;
+      ref = v.y < 0 ? -1 : 4 * v.y + (y & 3);
+    }
+  };
+  for (int k = 16 * blockIdx.z; k < nset; k += 16 * gridDim.z) {
+    int e, ref;
+    entry(k + ia < nset ? k + ia : k, e, ref);
+    const double* tp = targs + ndtarg * (int64_t)A.sorted[e].y;
+    const double tx = tp[0], ty = tp[1], tz = tp[2];
+    dbl4 acc[NC][CT];
+    // moments of cached triangle c over node steps q0 = first, first + stride, ...
+    auto integrate = [&](int c, int first, int stride) {
+#pragma unroll
+      for (int pa = 0; pa < NC; pa++)
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++) acc[pa][ct] = dbl4{0.0, 0.0, 0.0, 0.0};
+      const double* nb = cp + (size_t)CACHE_STRIDE * c * kq;
+      const double* pt = ptab + (size_t)c * kq * PW + 2 + ia;
+#pragma unroll 1
+      for (int q0 = first; q0 < kq; q0 += stride) {
+        const int q = q0 + ka;
+        // past the rule's last node: weight zero.  Rows of the table are read to the end of the
+        // column tiles: what they give past NP, or past the rule, is not used (the next rows,
+        // and the table's padding, are finite)
+        const double2* o = reinterpret_cast<const double2*>(nb + CACHE_STRIDE * (q < kq ? q : kq - 1));
+        const double2 o0 = o[0], o1 = o[1], o2 = o[2];
+        const double wq = q < kq ? o[3].x : 0.0;
+        double bb[CT];
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++) bb[ct] = pt[q * PW + 16 * ct];
+        double vr, vi;
+        if (HELM) {
+          helm_comb(tx - o0.x, ty - o0.y, tz - o1.x, o1.y, o2.x, o2.y, kp, vr, vi);
+        } else {
+          vr = lap_comb(tx - o0.x, ty - o0.y, tz - o1.x, o1.y, o2.x, o2.y, kp);
+          vi = 0.0;
+        }
+        vr *= wq;
+        vi *= wq;
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++) {
+          acc[0][ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(vr, bb[ct], acc[0][ct], 0, 0, 0);
+          if (HELM) acc[NC - 1][ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(vi, bb[ct], acc[NC - 1][ct], 0, 0, 0);
+        }
+      }
+      // accumulator element r: target ka + 4 r, basis function ia + 16 ct
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++) {
+          const int j = ia + 16 * ct;
+          if (j >= NP) continue;
+          double* o = lm + (w * 16 + ka + 4 * r) * VL + NC * j;
+          if (HELM) *reinterpret_cast<double2*>(o) = make_double2(acc[0][ct][r], acc[NC - 1][ct][r]);
+          else o[0] = acc[0][ct][r];
+        }
+    };
+    if (LEV == 0) {
+      integrate(0, 4 * w, 16);
+      __syncthreads();
+      for (int i = threadIdx.x; i < 16 * VL; i += 256)
+        lp[LEV == 0 ? i : 0] = (lm[i] + lm[16 * VL + i]) + (lm[32 * VL + i] + lm[48 * VL + i]);
+      __syncthreads();
+    }
+    integrate(cached_child(t, w), 0, 4);
+    __syncthreads();
+    // the refinement test of target tt
+    entry(k + tt < nset ? k + tt : k, e, ref);
+    const bool valid = k + tt < nset && (LEV == 0 || ref >= 0);
+    const double* par = LEV == 0 ? lp + tt * VL : A.slots + (size_t)(valid ? ref : 0) * VL;
+    auto ssum = [&](int i) {
+      const double* m = lm + tt * VL + i;
+      return ((m[0] + m[16 * VL]) + m[32 * VL]) + m[48 * VL];
+    };
+    double err = 0.0;
+    for (int j = sub; j < NP; j += 16) {
+      const double dr = ssum(NC * j) - par[NC * j];
+      double d = fabs(dr);
+      if (HELM) {
+        const double di = ssum(NC * j + 1) - par[NC * j + 1];
+        d = sqrt(dr * dr + di * di);
+      }
+      err = d > err ? d : err;
+    }
+#pragma unroll
+    for (int off = 8; off >= 1; off >>= 1) {
+      const double o = __shfl_xor(err, off, 64);
+      err = o > err ? o : err;
+    }
+    // refining would put leaves past the class's level cap: the prediction was wrong
+    const bool past = valid && err > eps && lmax < NLMAX && LEV + 2 > lmax;
+    if (past && sub == 0) adap_send_back(A, e, true);
+    const bool refine = valid && err > eps && !past;
+    if (sub == 0) refs[tt] = refine;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int n = 0;
+      for (int u = 0; u < 16; u++) n += refs[u];
+      base[0] = n ? atomicAdd(A.nslot, n) : 0;
+      base[1] = n ? atomicAdd(last ? A.nitem : (LEV == 0 ? A.cnt1 + bk : A.cnt2 + 4 * bk + y), n) : 0;
+    }
+    __syncthreads();
+    int pos = 0;
+    for (int u = 0; u < 16; u++) pos += u < tt ? refs[u] : 0;
+    if (refine) {
+      int slot = base[0] + pos;
+      if (slot >= A.cap) {
+        slot = -1;
+        if (sub == 0) adap_send_back(A, e, false);
+      } else {
+        double* o = A.slots + (size_t)slot * 4 * VL;
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+          for (int i = sub; i < VL; i += 16) o[c * VL + i] = lm[(c * 16 + tt) * VL + i];
+      }
+      if (sub == 0) {
+        const int at = base[1] + pos;
+        if (LEV == 0) A.list1[b0 + at] = make_int2(e, slot);
+        else if (!last) A.list2[4 * (size_t)b0 + (size_t)y * np + at] = make_int4(e, slot, ref, 0);
+        else if (at < A.cap) A.items[at] = make_int4(e, slot, ref, t + 65536 * cls);
+      }
+    } else if (valid && LEV > 0) {
+      for (int i = sub; i < VL; i += 16) A.slots[(size_t)ref * VL + i] = ssum(i);
+    }
+    if (valid && sub == 0) {
+      const int j = A.sorted[e].x;
+      if (A.nref) atomicAdd(A.nref + j, 1);
+      if (A.lev && !refine) atomicMax(A.lev + j, LEV + 1);
+    }
+    if (LEV == 0) {
+      // leaves at the root: their weights
+      const bool leaf = valid && !refine && !past;
+      if (leaf)
+        for (int i = sub; i < VL; i += 16) lp[LEV == 0 ? tt * VL + i : 0] = ssum(i);
+      __syncthreads();
+      if (leaf) tile_weights<NP, HELM>(lp, tt, sub, A.umat, wnear, iquad[A.sorted[e].x] - 1);
+    }
+    __syncthreads();
+  }
+}
+
+// Statistics of pairs that are integrated again start over.
+__global__ void k_adap_reset(const int* __restrict__ n, const int2* __restrict__ list, int* nref, int* lev, int* unc) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= *n) return;
+  const int j = list[i].x;
+  if (nref) nref[j] = 0;
+  if (lev) lev[j] = 0;
+  if (unc) unc[j] = 0;
+}
+
+// Final moments of the level-1 triangles refined at level 1: the sum of their slot.
+template <int NP, bool HELM>
+__global__ void __launch_bounds__(256) k_adap_comb(AdapTiles A, AdapRules R) {
+  constexpr int VL = NP * (HELM ? 2 : 1);
+  const int bk = blockIdx.x, q = blockIdx.y, n = A.cnt2[4 * bk + q];
+  if (n == 0) return;
+  const int64_t bs = R.b0[bk / A.npat] + bk % A.npat;
+  const int b0 = A.boff[bs], np = A.boff[bs + 1] - b0;
+  const int tt = threadIdx.x >> 4, sub = threadIdx.x & 15;
+  for (int i = tt; i < n; i += 16) {
+    const int4 v = A.list2[4 * (size_t)b0 + (size_t)q * np + i];
+    if (v.y < 0) continue;
+    const double* m = A.slots + (size_t)v.y * 4 * VL;
+    for (int l = sub; l < VL; l += 16)
+      A.slots[(size_t)v.z * VL + l] = ((m[l] + m[VL + l]) + m[2 * VL + l]) + m[3 * VL + l];
+  }
+}
+
+// Weights of the pairs refined at the root: umat^T times the sum of their root slot.
+template <int NP, bool HELM>
+__global__ void __launch_bounds__(256) k_adap_final(AdapTiles A, AdapRules R, const int64_t* __restrict__ iquad,
+                                                    double* __restrict__ wnear) {
+  constexpr int VL = NP * (HELM ? 2 : 1);
+  __shared__ __align__(16) double mom[16 * VL];
+  const int bk = blockIdx.x, b0 = A.boff[R.b0[bk / A.npat] + bk % A.npat], n = A.cnt1[bk];
+  const int tt = threadIdx.x >> 4, sub = threadIdx.x & 15;
+  for (int k = 16 * blockIdx.y; k < n; k += 16 * gridDim.y) {
+    const int i = k + tt;
+    const int2 v = i < n ? A.list1[b0 + i] : make_int2(0, -1);
+    const bool ok = v.y >= 0 && !(A.flag && A.flag[v.x]);
+    const double* m = A.slots + (size_t)(ok ? v.y : 0) * 4 * VL;
+    if (ok)
+      for (int l = sub; l < VL; l += 16) mom[tt * VL + l] = ((m[l] + m[VL + l]) + m[2 * VL + l]) + m[3 * VL + l];
+    __syncthreads();
+    if (ok) tile_weights<NP, HELM>(mom, tt, sub, A.umat, wnear, iquad[A.sorted[v.x].x] - 1);
+    __syncthreads();
   }
 }
 
@@ -1085,29 +1442,38 @@ __global__ void k_features(int nadap, const int2* __restrict__ list, const int64
     for (int k = 0; k < 8; k++) feat_full[8 * (int64_t)jt.x + k] = f[k];
 }
 
-// Bucket key of an adaptive pair (MLP_OUT * npatches keys): rule class, then patch.
-// Without a prediction every pair is in class 0 (the plain rule), sorted by patch.
-__device__ __forceinline__ int64_t bucket_key(int c, int64_t patch, int64_t npat) { return c * npat + patch; }
-
-__global__ void k_bucket_count(int n, const int2* __restrict__ list, const int* __restrict__ pred,
-                               const int64_t* __restrict__ col_ind, int64_t npat, int* __restrict__ cnt) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  atomicAdd(cnt + bucket_key(pred ? pred[i] : 0, col_ind[list[i].x] - 1, npat), 1);
+// Bucket key of an adaptive pair (MLP_OUT * npatches keys): place of its rule class (the 4 bits of
+// place from 4 c), then patch.  Without a prediction every pair is in class 0 (the plain rule),
+// sorted by patch.
+__device__ __forceinline__ int64_t bucket_key(int c, int place, int64_t patch, int64_t npat) {
+  return ((place >> (4 * c)) & 15) * npat + patch;
 }
 
-__global__ void k_bucket_scatter(int n, const int2* __restrict__ list, const int* __restrict__ pred,
-                                 const int64_t* __restrict__ col_ind, int64_t npat, const int* __restrict__ off,
-                                 int* __restrict__ fill, int2* __restrict__ out, int* __restrict__ pred_full) {
+// (list: n pairs, and *more after them)
+__global__ void k_bucket_count(int n, const int* __restrict__ more, const int2* __restrict__ list,
+                               const int* __restrict__ pred, int place, const int64_t* __restrict__ col_ind, int64_t npat,
+                               int* __restrict__ cnt) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  if (i >= n + (more ? *more : 0)) return;
+  atomicAdd(cnt + bucket_key(pred ? pred[i] : 0, place, col_ind[list[i].x] - 1, npat), 1);
+}
+
+__global__ void k_bucket_scatter(int n, const int* __restrict__ more, const int2* __restrict__ list,
+                                 const int* __restrict__ pred, int place, const int64_t* __restrict__ col_ind, int64_t npat,
+                                 const int* __restrict__ off, int* __restrict__ fill, int2* __restrict__ out, int* __restrict__ pred_full) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n + (more ? *more : 0)) return;
   const int2 jt = list[i];
-  const int64_t key = bucket_key(pred ? pred[i] : 0, col_ind[jt.x] - 1, npat);
+  const int64_t key = bucket_key(pred ? pred[i] : 0, place, col_ind[jt.x] - 1, npat);
   out[off[key] + atomicAdd(fill + key, 1)] = jt;
   if (pred_full) pred_full[jt.x] = pred[i];
 }
 
 // ------------------------------------------------------------------ 5. self
+// Rows of the basis recurrence unrolled in k_self's geometry: the chain of dependent multiply-adds of
+// a row leaves the FP64 pipe idle at the kernel's occupancy (the deformed sphere's 344k points:
+// rolled 14.9 ms, 4 rows 11.9 ms).
+constexpr int SELF_UN = 4;
 template <int N, bool HELM>
 __global__ void __launch_bounds__(64) k_self(int nself, const int2* __restrict__ list,
                                              const int64_t* __restrict__ col_ind,
@@ -1268,7 +1634,7 @@ __global__ void __launch_bounds__(64) k_self(int nself, const int2* __restrict__
       const double xi0 = rho * px, xi1 = rho * py;
       const double dv = xi1 / l22, du = (xi0 - l12 * dv) / l11;
       double g[12];
-      koorn_geom_row<N>(u0 + du, v0 + dv, sc, g, row + 2);
+      koorn_geom_row<N, SELF_UN>(u0 + du, v0 + dv, sc, g, row + 2);
       const double jac = geom_finish(g);
       const double w = g_self_gl.wr[ir] * wtau * rho * d * d * ch / detl * jac;
       double vr, vi;
@@ -1333,6 +1699,7 @@ T* dalloc(size_t n) {
 enum WsSlot {
   W_CMS, W_RADS, W_EPSP, W_AREA, W_CNT, W_OFF, W_FILL, W_CLS, W_COUNTS, W_ADAP, W_SELF, W_FIXED, W_NREF,
   W_CACHE, W_STACK, W_X, W_PRED, W_BCNT, W_BOFF, W_SORTED, W_FB, W_PFULL, W_QCTR, W_LEV, W_SEG, W_UNC,
+  W_SLOTS, W_ITEMS, W_LIST1, W_LIST2, W_TCNT, W_FLAG,
   W_RCACHE0,  // tree caches of the routed rule classes: W_RCACHE0 + class
   W_NSLOTS = W_RCACHE0 + MAX_RULES
 };
@@ -1497,7 +1864,8 @@ int build_tables(int nqorder, int nlev, int nqorder_f, OrderTables& T, hipStream
   std::vector<double> xq, xw, fuv, fw;
   const int kq = fmmhost::xg_rule(nqorder, xq, xw);
   const int nf = fmmhost::xg_unif_nodes(nlev, nqorder_f, fuv, fw);
-  std::vector<double> xg(3 * kq), Pq((size_t)nf * NP), Bq((size_t)nf * NP), pols(NP);
+  // (64 doubles of padding: k_fixed_mfma reads whole tiles of 16 columns)
+  std::vector<double> xg(3 * kq), Pq((size_t)nf * NP), Bq((size_t)nf * NP + 64, 0.0), pols(NP);
   for (int q = 0; q < kq; q++) { xg[3 * q] = xq[2 * q]; xg[3 * q + 1] = xq[2 * q + 1]; xg[3 * q + 2] = xw[q]; }
   for (int q = 0; q < nf; q++) {
     fmmhost::koorn_pols(fuv[2 * q], fuv[2 * q + 1], N, pols.data());
@@ -1587,13 +1955,48 @@ int adaptive_slots() {
   return n;
 }
 
+// Slot pool of the adaptive levels: every triangle of the batched levels for up to
+// SLOT_ALL_BYTES, beyond that SLOTS_PER_PAIR slots per pair (measured need: 1.7 on the
+// deformed sphere of order 6, 1.0 to 1.5 on the other surfaces), pairs that find it empty
+// being integrated in another pass.
+constexpr int SLOTS_ALL = 21;
+constexpr size_t SLOT_ALL_BYTES = (size_t)2 << 30;
+constexpr double SLOTS_PER_PAIR = 2.25;
+
+// One pass over n adaptive pairs (T.sorted by bucket; classes R): batched levels, subtrees below,
+// weights.  cap: slots of the pool; T.flag and T.fb where pairs can be sent back.
 template <int N, bool HELM>
-void launch_adaptive(int g, hipStream_t s, int nlist, const int* nlist_dev, const int2* list, const AdapRules& R,
-                     int2* fb_out, int* fb_cnt, int* qctr, const NearQuadArgs& A, const double* epsp,
-                     const double* umat, const KPar& kp, double* stack, int* nref, int* lev, int* unc, int* over) {
-  k_adaptive<N, HELM><<<g, 64, 0, s>>>(nlist, nlist_dev, list, R, fb_out, fb_cnt, qctr, A.col_ind, A.ixyzs,
-                                       A.srccoefs, A.ndtarg, A.targs, A.iquad, epsp, umat, kp, stack, nref, lev, unc,
-                                       over, A.wnear);
+int run_tiles(const NearQuadArgs& A, const AdapRules& R, AdapTiles T, int n, int nwaves, const KPar& kp, double* stack,
+              int* qctr, int* unc, int* over, hipStream_t s) {
+  constexpr int NP = (N + 1) * (N + 2) / 2;
+  const int64_t nb = A.npatches * R.nrules;
+  int* c = wsalloc<int>(W_TCNT, 16 + 5 * nb);
+  if (!c) return -2;
+  T.nslot = c;
+  T.nitem = c + 1;
+  T.cnt1 = c + 16;
+  T.cnt2 = c + 16 + nb;
+  HCHK(hipMemsetAsync(c, 0, sizeof(int) * (16 + 5 * nb), s));
+  HCHK(hipMemsetAsync(qctr, 0, sizeof(int) * 8 * QUEUE_STRIDE, s));
+  // tiles of a patch's pairs at levels 0 and 1: about one per workgroup, two on large surfaces
+  int64_t z = (n + 16 * nb - 1) / (16 * nb);
+  if (A.npatches > 2048) z = (z + 1) / 2;
+  z = z < 1 ? 1 : (z > 16 ? 16 : z);
+  const unsigned g = (unsigned)nb, gd = (unsigned)(A.npatches * R.ndeep), nz = (unsigned)z;
+  k_adap_tile<N, HELM, 0><<<dim3(g, 1, nz), 256, 0, s>>>(T, R, A.ndtarg, A.targs, A.iquad, kp, A.wnear);
+  k_adap_tile<N, HELM, 1><<<dim3(g, 4, nz), 256, 0, s>>>(T, R, A.ndtarg, A.targs, A.iquad, kp, A.wnear);
+  if (gd > 0)
+    k_adap_tile<N, HELM, 2><<<dim3(gd, 16, 1), 256, 0, s>>>(T, R, A.ndtarg, A.targs, A.iquad, kp, A.wnear);
+  // (rules with two batched levels and a level cap of 2 leave nothing below)
+  bool below = gd > 0;
+  for (int r = 0; r < R.nrules; r++) below = below || R.lmax[r] > 2;
+  if (below)
+    k_adaptive<N, HELM><<<nwaves, 64, 0, s>>>(T, R, qctr, A.col_ind, A.ixyzs, A.srccoefs, A.ndtarg, A.targs, T.epsp,
+                                              kp, stack, unc, over);
+  if (gd > 0) k_adap_comb<NP, HELM><<<dim3(gd, 4), 256, 0, s>>>(T, R);
+  k_adap_final<NP, HELM><<<dim3(g, nz), 256, 0, s>>>(T, R, A.iquad, A.wnear);
+  HCHK(hipGetLastError());
+  return 0;
 }
 
 template <int N, bool HELM>
@@ -1750,23 +2153,22 @@ int run_order(const NearQuadArgs& A, NearQuadStats* st, hipStream_t s) {
   float* d_X = want_feat ? wsalloc<float>(W_X, (size_t)nadap * 8) : nullptr;
   int *d_pred = nullptr, *d_boff = nullptr, *d_bcnt = nullptr, *d_pfull = nullptr, *d_qctr = nullptr;
   int *d_lev = nullptr, *d_seg = nullptr, *d_unc = nullptr;
-  int2 *d_sorted = nullptr, *d_fb = nullptr;
+  int2* d_sorted = nullptr;
   if (want_feat && !d_X) return -2;
   if (nadap > 0) {
     d_bcnt = wsalloc<int>(W_BCNT, MLP_OUT * npat);
     d_boff = wsalloc<int>(W_BOFF, MLP_OUT * npat + 1);
-    d_sorted = wsalloc<int2>(W_SORTED, nadap);
-    d_qctr = wsalloc<int>(W_QCTR, 16);
+    d_sorted = wsalloc<int2>(W_SORTED, 2 * (size_t)nadap);
+    d_qctr = wsalloc<int>(W_QCTR, 8 * QUEUE_STRIDE);
     if (A.lev_host) d_lev = wsalloc<int>(W_LEV, A.nnz);
     if (A.unc_host) d_unc = wsalloc<int>(W_UNC, A.nnz);
     if (!d_bcnt || !d_boff || !d_sorted || !d_qctr || (A.lev_host && !d_lev) || (A.unc_host && !d_unc)) return -2;
   }
   if (learned) {
     d_pred = wsalloc<int>(W_PRED, nadap);
-    d_fb = wsalloc<int2>(W_FB, nadap);
     d_seg = wsalloc<int>(W_SEG, MAX_RULES + 1);
     if (A.pred_host) d_pfull = wsalloc<int>(W_PFULL, A.nnz);
-    if (!d_pred || !d_fb || !d_seg || (A.pred_host && !d_pfull)) return -2;
+    if (!d_pred || !d_seg || (A.pred_host && !d_pfull)) return -2;
   }
   HCHK(hipEventRecord(ev[5], s));
   if (want_feat) {
@@ -1780,39 +2182,53 @@ int run_order(const NearQuadArgs& A, NearQuadStats* st, hipStream_t s) {
     if (mlp_predict_device(A.mlp_params, d_X, nadap, d_pred, nullptr, s) != 0) return -1;
     if (d_pfull) HCHK(hipMemsetAsync(d_pfull, 0xff, sizeof(int) * A.nnz, s));
   }
+  if (d_nref) HCHK(hipMemsetAsync(d_nref, 0, sizeof(int) * A.nnz, s));
   if (d_lev) HCHK(hipMemsetAsync(d_lev, 0, sizeof(int) * A.nnz, s));
   if (d_unc) HCHK(hipMemsetAsync(d_unc, 0, sizeof(int) * A.nnz, s));
+  // places of the rule classes in the sorted list: those of another degree than the plain rule's
+  // first, from place nother on those of the plain rule
+  int place = 0, nother = 0;
+  int at[MAX_RULES] = {0};
+  if (learned) {
+    int k = 0;
+    for (int c = 0; c < MAX_RULES; c++)
+      if (class_degree(nqorder, c) != nqorder) at[c] = k++;
+    nother = k;
+    for (int c = 0; c < MAX_RULES; c++)
+      if (class_degree(nqorder, c) == nqorder) at[c] = k++;
+    for (int c = 0; c < MAX_RULES; c++) place |= at[c] << (4 * c);
+  }
   if (nadap > 0) {
     HCHK(hipMemsetAsync(d_bcnt, 0, sizeof(int) * MLP_OUT * npat, s));
-    HCHK(hipMemsetAsync(d_qctr, 0, sizeof(int) * 16, s));
-    k_bucket_count<<<(nadap + tb - 1) / tb, tb, 0, s>>>(nadap, d_adap, d_pred, A.col_ind, npat, d_bcnt);
+    k_bucket_count<<<(nadap + tb - 1) / tb, tb, 0, s>>>(nadap, nullptr, d_adap, d_pred, place, A.col_ind, npat, d_bcnt);
     k_scan<<<1, 1024, 0, s>>>(MLP_OUT * npat, d_bcnt, d_boff);
     HCHK(hipMemsetAsync(d_bcnt, 0, sizeof(int) * MLP_OUT * npat, s));
-    k_bucket_scatter<<<(nadap + tb - 1) / tb, tb, 0, s>>>(nadap, d_adap, d_pred, A.col_ind, npat, d_boff, d_bcnt,
-                                                          d_sorted, d_pfull);
+    k_bucket_scatter<<<(nadap + tb - 1) / tb, tb, 0, s>>>(nadap, nullptr, d_adap, d_pred, place, A.col_ind, npat,
+                                                          d_boff, d_bcnt, d_sorted, d_pfull);
     HCHK(hipGetLastError());
   }
-  // rule classes: the plain rule alone, or with a selector every class (class c: XG
-  // degree class_degree(nqorder, c), level cap from route_lmax) whose segment of the
-  // sorted list is not empty
-  AdapRules R = {};
+  // rules: the plain rule (P), and with a selector those of the other classes (R, class c: XG
+  // degree class_degree(nqorder, c), level cap from route_lmax) whose segment of the sorted list is
+  // not empty
+  AdapRules R = {}, P = {};
   int seg[MAX_RULES + 1] = {0};
-  int nroute = 0;  // routed classes with pairs
+  int nroute = 0;                  // classes with pairs
+  bool capped = false;             // a class of the plain rule has a level cap
+  auto plain_rule = [&](AdapRules& D, int lmax, int64_t b0) {
+    const int r = D.nrules++;
+    D.ndeep++;
+    D.b0[r] = b0;
+    D.kq[r] = kq;
+    D.lmax[r] = lmax;
+    D.npar[r] = npar_plain;
+    D.xg[r] = d_xg;
+    D.ptab[r] = d_ptab;
+    D.cache[r] = d_cache;
+  };
   if (learned) {
     k_seg_bounds<<<1, 64, 0, s>>>(MAX_RULES, npat, d_boff, d_seg);
     HCHK(hipMemcpyAsync(seg, d_seg, sizeof(int) * (MAX_RULES + 1), hipMemcpyDeviceToHost, s));
     HCHK(hipStreamSynchronize(s));
-    R.nrules = MAX_RULES;
-    for (int c = 0; c <= MAX_RULES; c++) R.seg[c] = seg[c];
-  } else {
-    R.nrules = 1;
-    R.seg[0] = 0;
-    R.seg[1] = nadap;
-    R.kq[0] = kq;
-    R.lmax[0] = NLMAX;
-    R.npar[0] = npar_plain;
-    R.xg[0] = d_xg;
-    R.ptab[0] = d_ptab;
   }
   HCHK(hipEventRecord(ev[6], s));
   if (nadap > 0) {
@@ -1825,61 +2241,134 @@ int run_order(const NearQuadArgs& A, NearQuadStats* st, hipStream_t s) {
     }
     HCHK(hipEventRecord(ev[11], s));
     if (learned) {
-      // tree caches of the routed classes (the plain class shares the plain cache)
+      // tree caches of the classes of other rules (those of the plain rule share its cache)
       for (int c = 0; c < MAX_RULES; c++) {
         const int q = class_degree(nqorder, c);
-        const RuleTables* RT = nullptr;
-        if (rule_tables<N>(q, &RT, s) != 0) return -2;
-        R.kq[c] = RT->kq;
-        R.xg[c] = RT->xg;
-        R.ptab[c] = RT->ptab;
-        R.lmax[c] = A.route_lmax ? A.route_lmax[c] : NLMAX;
-        if (R.lmax[c] < 1 || R.lmax[c] > NLMAX) R.lmax[c] = NLMAX;
-        R.cache[c] = nullptr;
-        if (seg[c + 1] == seg[c]) continue;
+        if (seg[at[c] + 1] == seg[at[c]]) continue;
         nroute++;
+        int lmax = A.route_lmax ? A.route_lmax[c] : NLMAX;
+        if (lmax < 1 || lmax > NLMAX) lmax = NLMAX;
         if (q == nqorder) {
-          R.npar[c] = npar_plain;
-          R.cache[c] = d_cache;
+          plain_rule(P, lmax, at[c] * npat);
+          capped = capped || lmax < NLMAX;
           continue;
         }
+        const RuleTables* RT = nullptr;
+        if (rule_tables<N>(q, &RT, s) != 0) return -2;
+        const int r = R.nrules++;
+        R.b0[r] = at[c] * npat;
+        R.kq[r] = RT->kq;
+        R.xg[r] = RT->xg;
+        R.ptab[r] = RT->ptab;
+        R.lmax[r] = lmax;
         // the class's pairs evaluate no triangle below depth lmax (deeper ones go back to
         // the plain integrator); its cache holds depths 0 .. min(2, lmax): the pairs routed
         // to a rule of another degree mostly end at levels 1 and 2 (on the wavy torus, 99%
         // of them), and a deeper cache would cost every generation 4 times as much for
         // the few refinement tests below it
-        R.npar[c] = cache_parents(R.lmax[c] < 2 ? R.lmax[c] : 2);
-        const int ntri = cache_tris(R.npar[c]);
+        R.npar[r] = cache_parents(lmax < 2 ? lmax : 2);
+        const int ntri = cache_tris(R.npar[r]);
         double* cc = wsalloc<double>(W_RCACHE0 + c, (size_t)npat * CACHE_STRIDE * ntri * RT->kq);
         if (!cc) return -2;
         launch_tree_cache<N>(npat, ntri * RT->kq, RT->twq, RT->ptab, A.ixyzs, A.srccoefs, cc, s);
-        R.cache[c] = cc;
+        R.cache[r] = cc;
       }
       HCHK(hipGetLastError());
     } else {
-      R.cache[0] = d_cache;
+      plain_rule(P, NLMAX, 0);
     }
     HCHK(hipEventRecord(ev[7], s));
-    const int g = nadap < nwaves ? nadap : nwaves;
-    launch_adaptive<N, HELM>(g, s, nadap, nullptr, d_sorted, R, d_fb, d_counts + 4, d_qctr, A, d_epsp, d_umat,
-                             kp, d_stack, d_nref, d_lev, d_unc, d_over);
-    HCHK(hipGetLastError());
-    if (learned) {
-      // pairs whose tree went past their class's level: the plain rule and level cap
-      AdapRules P0 = {};
-      P0.nrules = 1;
-      P0.seg[0] = 0;
-      P0.seg[1] = 0x7fffffff;
-      P0.kq[0] = kq;
-      P0.lmax[0] = NLMAX;
-      P0.npar[0] = npar_plain;
-      P0.xg[0] = d_xg;
-      P0.ptab[0] = d_ptab;
-      P0.cache[0] = d_cache;
-      launch_adaptive<N, HELM>(g, s, 0, d_counts + 4, d_fb, P0, nullptr, nullptr, d_qctr + 8, A, d_epsp,
-                               d_umat, kp, d_stack, d_nref, d_lev, d_unc, d_over);
-      HCHK(hipGetLastError());
+    constexpr int VL = NP * (HELM ? 2 : 1);
+    const int64_t all = SLOTS_ALL * (int64_t)nadap;
+    const bool bounded = (size_t)all * 4 * VL * sizeof(double) > SLOT_ALL_BYTES;
+    AdapTiles T = {};
+    T.cap = (int)(bounded ? (int64_t)(SLOTS_PER_PAIR * nadap) : all);
+    T.slots = wsalloc<double>(W_SLOTS, (size_t)T.cap * 4 * VL);
+    T.items = wsalloc<int4>(W_ITEMS, T.cap);
+    T.list1 = wsalloc<int2>(W_LIST1, nadap);
+    T.list2 = wsalloc<int4>(W_LIST2, 4 * (size_t)nadap);
+    if (!T.slots || !T.items || !T.list1 || !T.list2) return -2;
+    T.boff = d_boff;
+    T.npat = (int)npat;
+    T.epsp = d_epsp;
+    T.umat = d_umat;
+    T.nref = d_nref;
+    T.lev = d_lev;
+    // Passes: the classes of other rules, whose pairs may be sent back by their level caps; the
+    // pairs of the plain rule, and with them those sent back (on their own a few hundred of them
+    // cost 0.3 ms of launches with most of the device idle); then pairs that the second pass
+    // sent back (no slot left, or a level cap for the plain rule), by the plain rule without a cap
+    // and as many at a time as the pool is sure to hold, so that none is sent back again.
+    const bool resend = bounded || learned;
+    int* d_flag = nullptr;
+    int2 *s0 = d_sorted, *s1 = d_sorted + nadap, *s2nd = nullptr;
+    if (resend) {
+      d_flag = wsalloc<int>(W_FLAG, nadap);
+      s2nd = wsalloc<int2>(W_FB, nadap);
+      if (!d_flag || !s2nd) return -2;
     }
+    // back: counters of pairs sent back to T.fb (all, past the cap; null: none can be), zero before
+    auto pass = [&](const AdapRules& rules, int n, int2* fb, int* back) -> int {
+      T.fb = fb;
+      T.flag = back ? d_flag : nullptr;
+      T.nfb = back;
+      T.npast = back ? back + 1 : nullptr;
+      if (back) HCHK(hipMemsetAsync(d_flag, 0, sizeof(int) * nadap, s));
+      const int rc = run_tiles<N, HELM>(A, rules, T, n, nwaves, kp, d_stack, d_qctr, d_unc, d_over, s);
+      if (!rc && back && (d_nref || d_lev || d_unc)) {
+        k_adap_reset<<<(unsigned)((nadap + tb - 1) / tb), tb, 0, s>>>(back, fb, d_nref, d_lev, d_unc);
+        HCHK(hipGetLastError());
+      }
+      return rc;
+    };
+    auto sent_back = [&](const int* back, int* n) -> int {
+      HCHK(hipMemcpyAsync(n, back, sizeof(int), hipMemcpyDeviceToHost, s));
+      HCHK(hipStreamSynchronize(s));
+      return 0;
+    };
+    // n pairs of list and *more after them (at most nadap in all), by patch, to out
+    auto sort_plain = [&](int n, const int* more, const int2* list, int2* out) -> int {
+      const unsigned nbk = (unsigned)(((more ? nadap : n) + tb - 1) / tb);
+      HCHK(hipMemsetAsync(d_bcnt, 0, sizeof(int) * npat, s));
+      k_bucket_count<<<nbk, tb, 0, s>>>(n, more, list, nullptr, 0, A.col_ind, npat, d_bcnt);
+      k_scan<<<1, 1024, 0, s>>>(npat, d_bcnt, d_boff);
+      HCHK(hipMemsetAsync(d_bcnt, 0, sizeof(int) * npat, s));
+      k_bucket_scatter<<<nbk, tb, 0, s>>>(n, more, list, nullptr, 0, A.col_ind, npat, d_boff, d_bcnt, out, nullptr);
+      HCHK(hipGetLastError());
+      return 0;
+    };
+    const int nplain = learned ? nadap - seg[nother] : nadap;
+    int *back1 = d_counts + 4, *back2 = d_counts + 6;
+    int nleft[2] = {0, 0}, rc = 0;
+    T.sorted = s0;
+    if (nplain < nadap && (rc = pass(R, nadap - nplain, s1, back1))) return rc;
+    AdapRules P0 = {};
+    plain_rule(P0, NLMAX, 0);
+    // (the plain rule's segment ends where the pairs sent back begin; how many these are the device
+    // knows)
+    const bool join = nplain < nadap && !capped;
+    if (join) {
+      if ((rc = sort_plain(nplain, back1, s0 + (nadap - nplain), s2nd))) return rc;
+      T.sorted = s2nd;
+    } else if (nplain < nadap && (rc = sent_back(back1, nleft))) {
+      return rc;
+    }
+    int2* fb2 = join ? s0 : s2nd;
+    if (nplain > 0 || join) {
+      const bool back = bounded || capped;
+      if ((rc = pass(join ? P0 : P, nplain, fb2, back ? back2 : nullptr))) return rc;
+      if (back && (rc = sent_back(back2, nleft + 1))) return rc;
+    }
+    const int2* left[2] = {s1, fb2};
+    const int most = T.cap / SLOTS_ALL > 0 ? T.cap / SLOTS_ALL : 1;
+    int2* spare = join ? s2nd : s0;  // holds neither list
+    T.sorted = spare;
+    for (int l = 0; l < 2; l++)
+      for (int i = 0; i < nleft[l]; i += most) {
+        const int n = nleft[l] - i < most ? nleft[l] - i : most;
+        if ((rc = sort_plain(n, nullptr, left[l] + i, spare))) return rc;
+        if ((rc = pass(P0, n, nullptr, nullptr))) return rc;
+      }
   } else {
     if (!early_tree) {
       HCHK(hipEventRecord(ev[9], s));
@@ -1920,8 +2409,8 @@ int run_order(const NearQuadArgs& A, NearQuadStats* st, hipStream_t s) {
     st->ms_self = elapsed(12, 13);
     st->nroute = nroute;
     st->cache_tris = ntri_plain;
-    st->nfallback = counts8[4];
-    for (int c = 0; c < MAX_RULES; c++) st->ncls[c] = learned ? seg[c + 1] - seg[c] : (c == 0 ? nadap : 0);
+    st->nfallback = counts8[5] + counts8[7];
+    for (int c = 0; c < MAX_RULES; c++) st->ncls[c] = learned ? seg[at[c] + 1] - seg[at[c]] : (c == 0 ? nadap : 0);
     st->nref_total = 0;
     if (d_nref && A.nref_host) HCHK(hipMemcpy(A.nref_host, d_nref, sizeof(int) * A.nnz, hipMemcpyDeviceToHost));
     if (A.class_host) HCHK(hipMemcpy(A.class_host, d_cls, sizeof(int) * A.nnz, hipMemcpyDeviceToHost));

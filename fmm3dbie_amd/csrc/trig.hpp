@@ -1,4 +1,6 @@
-// sin and cos of an FP64 argument of bounded size, for the Helmholtz kernel evaluations.
+// sin and cos of FP64 arguments of bounded size, for the Helmholtz kernel evaluations
+// (sincos_turns: far sums; sincos_half_pi: quadrature, with the reduction of sincos_near in
+// common.hpp) and for callers of the library on the host (sincos_red).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -95,4 +97,37 @@ __host__ __device__ __forceinline__ void sincos_turns(double r, double khi, doub
   } b;
   b.d = m;
   neg = b.u & 1;
+}
+
+// sin x and cos x for |x| <= pi/2 without a reduction: minimax polynomials (sin x / x - 1) / x^2
+// and (cos x - 1) / x^2 of degree 7 in x^2 (Remez exchange in 300 bits, errors 2.0e-19 and
+// 4.3e-18).
+// The coefficients are kept in scalar registers (scalar_const): as literals each costs two
+// vector moves at every use, as many instructions as the polynomials themselves.
+__device__ __forceinline__ double scalar_const(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("" : "+s"(x));
+#endif
+  return x;
+}
+__device__ __forceinline__ void sincos_half_pi(double x, double& s, double& c) {
+  const double z = x * x;
+  double ps = scalar_const(0x1.87cf34cb45316p-49);
+  ps = fma(ps, z, scalar_const(-0x1.ae3f72f9ed52ap-41));
+  ps = fma(ps, z, scalar_const(0x1.6123bb933d336p-33));
+  ps = fma(ps, z, scalar_const(-0x1.ae645485a9287p-26));
+  ps = fma(ps, z, scalar_const(0x1.71de3a51d914ep-19));
+  ps = fma(ps, z, scalar_const(-0x1.a01a01a012a97p-13));
+  ps = fma(ps, z, scalar_const(0x1.1111111111098p-7));
+  ps = fma(ps, z, scalar_const(-0x1.5555555555555p-3));
+  s = fma(ps, z * x, x);
+  double pc = scalar_const(0x1.9f4e7cd1ca798p-45);
+  pc = fma(pc, z, scalar_const(-0x1.93525f737d4a0p-37));
+  pc = fma(pc, z, scalar_const(0x1.1eece69a30ce8p-29));
+  pc = fma(pc, z, scalar_const(-0x1.27e4f99a6d27fp-22));
+  pc = fma(pc, z, scalar_const(0x1.a01a0199f59b7p-16));
+  pc = fma(pc, z, scalar_const(-0x1.6c16c16c0b99ap-10));
+  pc = fma(pc, z, scalar_const(0x1.555555555541ep-5));
+  pc = fma(pc, z, scalar_const(-0x1.ffffffffffffdp-2));
+  c = fma(pc, z, 1.0);
 }

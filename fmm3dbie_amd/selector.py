@@ -16,8 +16,8 @@ level past its class's cap is integrated again by the plain integrator.
 
 Labels come from the integrator itself: every adaptive pair is integrated once per class
 (forced routing, no cap) and labelled with the class of least cost, the cost being the
-pair's own work in 64-node chunks (on the cached tree, and below it where the geometry
-is computed) weighted by unit costs fitted to the measured launch times of the six
+pair's own work (node steps on the cached tree, 64-node chunks below it where the
+geometry is computed) weighted by unit costs fitted to the measured launch times of the six
 classes; the class's level cap is the deepest tree among the training pairs labelled
 with it, and its tree cache holds no depth below that cap.
 
@@ -98,7 +98,7 @@ def per_triangle(norder, kq):
 
 
 def chunks(norder, kq):
-    """Chunks of the adaptive kernel's root step and of a refinement test with a rule of
+    """Chunks of the adaptive kernel for one triangle and for a refinement test with a rule of
     kq nodes: one per triangle (per_triangle), else the nodes of the step in equal
     chunks."""
     if per_triangle(norder, kq):
@@ -107,24 +107,32 @@ def chunks(norder, kq):
     return -(-kq // cr), -(-4 * kq // cr)
 
 
+# Cost of a node step on the cached tree in chunks of the subtrees below it, measured on the
+# deformed sphere of order 6: 25 ps per pair and step, 2.2 ns per chunk.
+STEP_CHUNKS = 0.011
+
+
+def tile_steps(kq):
+    """Node steps of a triangle in the batched levels (4 nodes of 16 targets a step)."""
+    return -(-kq // 4)
+
+
 def collect(nq, stream=None):
     """Features of every adaptive pair (from a plain run) and its label: the rule class
     whose adaptive integration takes the least time.  Every pair is integrated once
     with each class (forced routing, no level cap, every kernel in order on one stream).
-    The kernel works in chunks of at most chunk_rows(norder) nodes (one node per lane;
-    chunks() counts them for the root and a refinement test), and a
-    chunk costs the same whether its lanes are all busy or not, so the measured time of
-    each class's launch is fitted by a cost per chunk on the cached tree (one for the
-    classes with a chunk per triangle, one for the others: the two code paths), a
-    cost per chunk below it (geometry evaluated) and a cost per pair, summed over the
-    pairs' own counts; the label is the class of least fitted chunk cost among the
-    classes worth their tree cache (open_classes).  Returns (X
-    (nadap, 8) float32, y (nadap,) int32, CSR entry index of each adaptive pair, info
-    with the per-class fitted cost 'cost', kernel evaluations 'evals', deepest levels
-    'lev' (6, nadap), launch times 'ms', the fitted unit costs 'unit' (ms per cached
-    chunk of the per-triangle classes and of the others, per computed chunk, per pair),
-    node counts 'kq', the plain degree 'q0', the
-    classes used 'used' and the plain rule's tree-cache time for depths 0..2 'ms_tree')."""
+    The first levels of the trees are integrated in steps of 4 nodes for 16 targets at a
+    time (tile_steps per triangle), the subtrees below them in chunks of at most
+    chunk_rows(norder) nodes (chunks() per refinement test; a chunk costs the same whether
+    its lanes are all busy or not).  A pair's work is its steps on the cached tree, at
+    STEP_CHUNKS chunks each, and its chunks below it (geometry evaluated); the measured times
+    of the six launches are fitted by a cost per chunk and a cost per pair, and the label is
+    the class of least fitted cost among the classes worth their tree cache (open_classes).
+    Returns (X (nadap, 8) float32, y (nadap,) int32, CSR entry index of each adaptive pair,
+    info with the per-class fitted cost 'cost', kernel evaluations 'evals', deepest levels
+    'lev' (6, nadap), launch times 'ms', the fitted unit costs 'unit' (ms per chunk, per
+    pair), node counts 'kq', the plain degree 'q0', the classes used 'used' and the plain
+    rule's tree-cache time for depths 0..2 'ms_tree')."""
     from scipy.optimize import nnls
     from . import layer
     torch = _torch()
@@ -155,21 +163,20 @@ def collect(nq, stream=None):
             unc = st["unc"][idx].astype(np.float64)
             ncached[c] = kq[c] * (1 + 4 * (nref - unc))
             ncomp[c] = kq[c] * 4 * unc
-            croot, cstep = chunks(nq.norder, kq[c])
-            ccached[c] = croot + cstep * (nref - unc)
-            ccomp[c] = cstep * unc
+            ccached[c] = tile_steps(kq[c]) * (1 + 4 * (nref - unc))
+            ccomp[c] = chunks(nq.norder, kq[c])[1] * unc
             lev[c] = st["lev"][idx]
             ms[c] = st["ms_adap"]
     finally:
         layer.set_side_stream(side)
-    # a cost per pair (queue, staging, weights: the same for every class) keeps the chunk
-    # costs from absorbing it
-    tri = np.array([per_triangle(nq.norder, int(k)) for k in kq])
-    A = np.stack([np.where(tri, ccached.sum(1), 0.0), np.where(tri, 0.0, ccached.sum(1)), ccomp.sum(1),
-                  np.full(NCLASS, float(len(idx)))], 1)
-    unit, _ = nnls(A, ms)
-    cost = np.where(tri, unit[0], unit[1])[:, None] * ccached + unit[2] * ccomp
-    y, used = open_classes(cost, tree_cost(ms_tree, kq, q0))
+    # a cost per pair (lists, test, weights: the same for every class) keeps the step costs from
+    # absorbing it
+    work = STEP_CHUNKS * ccached + ccomp
+    unit, _ = nnls(np.stack([work.sum(1), np.full(NCLASS, float(len(idx)))], 1), ms)
+    cost = unit[0] * work
+    tree = tree_cost(ms_tree, kq, q0)
+    fill = np.where(tree > 0.0, fill_cost(nq.npatches, kq, STEP_CHUNKS * unit[0]), 0.0)
+    y, used = open_classes(cost, tree + fill)
     return X, y, idx, dict(cost=cost, evals=ncached + ncomp, lev=lev, ms=ms, unit=unit, kq=kq, q0=q0,
                            used=used, ms_tree=ms_tree)
 
@@ -184,9 +191,19 @@ def tree_cost(ms_tree, kq, q0):
     return c
 
 
+def fill_cost(npatches, kq, step):
+    """Cost of the partly filled tiles that one more class brings: the batched levels take 16
+    targets of a patch and class at a time, so a class leaves half a tile empty at the root
+    and at each of its children (5 triangles each), step being the cost per pair and node
+    step.  Measured on the wavy torus of order 6 (1536 patches, plain 6.2 ms): classes
+    of 79, 112 and 150 nodes beside the plain one 5.75 ms with the first alone, 5.80 with
+    two, 6.00 with all three, whose pairs alone would save 0.65, 0.90 and 1.06 ms."""
+    return 8.0 * npatches * 25 * step * np.array([tile_steps(int(k)) for k in kq])
+
+
 def open_classes(cost, cache):
     """Which rule classes to use and each pair's label.  A class other than the plain one
-    costs the build of its tree cache once per generation (cache[c], same unit as cost);
+    costs its tree cache and partly filled tiles once per generation (cache[c], same unit as cost);
     starting from the plain class alone, the class whose pairs would save the most
     (sum over pairs of the drop in their least cost, minus its cache) is added while that
     saving is positive.  Returns (labels: the least-cost used class of every pair, used
@@ -209,11 +226,12 @@ def open_classes(cost, cache):
 
 def level_caps(y, info):
     """Level cap of each class: the deepest tree among the pairs labelled with it (20,
-    the integrator's own cap, for a class without pairs)."""
+    the integrator's own cap, for a class without pairs and for the plain class: a pair sent
+    back from there would be integrated the same way once more)."""
     caps = np.full(NCLASS, 20, np.int32)
     for c in range(NCLASS):
         m = y == c
-        if m.any():
+        if c != PLAIN_CLASS and m.any():
             caps[c] = max(1, int(info["lev"][c][m].max()))
     return caps
 
