@@ -462,6 +462,232 @@ __global__ void __launch_bounds__(64 * FW) k_farsum_mfma(int ntarg, const T* __r
   }
 }
 
+// Far sum of NG = 2, 3 or 4 groups of 16 right-hand sides, FP32 (grid z: NG groups each).  The kernel
+// values are computed once for all groups, and the products run in bfloat16, where the matrix
+// cores have sixteen times their FP32 rate, exact products and FP32 sums: each value is split
+// into three bfloat16 terms (hi + mid + lo, rounded to nearest, is the FP32 value to its last bit),
+// and six products of terms take the place of one (those left out are below 2^-26 of it).
+// A wavefront takes MT tiles of 16 targets; in a tile of ST = 32 sources lane l evaluates the pairs
+// (target l % 16, sources 8 (l / 16) ..) on the vector units, which are the operand of the 16x16x32
+// products as they stand.  The workgroup stages the sources' geometry and the split strengths in
+// LDS, in the order in which the lanes read them; the next tile's are loaded while one is summed.
+// Bound by issue: per 64 pairs and group 36 x 4.5 cycles of products, 40 instructions of kernel
+// values and splits per pair, and the staging, which MT = 2 tiles share.  The apply of 86016
+// points (139206 sources) in FP32 products, a group at a time, against this: 32 densities 32.7 to
+// 21.9 ms, 48 49.0 to 29.0, 64 65.4 to 34.3, its error against the FP64 apply 1.7e-6 to 1.3e-6, 2.2e-6
+// to 1.7e-6 and 2.4e-6 to 1.9e-6.  One group keeps the FP32 products (16.5 against 17.9 ms: the
+// splits cost what the products save).
+typedef float flt2 __attribute__((ext_vector_type(2)));
+typedef float flt4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+constexpr int ST = 32;        // sources per tile
+constexpr int SPLIT_MAX = 4;  // groups per wavefront
+struct Split8 {               // the terms of eight values
+  union {
+    bf8 v;
+    bf2 p[4];
+  } t[3];
+};
+// The next terms of a and b, which keep what is left
+__device__ __forceinline__ bf2 next_term(float& a, float& b) {
+  const bf2 h = __builtin_convertvector(flt2{a, b}, bf2);
+  a -= (float)h.x;
+  b -= (float)h.y;
+  return h;
+}
+
+template <int KIND, int NG>
+__global__ void __launch_bounds__(64 * FW, 2)
+    k_farsum_split(int ntarg, const float* __restrict__ tx, const float* __restrict__ ty, const float* __restrict__ tz,
+                   int nsrc, const float* __restrict__ geo, const int64_t* __restrict__ ixyzso,
+                   const V2<float>* __restrict__ str, const int64_t* __restrict__ row_ptr,
+                   const int* __restrict__ near_sorted, FarPar<float> P, int chunk, int nrhs,
+                   V2<float>* __restrict__ part, int64_t ldpart) {
+  using T = float;
+  constexpr int NM = KIND == 0 ? 1 : 3;  // kernel matrices: Re K, Im K, Re K + Im K
+  constexpr int NB = KIND == 0 ? 2 : 3;  // strength matrices: Re s, Im s, Re s + Im s
+  constexpr int SI = NG == 2 ? 4 : 8;    // sources that a thread stages, of one right-hand side
+  constexpr int NT = MT<T>;
+  __shared__ __align__(16) T lgeo[ST * 8];
+  __shared__ __align__(16) bf8 lstr[NG][NB][3][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int g0 = blockIdx.z * NG, ngrp = (nrhs + MG - 1) / MG;
+  const int t0 = (blockIdx.x * FW + wv) * (16 * NT);
+  const int ks = lane >> 4;  // this lane's sources: 8 ks .. 8 ks + 7 of a tile
+  const int jbeg = blockIdx.y * chunk;
+  const int jend = jbeg + chunk < nsrc ? jbeg + chunk : nsrc;
+  T x[NT], y[NT], z[NT];
+  NearCursor nc[NT];
+  bool act[NT];
+#pragma unroll
+  for (int t = 0; t < NT; t++) {
+    const int i = t0 + 16 * t + (lane & 15);
+    act[t] = i < ntarg;
+    x[t] = act[t] ? tx[i] : (T)0;
+    y[t] = act[t] ? ty[i] : (T)0;
+    z[t] = act[t] ? tz[i] : (T)0;
+    nc[t] = NearCursor{near_sorted, ixyzso};
+    if (act[t] && jbeg < jend) {
+      nc[t].ptr = row_ptr[i] - 1;
+      nc[t].end = row_ptr[i + 1] - 1;
+      nc[t].seek(jbeg);
+    }
+  }
+  // this thread's part of a tile: right-hand side sr of group sg, sources sj .. sj + SI - 1
+  const int sr = threadIdx.x & 15, sj = SI * ((threadIdx.x >> 4) % (ST / SI)), sg = (threadIdx.x >> 4) / (ST / SI);
+  const bool stager = sg < NG, live = stager && g0 + sg < ngrp;
+  const V2<T>* sp = str + (int64_t)(live ? g0 + sg : 0) * nsrc * MG + sr;
+  V2<T> next[SI];
+  T nextg;  // and one value of the geometry
+  static_assert(ST * 8 == 64 * FW, "");
+  // (loads without a condition, in flight together while a tile is summed; sources past the chunk
+  // and groups past the last are zeroed below)
+  auto load = [&](int base) {
+#pragma unroll
+    for (int u = 0; u < SI; u++) {
+      const int j = base + sj + u;
+      next[u] = sp[(int64_t)(j < nsrc ? j : nsrc - 1) * MG];
+    }
+    const int64_t e = (int64_t)base * 8 + threadIdx.x;
+    nextg = geo[e < (int64_t)nsrc * 8 ? e : 0];
+  };
+  auto stage = [&](int base) {
+    lgeo[threadIdx.x] = base + (int)(threadIdx.x / 8) < jend ? nextg : (T)0;
+#pragma unroll
+    for (int u = 0; u < SI; u++)
+      if (!live || base + sj + u >= jend) next[u] = V2<T>{0.0f, 0.0f};
+    if (!stager) return;
+    bf2* o = reinterpret_cast<bf2*>(&lstr[sg][0][0][sj / 8 * 16 + sr]) + (sj % 8) / 2;
+#pragma unroll
+    for (int m = 0; m < NB; m++) {
+      bf2 v[3][SI / 2];
+#pragma unroll
+      for (int u = 0; u < SI; u += 2) {
+        T a = m == 0 ? next[u].x : (m == 1 ? next[u].y : next[u].x + next[u].y);
+        T b = m == 0 ? next[u + 1].x : (m == 1 ? next[u + 1].y : next[u + 1].x + next[u + 1].y);
+#pragma unroll
+        for (int k = 0; k < 3; k++) v[k][u / 2] = next_term(a, b);
+      }
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        bf2* q = o + (m * 3 + k) * 64 * 4;
+        if constexpr (SI == 8) *reinterpret_cast<bf8*>(q) = *reinterpret_cast<const bf8*>(v[k]);
+        else *reinterpret_cast<bf4*>(q) = *reinterpret_cast<const bf4*>(v[k]);
+      }
+    }
+  };
+  flt4 acc[NT][NG][NB];
+#pragma unroll
+  for (int t = 0; t < NT; t++)
+#pragma unroll
+    for (int g = 0; g < NG; g++)
+#pragma unroll
+      for (int m = 0; m < NB; m++) acc[t][g][m] = flt4{0.0f, 0.0f, 0.0f, 0.0f};
+  if (jbeg < jend) load(jbeg);
+#pragma unroll 1
+  for (int base = jbeg; base < jend; base += ST) {
+    __syncthreads();
+    stage(base);
+    __syncthreads();
+    if (base + ST < jend) load(base + ST);
+    bool mine = base + ST <= jend;
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      if (base >= nc[t].eb) nc[t].seek(base);
+      mine = mine && act[t] && nc[t].ea >= base + ST;
+    }
+    Split8 A[NT][NM];
+    // FULL: no source of the step is skipped for any target of the wavefront
+    auto eval = [&](auto full_tag) {
+      constexpr bool FULL = decltype(full_tag)::value;
+#pragma unroll
+      for (int u = 0; u < 8; u += 2) {
+        T gg[2][6];
+#pragma unroll
+        for (int v = 0; v < 2; v++)
+#pragma unroll
+          for (int e = 0; e < 6; e++) gg[v][e] = lgeo[(8 * ks + u + v) * 8 + e];
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+          T vr[2], vi[2], vs[2];
+#pragma unroll
+          for (int v = 0; v < 2; v++) {
+            const T* g = gg[v];
+            const T dx = x[t] - g[0], dy = y[t] - g[1], dz = z[t] - g[2];
+            const T r2 = dx * dx + dy * dy + dz * dz;
+            const T d = dx * g[3] + dy * g[4] + dz * g[5];
+            T rinv = far_rsqrt(r2);
+            if constexpr (!FULL) {
+              const int j = base + 8 * ks + u + v;
+              if (j >= nc[t].eb) nc[t].seek(j);
+              rinv = (act[t] && j < jend && j < nc[t].ea) ? rinv : (T)0;
+            }
+            T gr, gi, c, s, q;
+            pair_factors<T, KIND>(r2, rinv, d, P, gr, gi, c, s, q);
+            pair_value<T, KIND>(gr, gi, c, s, q, vr[v], vi[v]);
+            vs[v] = vr[v] + vi[v];
+          }
+#pragma unroll
+          for (int k = 0; k < 3; k++) {
+            A[t][0].t[k].p[u / 2] = next_term(vr[0], vr[1]);
+            if constexpr (NM == 3) {
+              A[t][NM - 2].t[k].p[u / 2] = next_term(vi[0], vi[1]);
+              A[t][NM - 1].t[k].p[u / 2] = next_term(vs[0], vs[1]);
+            }
+          }
+        }
+      }
+    };
+    if (__all(mine)) eval(std::true_type{});
+    else eval(std::false_type{});
+    // products, GB groups at a time (a register each more at 4 groups would halve the occupancy)
+    constexpr int GB = NG == 4 ? 1 : 2;
+#pragma unroll
+    for (int m = 0; m < NB; m++)
+#pragma unroll
+      for (int h = 0; h < NG; h += GB) {
+        bf8 b[GB][3];
+#pragma unroll
+        for (int g = 0; g < GB && h + g < NG; g++)
+#pragma unroll
+          for (int k = 0; k < 3; k++) b[g][k] = lstr[h + g][m][k][lane];
+        auto mul = [&](int ka, int kb) {
+#pragma unroll
+          for (int g = 0; g < GB && h + g < NG; g++)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+              acc[t][h + g][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[t][NM == 1 ? 0 : m].t[ka].v, b[g][kb],
+                                                                        acc[t][h + g][m], 0, 0, 0);
+        };
+        mul(2, 0);
+        mul(0, 2);
+        mul(1, 1);
+        mul(1, 0);
+        mul(0, 1);
+        mul(0, 0);
+      }
+  }
+#pragma unroll
+  for (int t = 0; t < NT; t++)
+#pragma unroll
+    for (int g = 0; g < NG; g++) {
+      const int r = (g0 + g) * MG + (lane & 15);
+      if (r >= nrhs) continue;
+      const flt4 a1 = acc[t][g][0], a2 = acc[t][g][1], a3 = acc[t][g][NB - 1];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int it = t0 + 16 * t + Mfma16<T>::row(lane, e);
+        if (it >= ntarg) continue;
+        V2<T> v;
+        if constexpr (KIND == 0) v = {a1[e], a2[e]};
+        else v = {a1[e] - a2[e], a3[e] - a1[e] - a2[e]};
+        part[(int64_t)blockIdx.y * ldpart + (int64_t)r * ntarg + it] = v;
+      }
+    }
+}
+
 // pot[r][i] = (sum over source splits of part) / (4 pi)
 template <typename T>
 __global__ void k_farsum_reduce(int64_t ntarg, int nrhs, int nsplit, const V2<T>* __restrict__ part,
@@ -1053,24 +1279,45 @@ static int launch_far(ApplyPlan* P, bool mask, int64_t wg_target, const V2<T>* s
 }
 
 // The matrix-core far sum: groups of 16 right-hand sides, the last one padded with zeros.
+// FP32 blocks of several groups take the split products, up to SPLIT_MAX groups at a time.
 template <typename T>
 static int launch_far_mfma(ApplyPlan* P, bool mask, int64_t wg_target, const V2<T>* str, int nrhs, V2<T>* part,
                            int64_t part_cap, int64_t* nsplit_out, hipStream_t s) {
   const T* const* trg = targets_of<T>(P);
   const unsigned g = nblk(P->ntarg, 16 * FW * MT<T>);
   const int ngrp = (nrhs + MG - 1) / MG;
+  const int ng = sizeof(T) == 4 && ngrp <= SPLIT_MAX ? ngrp : 1;
   int64_t chunk;
-  const int64_t nsplit = split_sources(P->nptso, FT, (int64_t)g * ngrp, wg_target, FAR_FILL / FW,
+  const int64_t nsplit = split_sources(P->nptso, FT, (int64_t)g * (ngrp / ng), wg_target, FAR_FILL / FW,
                                        part_cap / ((int64_t)nrhs * P->ntarg), &chunk);
-  const dim3 grid(g, (unsigned)nsplit, (unsigned)ngrp);
+  const dim3 grid(g, (unsigned)nsplit, (unsigned)(ngrp / ng));
   const T th2 = (T)(P->thresh * P->thresh);
+  const int kind = far_kind<T>(P);
+  if constexpr (sizeof(T) == 4) {
+#define FMM_FARS(KD, NG)                                                                                          \
+  k_farsum_split<KD, NG><<<grid, 64 * FW, 0, s>>>((int)P->ntarg, trg[0], trg[1], trg[2], (int)P->nptso,           \
+                                                  sources_of<T>(P), P->ixyzso, str, P->row_ptr, P->near_sorted,   \
+                                                  far_par<T>(P), (int)chunk, nrhs, part, (int64_t)nrhs * P->ntarg)
+#define FMM_FARK(NG)                     \
+  do {                                   \
+    if (kind == 0) FMM_FARS(0, NG);      \
+    else if (kind == 1) FMM_FARS(1, NG); \
+    else FMM_FARS(2, NG);                \
+  } while (0)
+    if (ng == 2) FMM_FARK(2);
+    else if (ng == 3) FMM_FARK(3);
+    else if (ng == 4) FMM_FARK(4);
+#undef FMM_FARK
+#undef FMM_FARS
+  }
 #define FMM_FARM(MK, KD)                                                                                       \
   k_farsum_mfma<T, MK, KD><<<grid, 64 * FW, 0, s>>>((int)P->ntarg, trg[0], trg[1], trg[2], (int)P->nptso,      \
                                                    sources_of<T>(P), P->ixyzso, str, P->row_ptr,               \
                                                    P->near_sorted, far_par<T>(P), th2, (int)chunk, nrhs, part, \
                                                    (int64_t)nrhs * P->ntarg)
-  const int kind = far_kind<T>(P);
-  if (mask || sizeof(T) == 4) {
+  if (ng > 1) {
+    // launched above
+  } else if (mask || sizeof(T) == 4) {
     if (kind == 0) FMM_FARM(true, 0);
     else if (kind == 1) FMM_FARM(true, 1);
     else FMM_FARM(true, 2);

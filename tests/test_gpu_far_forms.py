@@ -78,3 +78,28 @@ def test_far_sum_forms_match_a_64_bit_sum(cuda, helm, pars, norder):
             err = np.linalg.norm(out - ref[:nrhs]) / np.linalg.norm(size[:nrhs])
             assert err < 30 * unit, (nrhs, prec, mode, err / unit)
     plan.close()
+
+
+# several groups of 16 in FP32 (split products), at the edges of the groups; the 10-point patches
+# leave a ragged last tile of 32 sources
+@pytest.mark.parametrize("helm,pars", [(False, (0.7, -1.3)), (True, (5.0, 5.0j, 1.0)), (True, (2.0 + 0.7j, 1.0, 1.0))])
+def test_far_sum_split_products_match_a_64_bit_sum(cuda, helm, pars):
+    import torch
+    from fmm3dbie_amd import geometry as G, layer, problem
+    g = G.get_sphere_npat(1.0, 2, (0, 0, 0), 3)
+    pars = np.array(pars)
+    P = problem.setup(g, 1e-6, helm, pars)
+    plan = layer.ApplyPlan(g, helm, pars, P["row_ptr"], P["col_ind"], P["iquad"],
+                           np.zeros(P["nquad"], complex if helm else float), P["novers"], P["ixyzso"], P["srcover"],
+                           P["whtsover"])
+    rng = np.random.default_rng(5)
+    N = len(g["srcvals"])
+    # (the size of a right-hand side is its own: each is checked by itself, from 1e-20 to 1e12)
+    S = (rng.standard_normal((64, N)) + 1j * rng.standard_normal((64, N))) * 10.0 ** (np.arange(64) / 2 - 20)[:, None]
+    ref, size, _ = _sum64(g, P, helm, pars, S)
+    for nrhs in (18, 32, 34, 48, 50, 64):
+        s = torch.as_tensor(S[:nrhs], device=cuda).to(torch.complex64).contiguous()
+        out = plan.apply(s, 32, 1).cpu().numpy()
+        err = np.linalg.norm(out - ref[:nrhs], axis=1) / np.linalg.norm(size[:nrhs], axis=1)
+        assert err.max() < 30 * 2.0 ** -24, (nrhs, err.max() * 2.0 ** 24)  # the bound above
+    plan.close()
