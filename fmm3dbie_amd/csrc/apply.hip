@@ -968,6 +968,7 @@ inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
   } while (0)
 
 ApplyPlan::~ApplyPlan() {
+  apply_plan_free_ws(this);
   for (void* p : owned)
     if (p) (void)hipFree(p);
 }
