@@ -1243,7 +1243,7 @@ static int64_t split_sources(int64_t nsrc, int tile, int64_t g, int64_t wg_targe
   int64_t nsplit = (wg_target + g - 1) / g;
   const int64_t need = (fill + g - 1) / g;
   nsplit = std::min(nsplit, std::max((nsrc + 255) / 256, need));
-  nsplit = std::max<int64_t>(1, std::min({nsplit, cap, ntiles}));
+  nsplit = std::max<int64_t>(1, std::min({nsplit, cap, ntiles, (int64_t)65535}));  // (grid y)
   *chunk = ((ntiles + nsplit - 1) / nsplit) * tile;
   return (nsrc + *chunk - 1) / *chunk;
 }
