@@ -233,9 +233,9 @@ def main():
         "kernels_note": "timed steps: fixed-rule and self kernels on a second stream beside the adaptive one; "
                         "kernels_ms_alone: each kernel alone, in order on one stream",
         "kernels_ms_alone": iso,
-        "roofline": {"bound": "valu", "pipe": "fp64 VALU (no MFMA in this kernel; MI355X FP64 vector peak = "
-                                              "FP64 matrix peak = 78.6 TFLOP/s)",
-                     "kernel": "k_adaptive", "achieved": achieved / 1e12, "peak": PEAK_FP64 / 1e12,
+        "roofline": {"bound": "valu", "pipe": "fp64 VALU and FP64 MFMA, which share their issue (MI355X FP64 vector "
+                                              "peak = FP64 matrix peak = 78.6 TFLOP/s)",
+                     "kernel": "k_adap_tile + k_adaptive", "achieved": achieved / 1e12, "peak": PEAK_FP64 / 1e12,
                      "unit": "TFLOP/s", "frac": achieved / PEAK_FP64, "traffic": None,
                      "alone": {"ms": iso["adaptive"], "achieved": fl / (iso["adaptive"] * 1e-3) / 1e12,
                                "frac": fl / (iso["adaptive"] * 1e-3) / PEAK_FP64}},
@@ -243,7 +243,7 @@ def main():
         "setup_gpu_near_s": t_setup_gpu,
         "setup_gpu_near_identical": setup_same,
     }
-    tr = measured_traffic("k_adaptive", wname) if name == "adaptive" else None
+    tr = measured_traffic("k_adap_tile + k_adaptive", wname) if name == "adaptive" else None
     if tr is not None:
         out["roofline"]["traffic"] = tr["traffic_bytes"]
         out["roofline"]["traffic_source"] = "profiles/ PMC summary (FETCH_SIZE x %.2f + WRITE_SIZE x %.2f)" % (
