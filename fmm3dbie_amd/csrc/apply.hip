@@ -7,7 +7,7 @@
 // with s_j = sigma_over_j * whtsover_j and K the combined kernel (alpha S + beta D).
 //
 // The FMM is replaced by an all-pairs sum, one density on the vector units (k_farsum) and
-// blocks of densities on the matrix cores (k_farsum_mfma).  Two modes:
+// blocks of densities on the matrix cores (k_farsum_mfma, k_farsum_split).  Two modes:
 //   ADDSUB : all sources, then the near patches' contributions subtracted (the reference's
 //            algebra);
 //   MASKED : sources of the target's near patches are skipped inside the sum
@@ -308,59 +308,35 @@ __global__ void __launch_bounds__(64) k_farsum(int ntarg, const T* __restrict__ 
   }
 }
 
-// Far sum of a group of 16 right-hand sides on the matrix cores: the group's potentials are
-// the complex product pot = K S of the target x source kernel matrix with the source x 16
+// Far sum of a group of 16 right-hand sides on the matrix cores, FP64: the group's potentials
+// are the complex product pot = K S of the target x source kernel matrix with the source x 16
 // strength matrix.  A wavefront takes MT tiles of 16 targets; in a step of 4 sources lane l
 // evaluates the pairs (target l % 16 of each tile, source l / 16) once on the vector units,
 // and the 16x16x4 product of the matrix cores multiplies the 16 x 4 kernel blocks by the 4 x
 // 16 strength blocks (lane l supplies source l / 16, right-hand side l % 16).  The complex
-// product takes three real ones (Gauss): a1 = Re K Re s, a2 = Im K Im s, a3 = (Re K + Im K)
-// (Re s + Im s), so Re pot = a1 - a2 and Im pot = a3 - a1 - a2.  Laplace: two, K being real.
+// product takes four real ones (Laplace: two, K being real).  Three (Gauss) would save 64 of
+// these cycles, but leave the imaginary part an error relative to the real one: 1.9e-14 of
+// itself for a real density at k = 0.01, where this form has 4.3e-16.
 // The workgroup stages FT sources at a time in LDS, geometry and strengths; MT tiles share
 // each LDS read.
-// Bound by issue: on this chip FP32 and FP64 matrix instructions do not overlap with vector
-// ones of the same SIMD (measured: the times of wavefronts of either kind add up), so that the
-// products' 3 x 32 cycles (FP32; 3 x 64 in FP64) and the kernel values of 64 pairs add.  One
-// complex kernel matrix takes half the products of separate charge and dipole matrices: 209
-// against 337 cycles per 64 pairs in FP32 (the 16-density apply of 86016 points 27.1 -> 16.7
-// ms), 466 in FP64 for 16 densities, where groups of 4 on the vector units took 400 each.
+// Bound by issue: on this chip FP64 matrix instructions do not overlap with vector ones of the
+// same SIMD (measured: the times of wavefronts of either kind add up), so that the products' 4
+// x 64 cycles and the kernel values of 64 pairs add.  The 16-density apply of 86016 points
+// (139206 sources): 40.7 ms, with three products 38.3.
 // Tiles of 128 sources, 1, 3 or 4 target tiles and an unrolled loop were all 1 to 15% slower.
-template <typename T>
-struct Mfma16;
-template <>
-struct Mfma16<float> {
-  typedef float V __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ V mul(float a, float b, V c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  // target of the tile in accumulator element r of lane l (its right-hand side is l % 16)
-  static __device__ __forceinline__ int row(int l, int r) { return 4 * (l >> 4) + r; }
-};
-template <>
-struct Mfma16<double> {
-  typedef double V __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ V mul(double a, double b, V c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int l, int r) { return (l >> 4) + 4 * r; }
-};
-
+typedef double dbl4 __attribute__((ext_vector_type(4)));
 constexpr int FT = 64;  // sources per LDS tile
 constexpr int FW = 4;   // wavefronts per workgroup
-template <typename T>
-constexpr int MT = 2;  // tiles of 16 targets per wavefront
-template <typename T, bool MASK, int KIND>
-__global__ void __launch_bounds__(64 * FW) k_farsum_mfma(int ntarg, const T* __restrict__ tx, const T* __restrict__ ty,
-                                                         const T* __restrict__ tz, int nsrc, const T* __restrict__ geo,
-                                                         const int64_t* __restrict__ ixyzso,
-                                                         const V2<T>* __restrict__ str,
-                                                         const int64_t* __restrict__ row_ptr,
-                                                         const int* __restrict__ near_sorted, FarPar<T> P, T thresh2,
-                                                         int chunk, int nrhs, V2<T>* __restrict__ part,
-                                                         int64_t ldpart) {
-  using M = Mfma16<T>;
-  using V = typename M::V;
-  constexpr int NT = MT<T>, G = GEO<T>;
+constexpr int MT = 2;   // tiles of 16 targets per wavefront
+template <bool MASK, int KIND>
+__global__ void __launch_bounds__(64 * FW)
+    k_farsum_mfma(int ntarg, const double* __restrict__ tx, const double* __restrict__ ty,
+                  const double* __restrict__ tz, int nsrc, const double* __restrict__ geo,
+                  const int64_t* __restrict__ ixyzso, const V2<double>* __restrict__ str,
+                  const int64_t* __restrict__ row_ptr, const int* __restrict__ near_sorted, FarPar<double> P,
+                  double thresh2, int chunk, int nrhs, V2<double>* __restrict__ part, int64_t ldpart) {
+  using T = double;
+  constexpr int NT = MT, G = GEO<T>;
   __shared__ __align__(16) T lgeo[FT * G];
   __shared__ __align__(16) V2<T> lstr[FT * MG];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -369,7 +345,7 @@ __global__ void __launch_bounds__(64 * FW) k_farsum_mfma(int ntarg, const T* __r
   const int t0 = (blockIdx.x * FW + wv) * (16 * NT);
   const int ks = lane >> 4;  // this lane's source within a step of 4
   T x[NT], y[NT], z[NT];
-  V a1[NT], a2[NT], a3[NT];
+  dbl4 re[NT], im[NT];
   const int jbeg = blockIdx.y * chunk;
   const int jend = jbeg + chunk < nsrc ? jbeg + chunk : nsrc;
   NearCursor nc[NT];
@@ -381,7 +357,7 @@ __global__ void __launch_bounds__(64 * FW) k_farsum_mfma(int ntarg, const T* __r
     x[t] = act[t] ? tx[i] : (T)0;
     y[t] = act[t] ? ty[i] : (T)0;
     z[t] = act[t] ? tz[i] : (T)0;
-    a1[t] = a2[t] = a3[t] = V{(T)0, (T)0, (T)0, (T)0};
+    re[t] = im[t] = dbl4{0.0, 0.0, 0.0, 0.0};
     nc[t] = NearCursor{near_sorted, ixyzso};
     if (MASK && act[t] && jbeg < jend) {
       nc[t].ptr = row_ptr[i] - 1;
@@ -404,7 +380,7 @@ __global__ void __launch_bounds__(64 * FW) k_farsum_mfma(int ntarg, const T* __r
       const T* g = lgeo + jl * G;
       const T gx = g[0], gy = g[1], gz = g[2], nx = g[3], ny = g[4], nz = g[5];
       const V2<T> sv = lstr[jl * MG + (lane & 15)];  // source k + l / 16, right-hand side l % 16
-      const T ss = sv.x + sv.y;
+      const T neg = -sv.y;
 #pragma unroll
       for (int t = 0; t < NT; t++) {
         const T dx = x[t] - gx, dy = y[t] - gy, dz = z[t] - gz;
@@ -418,12 +394,11 @@ __global__ void __launch_bounds__(64 * FW) k_farsum_mfma(int ntarg, const T* __r
         T gr, gi, c, s, q, vr, vi;
         pair_factors<T, KIND>(r2, rinv, d, P, gr, gi, c, s, q);
         pair_value<T, KIND>(gr, gi, c, s, q, vr, vi);
-        a1[t] = M::mul(vr, sv.x, a1[t]);
-        if constexpr (KIND == 0) {
-          a2[t] = M::mul(vr, sv.y, a2[t]);
-        } else {
-          a2[t] = M::mul(vi, sv.y, a2[t]);
-          a3[t] = M::mul(vr + vi, ss, a3[t]);
+        re[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(vr, sv.x, re[t], 0, 0, 0);
+        im[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(vr, sv.y, im[t], 0, 0, 0);
+        if constexpr (KIND != 0) {
+          re[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(vi, neg, re[t], 0, 0, 0);
+          im[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(vi, sv.x, im[t], 0, 0, 0);
         }
       }
     };
@@ -445,46 +420,44 @@ __global__ void __launch_bounds__(64 * FW) k_farsum_mfma(int ntarg, const T* __r
       for (int k = 0; k < cnt; k += 4) step(k, std::false_type{});
     }
   }
+  // accumulator element e of lane l: target l / 16 + 4 e of the tile, right-hand side l % 16
   const int r = (int)rg * MG + (lane & 15);
   if (r < nrhs) {
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        const int it = t0 + 16 * t + M::row(lane, e);
-        if (it < ntarg) {
-          V2<T> v;
-          if constexpr (KIND == 0) v = {a1[t][e], a2[t][e]};
-          else v = {a1[t][e] - a2[t][e], a3[t][e] - a1[t][e] - a2[t][e]};
-          part[(int64_t)blockIdx.y * ldpart + (int64_t)r * ntarg + it] = v;
-        }
+        const int it = t0 + 16 * t + ks + 4 * e;
+        if (it < ntarg) part[(int64_t)blockIdx.y * ldpart + (int64_t)r * ntarg + it] = {re[t][e], im[t][e]};
       }
   }
 }
 
-// Far sum of NG = 2, 3 or 4 groups of 16 right-hand sides, FP32 (grid z: NG groups each).  The kernel
-// values are computed once for all groups, and the products run in bfloat16, where the matrix
-// cores have sixteen times their FP32 rate, exact products and FP32 sums: each value is split
-// into three bfloat16 terms (hi + mid + lo, rounded to nearest, is the FP32 value to its last bit),
-// and six products of terms take the place of one (those left out are below 2^-26 of it).
+// Far sum of all NG groups of 16 right-hand sides of a block, FP32.  The kernel values are
+// computed once for all groups, and the products run in bfloat16, where the matrix cores have
+// sixteen times their FP32 rate, exact products and FP32 sums: each value is split into three
+// bfloat16 terms (hi + mid + lo, rounded to nearest, is the FP32 value to its last bit), and six
+// products of terms take the place of one (those left out are below 2^-26 of it).
 // A wavefront takes MT tiles of 16 targets; in a tile of ST = 32 sources lane l evaluates the pairs
 // (target l % 16, sources 8 (l / 16) ..) on the vector units, which are the operand of the 16x16x32
 // products as they stand.  The workgroup stages the sources' geometry and the split strengths in
 // LDS, in the order in which the lanes read them; the next tile's are loaded while one is summed.
-// Bound by issue: per 64 pairs and group 36 x 4.5 cycles of products, 40 instructions of kernel
+// The complex product takes four real ones, as in k_farsum_mfma, and a tile's products are
+// summed by themselves before they are added to the potentials: the matrix cores round each sum
+// of a chain downwards, which over all sources would add up (error of the 64-density apply below
+// against the FP64 one 3.1e-6; 3.8e-7 in this way).  Re K Re s and Im K Im s have a sum each,
+// which costs less than to negate an operand.
+// Bound by issue: per 64 pairs and group 48 x 4.5 cycles of products, 35 instructions of kernel
 // values and splits per pair, and the staging, which MT = 2 tiles share.  The apply of 86016
-// points (139206 sources) in FP32 products, a group at a time, against this: 32 densities 32.7 to
-// 21.9 ms, 48 49.0 to 29.0, 64 65.4 to 34.3, its error against the FP64 apply 1.7e-6 to 1.3e-6, 2.2e-6
-// to 1.7e-6 and 2.4e-6 to 1.9e-6.  One group keeps the FP32 products (16.5 against 17.9 ms: the
-// splits cost what the products save).
+// points (139206 sources): 16 densities 15.1 ms, 32 21.8, 48 28.9, 64 33.0; in FP32 products, a group
+// at a time, 19.3 ms for each 16.
 typedef float flt2 __attribute__((ext_vector_type(2)));
 typedef float flt4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
-constexpr int ST = 32;        // sources per tile
-constexpr int SPLIT_MAX = 4;  // groups per wavefront
-struct Split8 {               // the terms of eight values
+constexpr int ST = 32;  // sources per tile
+struct Split8 {         // the terms of eight values
   union {
     bf8 v;
     bf2 p[4];
@@ -506,14 +479,12 @@ __global__ void __launch_bounds__(64 * FW, 2)
                    const int* __restrict__ near_sorted, FarPar<float> P, int chunk, int nrhs,
                    V2<float>* __restrict__ part, int64_t ldpart) {
   using T = float;
-  constexpr int NM = KIND == 0 ? 1 : 3;  // kernel matrices: Re K, Im K, Re K + Im K
-  constexpr int NB = KIND == 0 ? 2 : 3;  // strength matrices: Re s, Im s, Re s + Im s
-  constexpr int SI = NG == 2 ? 4 : 8;    // sources that a thread stages, of one right-hand side
-  constexpr int NT = MT<T>;
+  constexpr int NM = KIND == 0 ? 1 : 2;  // kernel matrices: Re K, Im K
+  constexpr int SI = NG == 1 ? 2 : (NG == 2 ? 4 : 8);  // sources that a thread stages, of one right-hand side
+  constexpr int NT = MT;
   __shared__ __align__(16) T lgeo[ST * 8];
-  __shared__ __align__(16) bf8 lstr[NG][NB][3][64];
+  __shared__ __align__(16) bf8 lstr[NG][2][3][64];  // Re s, Im s
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int g0 = blockIdx.z * NG, ngrp = (nrhs + MG - 1) / MG;
   const int t0 = (blockIdx.x * FW + wv) * (16 * NT);
   const int ks = lane >> 4;  // this lane's sources: 8 ks .. 8 ks + 7 of a tile
   const int jbeg = blockIdx.y * chunk;
@@ -537,13 +508,13 @@ __global__ void __launch_bounds__(64 * FW, 2)
   }
   // this thread's part of a tile: right-hand side sr of group sg, sources sj .. sj + SI - 1
   const int sr = threadIdx.x & 15, sj = SI * ((threadIdx.x >> 4) % (ST / SI)), sg = (threadIdx.x >> 4) / (ST / SI);
-  const bool stager = sg < NG, live = stager && g0 + sg < ngrp;
-  const V2<T>* sp = str + (int64_t)(live ? g0 + sg : 0) * nsrc * MG + sr;
+  const bool stager = sg < NG;
+  const V2<T>* sp = str + (int64_t)(stager ? sg : 0) * nsrc * MG + sr;
   V2<T> next[SI];
   T nextg;  // and one value of the geometry
   static_assert(ST * 8 == 64 * FW, "");
   // (loads without a condition, in flight together while a tile is summed; sources past the chunk
-  // and groups past the last are zeroed below)
+  // are zeroed below)
   auto load = [&](int base) {
 #pragma unroll
     for (int u = 0; u < SI; u++) {
@@ -557,16 +528,16 @@ __global__ void __launch_bounds__(64 * FW, 2)
     lgeo[threadIdx.x] = base + (int)(threadIdx.x / 8) < jend ? nextg : (T)0;
 #pragma unroll
     for (int u = 0; u < SI; u++)
-      if (!live || base + sj + u >= jend) next[u] = V2<T>{0.0f, 0.0f};
+      if (base + sj + u >= jend) next[u] = V2<T>{0.0f, 0.0f};
     if (!stager) return;
     bf2* o = reinterpret_cast<bf2*>(&lstr[sg][0][0][sj / 8 * 16 + sr]) + (sj % 8) / 2;
 #pragma unroll
-    for (int m = 0; m < NB; m++) {
+    for (int m = 0; m < 2; m++) {
       bf2 v[3][SI / 2];
 #pragma unroll
       for (int u = 0; u < SI; u += 2) {
-        T a = m == 0 ? next[u].x : (m == 1 ? next[u].y : next[u].x + next[u].y);
-        T b = m == 0 ? next[u + 1].x : (m == 1 ? next[u + 1].y : next[u + 1].x + next[u + 1].y);
+        T a = m == 0 ? next[u].x : next[u].y;
+        T b = m == 0 ? next[u + 1].x : next[u + 1].y;
 #pragma unroll
         for (int k = 0; k < 3; k++) v[k][u / 2] = next_term(a, b);
       }
@@ -574,17 +545,16 @@ __global__ void __launch_bounds__(64 * FW, 2)
       for (int k = 0; k < 3; k++) {
         bf2* q = o + (m * 3 + k) * 64 * 4;
         if constexpr (SI == 8) *reinterpret_cast<bf8*>(q) = *reinterpret_cast<const bf8*>(v[k]);
-        else *reinterpret_cast<bf4*>(q) = *reinterpret_cast<const bf4*>(v[k]);
+        else if constexpr (SI == 4) *reinterpret_cast<bf4*>(q) = *reinterpret_cast<const bf4*>(v[k]);
+        else *q = v[k][0];
       }
     }
   };
-  flt4 acc[NT][NG][NB];
+  flt4 re[NT][NG], im[NT][NG];
 #pragma unroll
   for (int t = 0; t < NT; t++)
 #pragma unroll
-    for (int g = 0; g < NG; g++)
-#pragma unroll
-      for (int m = 0; m < NB; m++) acc[t][g][m] = flt4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int g = 0; g < NG; g++) re[t][g] = im[t][g] = flt4{0.0f, 0.0f, 0.0f, 0.0f};
   if (jbeg < jend) load(jbeg);
 #pragma unroll 1
   for (int base = jbeg; base < jend; base += ST) {
@@ -611,7 +581,7 @@ __global__ void __launch_bounds__(64 * FW, 2)
           for (int e = 0; e < 6; e++) gg[v][e] = lgeo[(8 * ks + u + v) * 8 + e];
 #pragma unroll
         for (int t = 0; t < NT; t++) {
-          T vr[2], vi[2], vs[2];
+          T vr[2], vi[2];
 #pragma unroll
           for (int v = 0; v < 2; v++) {
             const T* g = gg[v];
@@ -627,63 +597,56 @@ __global__ void __launch_bounds__(64 * FW, 2)
             T gr, gi, c, s, q;
             pair_factors<T, KIND>(r2, rinv, d, P, gr, gi, c, s, q);
             pair_value<T, KIND>(gr, gi, c, s, q, vr[v], vi[v]);
-            vs[v] = vr[v] + vi[v];
           }
 #pragma unroll
           for (int k = 0; k < 3; k++) {
             A[t][0].t[k].p[u / 2] = next_term(vr[0], vr[1]);
-            if constexpr (NM == 3) {
-              A[t][NM - 2].t[k].p[u / 2] = next_term(vi[0], vi[1]);
-              A[t][NM - 1].t[k].p[u / 2] = next_term(vs[0], vs[1]);
-            }
+            if constexpr (NM == 2) A[t][1].t[k].p[u / 2] = next_term(vi[0], vi[1]);
           }
         }
       }
     };
     if (__all(mine)) eval(std::true_type{});
     else eval(std::false_type{});
-    // products, GB groups at a time (a register each more at 4 groups would halve the occupancy)
-    constexpr int GB = NG == 4 ? 1 : 2;
 #pragma unroll
-    for (int m = 0; m < NB; m++)
+    for (int g = 0; g < NG; g++) {
+      flt4 rr[NT], ii[NT], mix[NT];  // sums of Re K Re s, Im K Im s, Re K Im s + Im K Re s
 #pragma unroll
-      for (int h = 0; h < NG; h += GB) {
-        bf8 b[GB][3];
+      for (int t = 0; t < NT; t++) rr[t] = ii[t] = mix[t] = flt4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int g = 0; g < GB && h + g < NG; g++)
+      for (int m = 0; m < 2; m++) {
+        bf8 b[3];
 #pragma unroll
-          for (int k = 0; k < 3; k++) b[g][k] = lstr[h + g][m][k][lane];
-        auto mul = [&](int ka, int kb) {
+        for (int k = 0; k < 3; k++) b[k] = lstr[g][m][k][lane];
+        auto mul = [&](int km, flt4(&sum)[NT]) {
+          constexpr int ka[6] = {2, 0, 1, 1, 0, 0}, kb[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
-          for (int g = 0; g < GB && h + g < NG; g++)
+          for (int e = 0; e < 6; e++)
 #pragma unroll
             for (int t = 0; t < NT; t++)
-              acc[t][h + g][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[t][NM == 1 ? 0 : m].t[ka].v, b[g][kb],
-                                                                        acc[t][h + g][m], 0, 0, 0);
+              sum[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[t][km].t[ka[e]].v, b[kb[e]], sum[t], 0, 0, 0);
         };
-        mul(2, 0);
-        mul(0, 2);
-        mul(1, 1);
-        mul(1, 0);
-        mul(0, 1);
-        mul(0, 0);
+        mul(0, m == 0 ? rr : mix);
+        if constexpr (NM == 2) mul(1, m == 0 ? mix : ii);
       }
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        re[t][g] += rr[t] - ii[t];
+        im[t][g] += mix[t];
+      }
+    }
   }
+  // accumulator element e of lane l: target 4 (l / 16) + e of the tile, right-hand side l % 16
 #pragma unroll
   for (int t = 0; t < NT; t++)
 #pragma unroll
     for (int g = 0; g < NG; g++) {
-      const int r = (g0 + g) * MG + (lane & 15);
+      const int r = g * MG + (lane & 15);
       if (r >= nrhs) continue;
-      const flt4 a1 = acc[t][g][0], a2 = acc[t][g][1], a3 = acc[t][g][NB - 1];
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        const int it = t0 + 16 * t + Mfma16<T>::row(lane, e);
-        if (it >= ntarg) continue;
-        V2<T> v;
-        if constexpr (KIND == 0) v = {a1[e], a2[e]};
-        else v = {a1[e] - a2[e], a3[e] - a1[e] - a2[e]};
-        part[(int64_t)blockIdx.y * ldpart + (int64_t)r * ntarg + it] = v;
+        const int it = t0 + 16 * t + 4 * ks + e;
+        if (it < ntarg) part[(int64_t)blockIdx.y * ldpart + (int64_t)r * ntarg + it] = {re[t][g][e], im[t][g][e]};
       }
     }
 }
@@ -1279,55 +1242,65 @@ static int launch_far(ApplyPlan* P, bool mask, int64_t wg_target, const V2<T>* s
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// The matrix-core far sum: groups of 16 right-hand sides, the last one padded with zeros.
-// FP32 blocks of several groups take the split products, up to SPLIT_MAX groups at a time.
-template <typename T>
-static int launch_far_mfma(ApplyPlan* P, bool mask, int64_t wg_target, const V2<T>* str, int nrhs, V2<T>* part,
-                           int64_t part_cap, int64_t* nsplit_out, hipStream_t s) {
-  const T* const* trg = targets_of<T>(P);
-  const unsigned g = nblk(P->ntarg, 16 * FW * MT<T>);
+// The matrix-core far sums: groups of 16 right-hand sides, the last one padded with zeros.
+// FP64: a group per workgroup (grid z).
+static int launch_far_mfma(ApplyPlan* P, bool mask, int64_t wg_target, const V2<double>* str, int nrhs,
+                           V2<double>* part, int64_t part_cap, int64_t* nsplit_out, hipStream_t s) {
+  const double* const* trg = targets_of<double>(P);
+  const unsigned g = nblk(P->ntarg, 16 * FW * MT);
   const int ngrp = (nrhs + MG - 1) / MG;
-  const int ng = sizeof(T) == 4 && ngrp <= SPLIT_MAX ? ngrp : 1;
   int64_t chunk;
-  const int64_t nsplit = split_sources(P->nptso, FT, (int64_t)g * (ngrp / ng), wg_target, FAR_FILL / FW,
+  const int64_t nsplit = split_sources(P->nptso, FT, (int64_t)g * ngrp, wg_target, FAR_FILL / FW,
                                        part_cap / ((int64_t)nrhs * P->ntarg), &chunk);
-  const dim3 grid(g, (unsigned)nsplit, (unsigned)(ngrp / ng));
-  const T th2 = (T)(P->thresh * P->thresh);
-  const int kind = far_kind<T>(P);
-  if constexpr (sizeof(T) == 4) {
+  const dim3 grid(g, (unsigned)nsplit, (unsigned)ngrp);
+  const int kind = far_kind<double>(P);
+#define FMM_FARM(MK, KD)                                                                                         \
+  k_farsum_mfma<MK, KD><<<grid, 64 * FW, 0, s>>>((int)P->ntarg, trg[0], trg[1], trg[2], (int)P->nptso, P->geo64, \
+                                                 P->ixyzso, str, P->row_ptr, P->near_sorted, far_par<double>(P), \
+                                                 P->thresh * P->thresh, (int)chunk, nrhs, part,                  \
+                                                 (int64_t)nrhs * P->ntarg)
+  if (mask) {
+    if (kind == 0) FMM_FARM(true, 0);
+    else if (kind == 1) FMM_FARM(true, 1);
+    else FMM_FARM(true, 2);
+  } else {
+    if (kind == 0) FMM_FARM(false, 0);
+    else if (kind == 1) FMM_FARM(false, 1);
+    else FMM_FARM(false, 2);
+  }
+#undef FMM_FARM
+  *nsplit_out = nsplit;
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+// FP32: all groups (at most four) in each workgroup.
+static int launch_far_split(ApplyPlan* P, int64_t wg_target, const V2<float>* str, int nrhs, V2<float>* part,
+                            int64_t part_cap, int64_t* nsplit_out, hipStream_t s) {
+  const float* const* trg = targets_of<float>(P);
+  const unsigned g = nblk(P->ntarg, 16 * FW * MT);
+  const int ng = (nrhs + MG - 1) / MG;
+  int64_t chunk;
+  const int64_t nsplit = split_sources(P->nptso, FT, g, wg_target, FAR_FILL / FW,
+                                       part_cap / ((int64_t)nrhs * P->ntarg), &chunk);
+  const dim3 grid(g, (unsigned)nsplit);
+  const int kind = far_kind<float>(P);
 #define FMM_FARS(KD, NG)                                                                                          \
-  k_farsum_split<KD, NG><<<grid, 64 * FW, 0, s>>>((int)P->ntarg, trg[0], trg[1], trg[2], (int)P->nptso,           \
-                                                  sources_of<T>(P), P->ixyzso, str, P->row_ptr, P->near_sorted,   \
-                                                  far_par<T>(P), (int)chunk, nrhs, part, (int64_t)nrhs * P->ntarg)
+  k_farsum_split<KD, NG><<<grid, 64 * FW, 0, s>>>((int)P->ntarg, trg[0], trg[1], trg[2], (int)P->nptso, P->geo32, \
+                                                  P->ixyzso, str, P->row_ptr, P->near_sorted, far_par<float>(P),  \
+                                                  (int)chunk, nrhs, part, (int64_t)nrhs * P->ntarg)
 #define FMM_FARK(NG)                     \
   do {                                   \
     if (kind == 0) FMM_FARS(0, NG);      \
     else if (kind == 1) FMM_FARS(1, NG); \
     else FMM_FARS(2, NG);                \
   } while (0)
-    if (ng == 2) FMM_FARK(2);
-    else if (ng == 3) FMM_FARK(3);
-    else if (ng == 4) FMM_FARK(4);
+  if (ng == 1) FMM_FARK(1);
+  else if (ng == 2) FMM_FARK(2);
+  else if (ng == 3) FMM_FARK(3);
+  else if (ng == 4) FMM_FARK(4);
+  else return -6;
 #undef FMM_FARK
 #undef FMM_FARS
-  }
-#define FMM_FARM(MK, KD)                                                                                       \
-  k_farsum_mfma<T, MK, KD><<<grid, 64 * FW, 0, s>>>((int)P->ntarg, trg[0], trg[1], trg[2], (int)P->nptso,      \
-                                                   sources_of<T>(P), P->ixyzso, str, P->row_ptr,               \
-                                                   P->near_sorted, far_par<T>(P), th2, (int)chunk, nrhs, part, \
-                                                   (int64_t)nrhs * P->ntarg)
-  if (ng > 1) {
-    // launched above
-  } else if (mask || sizeof(T) == 4) {
-    if (kind == 0) FMM_FARM(true, 0);
-    else if (kind == 1) FMM_FARM(true, 1);
-    else FMM_FARM(true, 2);
-  } else if constexpr (sizeof(T) == 8) {
-    if (kind == 0) FMM_FARM(false, 0);
-    else if (kind == 1) FMM_FARM(false, 1);
-    else FMM_FARM(false, 2);
-  }
-#undef FMM_FARM
   *nsplit_out = nsplit;
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
@@ -1359,7 +1332,9 @@ static int dispatch_far(ApplyPlan* P, bool mask, int grp, int64_t wg, const V2<T
     case 2: return launch_far<T, 2>(P, mask, wg, str, nrhs, part, part_cap, nsplit, s);
     case 4: return launch_far<T, 4>(P, mask, wg, str, nrhs, part, part_cap, nsplit, s);
     case 8: return launch_far<T, 8>(P, mask, wg, str, nrhs, part, part_cap, nsplit, s);
-    case MG: return launch_far_mfma<T>(P, mask, wg, str, nrhs, part, part_cap, nsplit, s);
+    case MG:
+      if constexpr (sizeof(T) == 8) return launch_far_mfma(P, mask, wg, str, nrhs, part, part_cap, nsplit, s);
+      else return launch_far_split(P, wg, str, nrhs, part, part_cap, nsplit, s);
     default: return -6;
   }
 }

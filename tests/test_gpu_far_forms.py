@@ -8,23 +8,25 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-def _sum64(g, P, helm, pars, sig):
-    """All oversampled sources except those of near patches (near weights zero), (nrhs, npts)
-    in 64 bits (the add/subtract form is the same sum), and the sums of |K| |s| over those
-    sources and over all sources, which bound the rounding of either form."""
-    import torch
+def _over(g, P, sig):
+    """sigma_over * w at the oversampled nodes, (nrhs, nptso)."""
     from fmm3dbie_amd import basis
     no = int(g["norders"][0])
     p = len(basis.rv_nodes(no)[1])
     um = basis.rv_umat(no)
-    nrhs = len(sig)
-    over = np.zeros((nrhs, len(P["whtsover"])), complex)
+    over = np.zeros((len(sig), len(P["whtsover"])), complex)
     for ip, nv in enumerate(P["novers"]):
         uv, _ = basis.rv_nodes(int(nv))
         im = np.stack([basis.koorn_pols(u, v, no) for u, v in uv]) @ um
         a, b = P["ixyzso"][ip] - 1, P["ixyzso"][ip + 1] - 1
         over[:, a:b] = sig[:, ip * p:(ip + 1) * p] @ im.T
-    over *= P["whtsover"]
+    return over * P["whtsover"]
+
+
+def _kernel(g, P, helm, pars):
+    """Kernel matrix (npts, nptso) over all oversampled sources, and with those of each
+    target's near patches zeroed."""
+    import torch
     t = torch.as_tensor
     d = t(g["srcvals"][:, None, :3] - P["srcover"][None, :, :3])
     r = d.square().sum(-1).sqrt()
@@ -37,9 +39,18 @@ def _sum64(g, P, helm, pars, sig):
     near = np.zeros((len(r), len(P["novers"])), bool)
     rows = np.repeat(np.arange(len(r)), np.diff(P["row_ptr"]))
     near[rows, P["col_ind"] - 1] = True
-    far = torch.where(t(near[:, patch]), 0, ker)
-    size = [(t(over).abs() @ k.abs().T).numpy() for k in (far, ker)]
-    return (t(over) @ far.T).numpy(), size[0], size[1]
+    return ker, torch.where(t(near[:, patch]), 0, ker)
+
+
+def _sum64(g, P, helm, pars, sig):
+    """All oversampled sources except those of near patches (near weights zero), (nrhs, npts)
+    in 64 bits (the add/subtract form is the same sum), and the sums of |K| |s| over those
+    sources and over all sources, which bound the rounding of either form."""
+    import torch
+    over = torch.as_tensor(_over(g, P, sig))
+    ker, far = _kernel(g, P, helm, pars)
+    size = [(over.abs() @ k.abs().T).numpy() for k in (far, ker)]
+    return (over @ far.T).numpy(), size[0], size[1]
 
 
 # helm, (k, alpha, beta); the sphere's points are ragged: 27 targets of the last wavefront at
@@ -102,4 +113,35 @@ def test_far_sum_split_products_match_a_64_bit_sum(cuda, helm, pars):
         out = plan.apply(s, 32, 1).cpu().numpy()
         err = np.linalg.norm(out - ref[:nrhs], axis=1) / np.linalg.norm(size[:nrhs], axis=1)
         assert err.max() < 30 * 2.0 ** -24, (nrhs, err.max() * 2.0 ** 24)  # the bound above
+    plan.close()
+
+
+# The imaginary part of the single layer of a real density is k times the real part's size: the error
+# of each part is held to the sum of its own products, which a block's columns have to keep as a
+# density on its own does (the complex product is not to be formed from three real ones)
+@pytest.mark.parametrize("zk", [0.01, 1.0])
+def test_block_of_real_densities_keeps_each_part(cuda, zk):
+    import torch
+    from fmm3dbie_amd import geometry as G, layer, problem
+    g = G.get_sphere_npat(1.0, 1, (0, 0, 0), 4)
+    pars = np.array([zk, 1.0, 0.0])
+    P = problem.setup(g, 1e-6, True, pars)
+    plan = layer.ApplyPlan(g, True, pars, P["row_ptr"], P["col_ind"], P["iquad"], np.zeros(P["nquad"], complex),
+                           P["novers"], P["ixyzso"], P["srcover"], P["whtsover"])
+    rng = np.random.default_rng(9)
+    S = rng.standard_normal((64, len(g["srcvals"]))) + 0j
+    over = torch.as_tensor(_over(g, P, S).real)
+    ker, far = _kernel(g, P, True, pars)
+    for nrhs in (1, 3, 8, 9, 15, 16, 17, 33, 48, 64):
+        s = torch.as_tensor(S[:nrhs], device=cuda)
+        s = s[0] if nrhs == 1 else s
+        for prec, mode, unit, k in ((64, 1, 2.0 ** -53, far), (64, 0, 2.0 ** -53, ker), (32, 1, 2.0 ** -24, far)):
+            sp = s if prec == 64 else s.to(torch.complex64)
+            out = torch.as_tensor(np.atleast_2d(plan.apply(sp.contiguous(), prec, mode).cpu().numpy()))
+            for part in ("real", "imag"):
+                ref = over[:nrhs] @ getattr(far, part).T
+                size = over[:nrhs].abs() @ getattr(k, part).abs().T
+                err = float((getattr(out, part) - ref).norm() / size.norm())
+                # 30 roundings, the bound above
+                assert err < 30 * unit, (nrhs, prec, mode, part, err / unit)
     plan.close()
