@@ -1305,8 +1305,15 @@ static int launch_far_split(ApplyPlan* P, int64_t wg_target, const V2<float>* st
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// Right-hand sides per far-sum group: tuned, or by default the smallest of 1, 2, 4, 8 that
-// holds the block, and 16 (matrix cores) beyond; a last group is padded with zeros.  Measured
+// Right-hand sides per far-sum group by default: the smallest of 1, 2, 4, 8 that holds the
+// block, and 16 (matrix cores) beyond.
+static int default_group(int nrhs) {
+  int grp = 1;
+  while (grp < nrhs && grp < MG) grp *= 2;
+  return grp;
+}
+
+// Right-hand sides per far-sum group, tuned or default; a last group is padded with zeros.  Measured
 // in cycles of a SIMD per 64 pairs (43008 x 70000 pairs, Helmholtz): FP64 262 / 280 / 316 for
 // 1, 2 and 4 densities and 466 for 16; FP32 98 / 110 / 140 and 217.  str_cap: strengths
 // (complex values) that fit the buffer of the call; a padded block that does not falls back
@@ -1314,9 +1321,7 @@ static int launch_far_split(ApplyPlan* P, int64_t wg_target, const V2<float>* st
 static int far_group(const ApplyPlan* P, int nrhs, int prec, int64_t str_cap, int64_t* wg) {
   const auto it = P->tuned.find(prec * 1000 + nrhs);
   *wg = it != P->tuned.end() ? it->second.second : P->far_wg_target;
-  int grp = it != P->tuned.end() ? it->second.first : 1;
-  if (it == P->tuned.end())
-    while (grp < nrhs && grp < MG) grp *= 2;
+  int grp = it != P->tuned.end() ? it->second.first : default_group(nrhs);
   while (P->nptso * padded_rhs(nrhs, grp) > str_cap || grp > MG) {
     grp /= 2;
     while (nrhs % grp != 0) grp /= 2;
@@ -1552,10 +1557,11 @@ int apply_plan_run_noalloc(ApplyPlan* P, int prec, int mode, const void* sigma, 
 }
 
 // Autotuner of the far-sum launch shape for (prec, nrhs): every right-hand-side group size
-// that divides nrhs (1..16; in FP64 blocks of 16 and more leave out the group of one, 16 times
-// the kernel values of the matrix cores) and workgroup targets of 4096, 8192, 16384, 32768
-// are timed (one warm-up launch, then one launch each) on unit densities; the fastest is
-// kept in the plan and used by every later apply with the same (prec, nrhs).
+// from 1 to the default one, which pads the last group (FP64 blocks of 16 and more leave out
+// the group of one, 16 times the kernel values of the matrix cores), and workgroup targets of
+// 4096, 8192, 16384, 32768 are timed (one warm-up launch, then one launch each) on unit
+// densities; the fastest is kept in the plan and used by every later apply with the same
+// (prec, nrhs).
 int apply_plan_tune(ApplyPlan* P, int prec, int nrhs, hipStream_t s, double* report, int nreport) {
   if (nrhs < 1 || nrhs > 64 || (prec != 32 && prec != 64)) return -6;
   if (ensure_ws(P, nrhs) != 0) return -2;
@@ -1580,10 +1586,10 @@ int apply_plan_tune(ApplyPlan* P, int prec, int nrhs, hipStream_t s, double* rep
   int bg = 1, nrep = 0;
   int64_t bw = P->far_wg_target;
   // one warm-up launch, then one timed launch per shape
-  int rc = far(nrhs % MG == 0 ? MG : 1, P->far_wg_target);
+  int rc = far(default_group(nrhs), P->far_wg_target);
   if (rc) return rc;
   for (int gsz : groups) {
-    if (nrhs % gsz != 0 || (prec == 64 && gsz == 1 && nrhs % MG == 0)) continue;
+    if (gsz > default_group(nrhs) || (prec == 64 && gsz == 1 && nrhs >= MG)) continue;
     for (int64_t wg : wgs) {
       ACHK(hipEventRecord(e0, s));
       rc = far(gsz, wg);

@@ -345,8 +345,8 @@ size_t fmm3dbie_apply_scratch_bytes(void);
 int fmm3dbie_apply_plan_info(void *plan, int64_t *out4);
 void fmm3dbie_apply_plan_destroy(void *plan);
 /* Autotuner of the all-pairs far-sum launch (no reference counterpart): times every
- * right-hand-side group size dividing nrhs (1..16; FP64 blocks of a multiple of 16: 2..16)
- * and four workgroup targets (4096..32768), keeps the fastest for later applies with the same (prec, nrhs); report gets
+ * right-hand-side group size (1, 2, 4, 8, 16) up to the smallest that holds the block (a last
+ * group is padded; FP64 blocks of 16 and more: from 2) and four workgroup targets (4096..32768), keeps the fastest for later applies with the same (prec, nrhs); report gets
  * (group, workgroup target, ms) triples (nreport doubles).  Returns the number timed. */
 int fmm3dbie_apply_plan_tune(void *plan, int prec, int nrhs, void *stream, double *report, int nreport);
 

@@ -34,7 +34,7 @@ def test_batched_apply_and_tuning(cuda):
     for mode in (0, 1):
         assert _rel(plan.apply(dS, 64, mode).cpu().numpy(), single) < 1e-12
     rep64 = plan.tune(64, 64)
-    assert len(rep64) == 4 * 4  # groups 1, 2, 4, 8 x four workgroup targets
+    assert len(rep64) == 4 * 4  # groups 2, 4, 8, 16 x four workgroup targets
     assert _rel(plan.apply(dS, 64, 1).cpu().numpy(), single) < 1e-12
     S32 = dS.to(torch.complex64)
     before = plan.apply(S32, 32, 1).cpu().numpy()
@@ -44,8 +44,30 @@ def test_batched_apply_and_tuning(cuda):
     for r in range(64):
         assert _rel(after[r], single[r]) < 1e-5
         assert _rel(before[r], single[r]) < 1e-5
-    # odd batch sizes use the group sizes that divide them
+    # odd batch sizes are padded to a group size
     assert _rel(plan.apply(dS[:3], 64, 1).cpu().numpy(), single[:3]) < 1e-12
+    plan.close()
+
+
+def test_tuning_times_the_default_group(cuda):
+    """Blocks that are not a power of two: the untuned plan pads them to one group of 4, 8 or
+    16, which has to be among the shapes that the tuner times (it keeps the fastest of them);
+    results stay those of single densities."""
+    import torch
+    g, pars, P, plan = _sphere(5.0)
+    N = len(g["srcvals"])
+    rng = np.random.default_rng(6)
+    dS = torch.as_tensor(rng.standard_normal((33, N)) + 1j * rng.standard_normal((33, N)), device=cuda)
+    single = np.stack([plan.apply(dS[r], 64, 0).cpu().numpy() for r in range(33)])
+    for nrhs, group in ((2, 2), (3, 4), (5, 8), (7, 8), (9, 16), (17, 16), (33, 16)):
+        for prec in (64, 32):
+            rep = plan.tune(prec, nrhs)
+            first = 2 if prec == 64 and nrhs >= 16 else 1
+            want = [v for v in (1, 2, 4, 8, 16) if first <= v <= group]
+            assert sorted({r[0] for r in rep}) == want and len(rep) == 4 * len(want), (nrhs, prec, rep)
+            s = dS[:nrhs].contiguous()
+            out = plan.apply(s if prec == 64 else s.to(torch.complex64), prec, 1).cpu().numpy()
+            assert _rel(out, single[:nrhs]) < (1e-12 if prec == 64 else 1e-5), (nrhs, prec)
     plan.close()
 
 
