@@ -1321,6 +1321,9 @@ __global__ void __launch_bounds__(256) k_adap_tile(AdapTiles A, AdapRules R, int
         if (LEV == 0) A.list1[b0 + at] = make_int2(e, slot);
         else if (!last) A.list2[4 * (size_t)b0 + (size_t)y * np + at] = make_int4(e, slot, ref, 0);
         else if (at < A.cap) A.items[at] = make_int4(e, slot, ref, t + 65536 * cls);
+        // (the two counters are not one step: once the pool is empty, places of pairs without a
+        // slot may be taken before that of a pair with one)
+        else if (slot >= 0) adap_send_back(A, e, false);
       }
     } else if (valid && LEV > 0) {
       for (int i = sub; i < VL; i += 16) A.slots[(size_t)ref * VL + i] = ssum(i);
