@@ -627,15 +627,14 @@ void rsc_to_csc_(const int64_t* ncol, const int64_t* nrow, const int64_t* nnz, c
 // kpar6 = (k re, k im, alpha re, alpha im, beta re, beta im); Laplace: helm=0, k ignored.
 // stats (optional, 12 doubles): nself, nadap, nfixed, overflow, nf, kq, ms_prep, ms_fixed,
 // ms_adap, ms_self, 0, 0.
-int fmm3dbie_nearquad_dev(int helm, int norder, int norder_branch, int64_t npatches, const int64_t* ixyzs,
-                          const double* srccoefs, const double* srcvals, int64_t ndtarg, int64_t ntarg,
-                          const double* targs, const int64_t* ipatch_id, const double* uvs_targ, double eps,
-                          const double* kpar6, int64_t nnz, const int64_t* row_ptr, const int64_t* col_ind,
-                          const int64_t* iquad, double rfac0, double* wnear, int self_nr, int self_nt,
-                          double self_tau_panel,
-                          void* stream, double* stats, int* nref_host, int* class_host, const float* mlp_params,
-                          float* feat_out, int* pred_host, const int* route_lmax, int* lev_host,
-                          int* unc_host) {
+int fmm3dbie_nearquad_dev_slots(int helm, int norder, int norder_branch, int64_t npatches, const int64_t* ixyzs,
+                                const double* srccoefs, const double* srcvals, int64_t ndtarg, int64_t ntarg,
+                                const double* targs, const int64_t* ipatch_id, const double* uvs_targ, double eps,
+                                const double* kpar6, int64_t nnz, const int64_t* row_ptr, const int64_t* col_ind,
+                                const int64_t* iquad, double rfac0, double* wnear, int self_nr, int self_nt,
+                                double self_tau_panel, void* stream, double* stats, int* nref_host, int* class_host,
+                                const float* mlp_params, float* feat_out, int* pred_host, const int* route_lmax,
+                                int* lev_host, int* unc_host, int64_t max_slots) {
   NearQuadArgs A = {};
   A.helm = helm != 0;
   A.norder = norder;
@@ -661,19 +660,35 @@ int fmm3dbie_nearquad_dev(int helm, int norder, int norder_branch, int64_t npatc
   A.route_lmax = route_lmax;
   A.lev_host = lev_host;
   A.unc_host = unc_host;
+  A.max_slots = max_slots;
   NearQuadStats st = {};
   const int rc = fmm_nearquad_device(A, &st, (hipStream_t)stream);
   if (stats) {
     const double v[24] = {(double)st.nself,  (double)st.nadap,   (double)st.nfixed,  (double)st.overflow,
                           (double)st.nf,     (double)st.kq,      st.ms_prep,         st.ms_fixed,
                           st.ms_adap,        st.ms_self,         st.ms_tables,       st.ms_select,
-                          st.ms_tree,        st.ms_shallow,      (double)st.nroute,  0,
+                          st.ms_tree,        st.ms_shallow,      (double)st.nroute,  (double)st.nnoslot,
                           (double)st.nfallback, (double)st.ncls[0], (double)st.ncls[1], (double)st.ncls[2],
                           (double)st.ncls[3], (double)st.ncls[4], (double)st.ncls[5], (double)st.cache_tris};
     std::memcpy(stats, v, sizeof(v));
   }
   g_last_error = rc;
   return rc;
+}
+
+int fmm3dbie_nearquad_dev(int helm, int norder, int norder_branch, int64_t npatches, const int64_t* ixyzs,
+                          const double* srccoefs, const double* srcvals, int64_t ndtarg, int64_t ntarg,
+                          const double* targs, const int64_t* ipatch_id, const double* uvs_targ, double eps,
+                          const double* kpar6, int64_t nnz, const int64_t* row_ptr, const int64_t* col_ind,
+                          const int64_t* iquad, double rfac0, double* wnear, int self_nr, int self_nt,
+                          double self_tau_panel,
+                          void* stream, double* stats, int* nref_host, int* class_host, const float* mlp_params,
+                          float* feat_out, int* pred_host, const int* route_lmax, int* lev_host,
+                          int* unc_host) {
+  return fmm3dbie_nearquad_dev_slots(helm, norder, norder_branch, npatches, ixyzs, srccoefs, srcvals, ndtarg, ntarg,
+                                     targs, ipatch_id, uvs_targ, eps, kpar6, nnz, row_ptr, col_ind, iquad, rfac0,
+                                     wnear, self_nr, self_nt, self_tau_panel, stream, stats, nref_host, class_host,
+                                     mlp_params, feat_out, pred_host, route_lmax, lev_host, unc_host, 0);
 }
 
 void* fmm3dbie_apply_plan_create(int helm, int64_t npatches, const int64_t* norders, const int64_t* ixyzs,

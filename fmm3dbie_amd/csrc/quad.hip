@@ -1737,6 +1737,14 @@ T* wsalloc(int slot, size_t n) {
   return (T*)v[slot].p;
 }
 
+void wsfree(int slot) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || g_ws[dev].size() < W_NSLOTS) return;
+  WsBuf& b = g_ws[dev][slot];
+  if (b.p) (void)hipFree(b.p);
+  b = WsBuf();
+}
+
 // Patch-independent tables of one (order, rule) combination, built once per device.
 struct OrderTables {
   int kq = 0, nf = 0;
@@ -1964,7 +1972,10 @@ int adaptive_slots() {
 // Slot pool of the adaptive levels: every triangle of the batched levels for up to
 // SLOT_ALL_BYTES, beyond that SLOTS_PER_PAIR slots per pair (measured need: 1.7 on the
 // deformed sphere of order 6, 1.0 to 1.5 on the other surfaces), pairs that find it empty
-// being integrated in another pass.
+// being integrated in another pass.  A slot is 4 moment vectors (1792 bytes at order 6,
+// Helmholtz: 7.3 GB for the 1.8 million adaptive pairs of the deformed sphere's 344k points).
+// Where the device has no room for that, the pool is halved until it fits, down to the
+// triangles of one pair.
 constexpr int SLOTS_ALL = 21;
 constexpr size_t SLOT_ALL_BYTES = (size_t)2 << 30;
 constexpr double SLOTS_PER_PAIR = 2.25;
@@ -2286,14 +2297,24 @@ int run_order(const NearQuadArgs& A, NearQuadStats* st, hipStream_t s) {
     HCHK(hipEventRecord(ev[7], s));
     constexpr int VL = NP * (HELM ? 2 : 1);
     const int64_t all = SLOTS_ALL * (int64_t)nadap;
-    const bool bounded = (size_t)all * 4 * VL * sizeof(double) > SLOT_ALL_BYTES;
+    int64_t cap = (size_t)all * 4 * VL * sizeof(double) > SLOT_ALL_BYTES ? (int64_t)(SLOTS_PER_PAIR * nadap) : all;
+    if (A.max_slots > 0) cap = std::max<int64_t>(std::min(cap, A.max_slots), SLOTS_ALL);
     AdapTiles T = {};
-    T.cap = (int)(bounded ? (int64_t)(SLOTS_PER_PAIR * nadap) : all);
-    T.slots = wsalloc<double>(W_SLOTS, (size_t)T.cap * 4 * VL);
-    T.items = wsalloc<int4>(W_ITEMS, T.cap);
     T.list1 = wsalloc<int2>(W_LIST1, nadap);
     T.list2 = wsalloc<int4>(W_LIST2, 4 * (size_t)nadap);
-    if (!T.slots || !T.items || !T.list1 || !T.list2) return -2;
+    if (!T.list1 || !T.list2) return -2;
+    for (;;) {
+      T.slots = wsalloc<double>(W_SLOTS, (size_t)cap * 4 * VL);
+      T.items = T.slots ? wsalloc<int4>(W_ITEMS, cap) : nullptr;
+      if (T.items) break;
+      (void)hipGetLastError();  // the failed allocation's
+      if (cap <= SLOTS_ALL) return -2;
+      cap = std::max<int64_t>(cap / 2, SLOTS_ALL);
+      wsfree(W_SLOTS);
+      wsfree(W_ITEMS);
+    }
+    T.cap = (int)cap;
+    const bool bounded = cap < all;
     T.boff = d_boff;
     T.npat = (int)npat;
     T.epsp = d_epsp;
@@ -2416,6 +2437,7 @@ int run_order(const NearQuadArgs& A, NearQuadStats* st, hipStream_t s) {
     st->nroute = nroute;
     st->cache_tris = ntri_plain;
     st->nfallback = counts8[5] + counts8[7];
+    st->nnoslot = counts8[4] + counts8[6] - st->nfallback;
     for (int c = 0; c < MAX_RULES; c++) st->ncls[c] = learned ? seg[at[c] + 1] - seg[at[c]] : (c == 0 ? nadap : 0);
     st->nref_total = 0;
     if (d_nref && A.nref_host) HCHK(hipMemcpy(A.nref_host, d_nref, sizeof(int) * A.nnz, hipMemcpyDeviceToHost));

@@ -47,6 +47,7 @@ struct NearQuadArgs {
   const int* route_lmax;   // optional, host (6): deepest level of each rule class (default 20)
   int* lev_host;           // optional: deepest level of every adaptive pair's tree (nnz)
   int* unc_host;           // optional: refinement tests below the cached tree per pair (nnz)
+  int64_t max_slots;       // bound on the slot pool of the adaptive levels (0: none of the caller's)
 };
 
 struct NearQuadStats {
@@ -58,6 +59,7 @@ struct NearQuadStats {
   // tree cache, the routed classes' tree caches; ms_adap is the adaptive kernel launches.
   int nroute, nfallback, ncls[6];
   double ms_tables, ms_select, ms_tree, ms_shallow;
+  int nnoslot;     // pairs integrated in a further pass because the slot pool was used up
   int cache_tris;  // triangles of the plain rule's tree cache (85: depths 0..3, 341: 0..4)
 };
 

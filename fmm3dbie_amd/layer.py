@@ -348,7 +348,7 @@ class NearQuadDevice:
         self.wnear = torch.zeros(self.nquad, dtype=torch.complex128 if self.helm else torch.float64, device=device)
         self.stats = None
 
-    def run(self, stream=None, want_detail=False, selector=None, features=None, route_lmax=None):
+    def run(self, stream=None, want_detail=False, selector=None, features=None, route_lmax=None, max_slots=0):
         """Fill self.wnear.  selector: device float32 tensor of MLP parameters (learned
         order selection: every adaptive pair integrated with the rule class the network
         predicts), or None for the plain adaptive path.  route_lmax: the deepest level of
@@ -356,7 +356,9 @@ class NearQuadDevice:
         the plain integrator); default 20.  features: device float32 tensor (nnz, 8) that
         receives the selector features of the adaptive pairs.  want_detail adds per-pair
         class, refinement-test count, deepest level, tests below the cached tree and
-        (with a selector) predicted rule class to self.stats."""
+        (with a selector) predicted rule class to self.stats.  max_slots: bound on the
+        slots for the moments of refined triangles (at least 21; 0: none), for callers
+        short of device memory; fewer take more passes and give the same weights."""
         torch = _torch()
         st = np.zeros(24)
         nref = np.zeros(self.nnz, np.int32) if want_detail else None
@@ -377,7 +379,7 @@ class NearQuadDevice:
             if lm.shape != (6,):
                 raise ValueError("route_lmax must hold 6 levels")
         s = stream if stream is not None else torch.cuda.current_stream()
-        rc = lib().fmm3dbie_nearquad_dev(
+        rc = lib().fmm3dbie_nearquad_dev_slots(
             int(self.helm), self.norder, self.norder_branch, self.npatches, _dptr(self.d_ixyzs),
             _dptr(self.d_srccoefs), _dptr(self.d_srcvals), self.ndtarg, self.ntarg, _dptr(self.d_targs),
             _dptr(self.d_pid) if self.d_pid is not None else None,
@@ -387,14 +389,14 @@ class NearQuadDevice:
             C.c_void_p(s.cuda_stream), _p(st), _p(nref) if want_detail else None, _p(cls) if want_detail else None,
             _dptr(selector) if selector is not None else None, _dptr(features) if features is not None else None,
             _p(pred) if pred is not None else None, _p(lm) if lm is not None else None,
-            _p(lev) if want_detail else None, _p(unc) if want_detail else None)
+            _p(lev) if want_detail else None, _p(unc) if want_detail else None, int(max_slots))
         if rc != 0:
             raise RuntimeError("fmm3dbie_nearquad_dev failed (status %d)" % rc)
         self.stats = dict(nself=int(st[0]), nadap=int(st[1]), nfixed=int(st[2]), overflow=int(st[3]), nf=int(st[4]),
                           kq=int(st[5]), ms_prep=st[6], ms_fixed=st[7], ms_adap=st[8], ms_self=st[9],
                           ms_tables=st[10], ms_select=st[11], ms_tree=st[12], ms_tree_routed=st[13],
-                          nroute=int(st[14]), nfallback=int(st[16]), ncls=[int(v) for v in st[17:23]],
-                          cache_tris=int(st[23]))
+                          nroute=int(st[14]), nnoslot=int(st[15]), nfallback=int(st[16]),
+                          ncls=[int(v) for v in st[17:23]], cache_tris=int(st[23]))
         if want_detail:
             self.stats["nref"] = nref
             self.stats["cls"] = cls

@@ -233,7 +233,8 @@ int fmm3dbie_last_error(void);
  * length (<= 0: 8, 10 and 2.0).
  * stats (optional, 24 doubles): nself, nadap, nfixed, overflow, nf, kq; times in ms of
  * prep, fixed, adaptive, self, host tables, selector, plain tree cache, routed tree
- * caches; rule classes used, 0, pairs sent back to the plain integrator, pairs per rule
+ * caches; rule classes used, pairs that took a further pass because the slot pool was used
+ * up (fmm3dbie_nearquad_dev_slots), pairs sent back to the plain integrator, pairs per rule
  * class (6), triangles of the plain rule's tree cache (85: depths 0..3; 341: depths 0..4,
  * used from 300 near pairs per patch).  nref_host/class_host/lev_host/unc_host (optional, nnz ints): refinement
  * tests per pair, pair class (0 self, 1 adaptive, 2 fixed), deepest level of the pair's
@@ -253,6 +254,20 @@ int fmm3dbie_nearquad_dev(int helm, int norder, int norder_branch, int64_t npatc
                           const int64_t *iquad, double rfac0, double *wnear, int self_nr, int self_nt,
                           double self_tau_panel, void *stream, double *stats, int *nref_host, int *class_host, const float *mlp_params,
                           float *feat_out, int *pred_host, const int *route_lmax, int *lev_host, int *unc_host);
+/* No reference counterpart: fmm3dbie_nearquad_dev with at most max_slots slots (at least 21;
+ * 0: no bound) for the moments of refined triangles, 4 p complex or real doubles each with p
+ * nodes per patch, for callers short of device memory.  The default is 21 slots per adaptive
+ * pair up to 2 GiB and 2.25 per pair beyond, or what the device has room for.  Fewer slots
+ * take more passes and give the same weights; with a selector, pairs without a slot are
+ * integrated with the plain rule. */
+int fmm3dbie_nearquad_dev_slots(int helm, int norder, int norder_branch, int64_t npatches, const int64_t *ixyzs,
+                                const double *srccoefs, const double *srcvals, int64_t ndtarg, int64_t ntarg,
+                                const double *targs, const int64_t *ipatch_id, const double *uvs_targ, double eps,
+                                const double *kpar6, int64_t nnz, const int64_t *row_ptr, const int64_t *col_ind,
+                                const int64_t *iquad, double rfac0, double *wnear, int self_nr, int self_nt,
+                                double self_tau_panel, void *stream, double *stats, int *nref_host, int *class_host,
+                                const float *mlp_params, float *feat_out, int *pred_host, const int *route_lmax,
+                                int *lev_host, int *unc_host, int64_t max_slots);
 
 /* findnearmem / findnear on device arrays (xyzs (3,ns), rads (ns), targets (ndt,nt));
  * row_ptr may be null for the count. */

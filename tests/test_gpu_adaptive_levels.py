@@ -1,6 +1,7 @@
 """GPU tests of the adaptive integrator's batched levels: every patch order, ragged numbers of
-targets per patch, off-surface targets, deep trees, and pairs sent back to another pass,
-against the CPU oracle (same weights to rounding, same refinement counts)."""
+targets per patch, off-surface targets and deep trees against the CPU oracle (same weights to
+rounding, same refinement counts), and pairs that take another pass because the slot pool is
+used up or by a level cap against the run where none does (same bits)."""
 import numpy as np
 import pytest
 
@@ -12,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 def _targets(g, n, seed):
     """n targets off a surface: most within its near field, some on top of it (trees that go
-    several levels below the batched ones), one patch's neighbourhood with none."""
+    several levels below the batched ones)."""
     rng = np.random.default_rng(seed)
     x = g["srcvals"][rng.integers(0, len(g["srcvals"]), n)]
     dist = np.where(np.arange(n) % 4 == 0, 1e-3, rng.uniform(0.02, 0.5, n))
@@ -49,3 +50,46 @@ def test_batched_levels_match_oracle(cuda, helm, norder, nt):
     assert np.abs(w - ref).max() < 1e-11 * np.abs(ref).max()
     # another run: other places in the tiles, the same bits
     assert np.array_equal(nq.run().cpu().numpy(), w)
+
+
+# Slots in all: those of one pair (one pair at a time in the last passes), part of the root level's, and
+# all but a few of what the pairs need
+@pytest.mark.parametrize("helm,norder,slots", [(True, 3, 21), (True, 4, 100), (False, 6, 700), (True, 6, 100),
+                                               (False, 2, 450)])
+def test_pairs_without_a_slot_take_another_pass(cuda, helm, norder, slots):
+    import torch
+    from fmm3dbie_amd import geometry as G, layer, problem, selector as S
+    g = G.get_sphere_npat(1.0, 1, (0, 0, 0), norder)
+    pars = np.array([2.0, 2.0j, 1.0]) if helm else np.array([1.0, 0.5])
+    P = problem.setup(g, 1e-6, helm, pars)
+    nq = layer.NearQuadDevice(g, helm, pars, 1e-6, P["row_ptr"], P["col_ind"], P["iquad"], P["rfac0"], device=cuda)
+    w0 = nq.run(want_detail=True).cpu().numpy().copy()
+    st0 = nq.stats
+    assert st0["nnoslot"] == 0
+    nref0, lev0, unc0 = st0["nref"].copy(), st0["lev"].copy(), st0["unc"].copy()
+
+    def check(st):
+        assert 0 < st["nnoslot"] + st["nfallback"] <= st0["nadap"]
+        assert np.array_equal(st["nref"], nref0) and np.array_equal(st["lev"], lev0)
+        assert np.array_equal(st["unc"], unc0)
+
+    for rep in range(2):  # (which pairs find a slot differs from run to run)
+        assert np.array_equal(nq.run(want_detail=True, max_slots=slots).cpu().numpy(), w0)
+        check(nq.stats)
+        assert nq.stats["nfallback"] == 0
+    # with a selector: the plain class with a level cap (a list of its own for the pairs sent back),
+    # and another class whose pairs all go back at a cap of 1 or for want of a slot, joined with
+    # the plain class's
+    plain = torch.as_tensor(S.forced(S.PLAIN_CLASS), device=cuda)
+    w = nq.run(want_detail=True, selector=plain, route_lmax=[2] * 6, max_slots=slots).cpu().numpy()
+    assert np.array_equal(w, w0)
+    check(nq.stats)
+    other = torch.as_tensor(S.forced(4), device=cuda)
+    ad = st0["cls"] == 1
+    for caps in ([1] * 6, [20] * 6, [20, 20, 20, 20, 1, 20]):
+        w = nq.run(want_detail=True, selector=other, route_lmax=caps, max_slots=slots).cpu().numpy()
+        assert caps[4] == 20 or nq.stats["nfallback"] > 0
+        for j in np.nonzero(ad)[0]:
+            a, b = P["iquad"][j] - 1, P["iquad"][j + 1] - 1
+            # both rules are within the integrator's own tolerance of 1e-5
+            assert np.abs(w[a:b] - w0[a:b]).max() < 2e-5 * np.abs(w0[a:b]).max()
