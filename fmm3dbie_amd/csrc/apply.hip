@@ -102,7 +102,8 @@ __global__ void k_oversample(int64_t nptso, const int* __restrict__ opatch, cons
 // reduced to one revolution first; otherwise the FP32 phase k r / (2 pi) goes to the hardware
 // sine and cosine directly (they take revolutions, valid below 256, which the plan checks
 // against its bounding box): with KIND 1 the FP32 coordinates are stored in units of the
-// wavelength (scaled before they are rounded to FP32), so that r is the phase.
+// wavelength (scaled before they are rounded to FP32), so that r is the phase; a and the normals
+// carry the unit's powers, strengths and kernel values are those of the caller's units.
 template <typename T>
 struct FarPar {
   T ar, ai;    // a
@@ -860,8 +861,8 @@ __global__ void k_fill(int64_t n, T* __restrict__ a, T v) {
   if (i < n) a[i] = v;
 }
 
-// Source geometry records (normals scaled by ns; FP32 coordinates by unit32) from rows x y z
-// du dv n of 12 doubles
+// Source geometry records (normals scaled by ns; FP32 coordinates by unit32 and normals by its
+// square) from rows x y z du dv n of 12 doubles
 __global__ void k_geo(int64_t n, const double* __restrict__ s12, double ns, double unit32,
                       double* __restrict__ g64, float* __restrict__ g32) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -870,7 +871,7 @@ __global__ void k_geo(int64_t n, const double* __restrict__ s12, double ns, doub
   const double v[6] = {s[0], s[1], s[2], ns * s[9], ns * s[10], ns * s[11]};
   for (int m = 0; m < 6; m++) {
     g64[GEO<double> * i + m] = v[m];
-    g32[GEO<float> * i + m] = (float)(m < 3 ? unit32 * v[m] : v[m]);
+    g32[GEO<float> * i + m] = (float)(unit32 * (m < 3 ? v[m] : unit32 * v[m]));
   }
   g32[GEO<float> * i + 6] = g32[GEO<float> * i + 7] = 0.0f;
 }
@@ -1037,9 +1038,10 @@ int apply_plan_build(ApplyPlan* P, const ApplyPlanInput& in, hipStream_t s) {
                                 (mx[2] - mn[2]) * (mx[2] - mn[2]));
   P->phase_small = !in.helm || std::fabs(in.zk[0]) * diag * 0.15915494309189533577 < 200.0;
   // FP32 coordinates in wavelengths where the phase is r itself (KIND 1); units so long or so
-  // short that FP32 powers of r could leave its range keep the caller's (KIND 2)
+  // short, or surfaces so small against the wavelength, that FP32 powers of r could leave its
+  // range keep the caller's (KIND 2)
   const double rev = in.zk[0] * 0.15915494309189533577;
-  P->wave32 = in.helm && in.zk[1] == 0.0 && P->phase_small && rev > 1e-6 && rev < 1e6;
+  P->wave32 = in.helm && in.zk[1] == 0.0 && P->phase_small && rev > 1e-6 && rev < 1e6 && rev * diag > 1e-6;
   P->unit32 = P->wave32 ? rev : 1.0;
   // the FP64 kernel evaluations take sin/cos of k r for |k r| <= SINCOS_RED_MAX
   if (in.helm && std::fabs(in.zk[0]) * diag > SINCOS_RED_MAX) {
@@ -1170,9 +1172,9 @@ static FarPar<T> far_par(const ApplyPlan* P) {
   } else {
     F.khi = (T)(zr * 0.15915494309189533577);  // k / (2 pi)
     F.klo = (T)0;
-    // in wavelengths: a + t (1 - ikr) and 1 / r, each over the unit, the rest in the strengths
-    F.ar = (T)(P->far_a[0] / P->unit32);
-    F.ai = (T)(P->far_a[1] / P->unit32);
+    // in wavelengths 1 / r is over the unit, so that a + t (1 - ikr) takes it (k_geo: t's part)
+    F.ar = (T)(P->far_a[0] * P->unit32);
+    F.ai = (T)(P->far_a[1] * P->unit32);
     if (P->wave32) F.kr = (T)6.283185307179586;
   }
   return F;
@@ -1431,11 +1433,10 @@ static void oversample(ApplyPlan* P, const V2<T>* sigma, int nrhs, int grp, V2<T
   const T* wover;
   if constexpr (sizeof(T) == 8) wover = P->wover;
   else wover = P->wover32;
-  const double scale = sizeof(T) == 4 ? P->unit32 * P->unit32 : 1.0;
 #define FMM_OVER(RB)                                                                                             \
   k_oversample<T, RB><<<dim3(nblk(NO, 256), (unsigned)(nr / RB)), 256, 0, s>>>(                                  \
       NO, P->opatch, P->ixyzs, P->ixyzso, P->ioff, P->np_of, P->imat, sigma, nrhs, P->npts, wover,               \
-      scale * P->far_phase[0], scale * P->far_phase[1], grp, str)
+      P->far_phase[0], P->far_phase[1], grp, str)
   if (grp % 4 == 0) FMM_OVER(4);
   else if (grp == 2) FMM_OVER(2);
   else FMM_OVER(1);

@@ -91,6 +91,29 @@ def test_far_sum_forms_match_a_64_bit_sum(cuda, helm, pars, norder):
     plan.close()
 
 
+# densities far down FP32's range at a long wavelength: the unit in which a plan stores its coordinates
+# must not enter the strengths (k / (2 pi) squared is 2.5e-10 here, which would leave them 1e-42)
+@pytest.mark.parametrize("nrhs", [1, 3, 8])
+def test_small_densities_at_a_long_wavelength(cuda, nrhs):
+    import torch
+    from fmm3dbie_amd import geometry as G, layer, problem
+    g = G.get_sphere_npat(1.0, 1, (0, 0, 0), 4)
+    pars = np.array([1e-4, 1.0, 1.0])
+    P = problem.setup(g, 1e-6, True, pars)
+    plan = layer.ApplyPlan(g, True, pars, P["row_ptr"], P["col_ind"], P["iquad"], np.zeros(P["nquad"], complex),
+                           P["novers"], P["ixyzso"], P["srcover"], P["whtsover"])
+    rng = np.random.default_rng(2)
+    N = len(g["srcvals"])
+    S = 1e-31 * (rng.standard_normal((nrhs, N)) + 1j * rng.standard_normal((nrhs, N)))
+    ref, size, _ = _sum64(g, P, True, pars, S)
+    s = torch.as_tensor(S, device=cuda).to(torch.complex64)
+    out = np.atleast_2d(plan.apply(s[0].contiguous() if nrhs == 1 else s.contiguous(), 32, 1).cpu().numpy())
+    # (norms of values whose squares underflow in FP32: complex128 from here on)
+    err = np.linalg.norm((out.astype(complex) - ref) * 1e30) / np.linalg.norm(size * 1e30)
+    assert err < 30 * 2.0 ** -24, err * 2.0 ** 24  # the bound above
+    plan.close()
+
+
 # several groups of 16 in FP32 (split products), at the edges of the groups; the 10-point patches
 # leave a ragged last tile of 32 sources
 @pytest.mark.parametrize("helm,pars", [(False, (0.7, -1.3)), (True, (5.0, 5.0j, 1.0)), (True, (2.0 + 0.7j, 1.0, 1.0))])
