@@ -51,14 +51,18 @@ constexpr int MG = 16;
 // right-hand sides: group g, node i, right-hand side r of the group at (g nptso + i) nr + r.
 // Right-hand sides from nrhs to the end of the last group are zero.
 // A thread takes RB right-hand sides of one node (grid y).
+// bmax (FP32, optional): the largest |Re s|, |Im s| of the workgroup's nodes for each right-hand
+// side, at workgroup * right-hand sides (padded) + right-hand side.
 template <typename T, int RB>
-__global__ void k_oversample(int64_t nptso, const int* __restrict__ opatch, const int64_t* __restrict__ ixyzs,
+__global__ void __launch_bounds__(256) k_oversample(int64_t nptso, const int* __restrict__ opatch, const int64_t* __restrict__ ixyzs,
                              const int64_t* __restrict__ ixyzso, const int64_t* __restrict__ ioff,
                              const int* __restrict__ np_of, const double* __restrict__ imat,
                              const V2<T>* __restrict__ sigma, int nrhs, int64_t ldsig,
-                             const T* __restrict__ wover, double pr, double pi, int nr, V2<T>* __restrict__ str) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= nptso) return;
+                             const T* __restrict__ wover, double pr, double pi, int nr, V2<T>* __restrict__ str,
+                             float* __restrict__ bmax) {
+  const int64_t it = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  const bool in = it < nptso;
+  const int64_t i = in ? it : nptso - 1;
   const int r0 = blockIdx.y * RB;
   const int ip = opatch[i];
   const int p = np_of[ip];
@@ -88,9 +92,32 @@ __global__ void k_oversample(int64_t nptso, const int* __restrict__ opatch, cons
   for (int r = 0; r < RB; r++) {
     const double a = sr[r] * w, b = si[r] * w;
     const bool live = r0 + r < nrhs;
-    o[r] = {live ? (T)(pr * a - pi * b) : (T)0, live ? (T)(pr * b + pi * a) : (T)0};
+    const V2<T> v = {live ? (T)(pr * a - pi * b) : (T)0, live ? (T)(pr * b + pi * a) : (T)0};
+    if (in) o[r] = v;
+    sr[r] = v.x;
+    si[r] = v.y;
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (!bmax) return;
+    __shared__ float wmax[4][RB];
+#pragma unroll
+    for (int r = 0; r < RB; r++) {
+      float m = fmaxf(fabsf((float)sr[r]), fabsf((float)si[r]));  // (past the last node: that node's)
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+      if (threadIdx.x % 64 == 0) wmax[threadIdx.x / 64][r] = m;
+    }
+    __syncthreads();
+    if (threadIdx.x < RB) {
+      const int r = threadIdx.x;
+      bmax[(int64_t)blockIdx.x * (gridDim.y * RB) + r0 + r] =
+          fmaxf(fmaxf(wmax[0][r], wmax[1][r]), fmaxf(wmax[2][r], wmax[3][r]));
+    }
   }
 }
+
+// Values that k_oversample leaves after the strengths of nr right-hand sides (bmax)
+static int64_t bmax_values(int64_t nptso, int nr) { return (nptso + 255) / 256 * nr; }
 
 // ---- kernel values of the far sum
 // The combined kernel is K = (alpha + beta t (1 - ikr)) e^{ikr} / (4 pi r), t = (x - y).n / r^2.
@@ -443,6 +470,11 @@ __global__ void __launch_bounds__(64 * FW)
 // (target l % 16, sources 8 (l / 16) ..) on the vector units, which are the operand of the 16x16x32
 // products as they stand.  The workgroup stages the sources' geometry and the split strengths in
 // LDS, in the order in which the lanes read them; the next tile's are loaded while one is summed.
+// The strengths of a right-hand side are scaled by the power of two that takes the largest to 1
+// and its potentials back: the last term of an FP32 value, 2^-24 of it, is then above bfloat16's
+// smallest value whatever the size of a density (unscaled, strengths of 1e-34 lose 1e-5).  The
+// largest comes from k_oversample's workgroups.  (Scaled by tiles instead, with no such pass, 16
+// densities took 18.1 ms and 64 37.4.)
 // The complex product takes four real ones, as in k_farsum_mfma, and a tile's products are
 // summed by themselves before they are added to the potentials: the matrix cores round each sum
 // of a chain downwards, which over all sources would add up (error of the 64-density apply below
@@ -476,15 +508,16 @@ template <int KIND, int NG>
 __global__ void __launch_bounds__(64 * FW, 2)
     k_farsum_split(int ntarg, const float* __restrict__ tx, const float* __restrict__ ty, const float* __restrict__ tz,
                    int nsrc, const float* __restrict__ geo, const int64_t* __restrict__ ixyzso,
-                   const V2<float>* __restrict__ str, const int64_t* __restrict__ row_ptr,
-                   const int* __restrict__ near_sorted, FarPar<float> P, int chunk, int nrhs,
-                   V2<float>* __restrict__ part, int64_t ldpart) {
+                   const V2<float>* __restrict__ str, const float* __restrict__ bmax,
+                   const int64_t* __restrict__ row_ptr, const int* __restrict__ near_sorted, FarPar<float> P, int chunk,
+                   int nrhs, V2<float>* __restrict__ part, int64_t ldpart) {
   using T = float;
   constexpr int NM = KIND == 0 ? 1 : 2;  // kernel matrices: Re K, Im K
   constexpr int SI = NG == 1 ? 2 : (NG == 2 ? 4 : 8);  // sources that a thread stages, of one right-hand side
   constexpr int NT = MT;
   __shared__ __align__(16) T lgeo[ST * 8];
   __shared__ __align__(16) bf8 lstr[NG][2][3][64];  // Re s, Im s
+  __shared__ int lexp[NG * MG];                     // exponent bits of a right-hand side's largest strength
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int t0 = (blockIdx.x * FW + wv) * (16 * NT);
   const int ks = lane >> 4;  // this lane's sources: 8 ks .. 8 ks + 7 of a tile
@@ -511,6 +544,23 @@ __global__ void __launch_bounds__(64 * FW, 2)
   const int sr = threadIdx.x & 15, sj = SI * ((threadIdx.x >> 4) % (ST / SI)), sg = (threadIdx.x >> 4) / (ST / SI);
   const bool stager = sg < NG;
   const V2<T>* sp = str + (int64_t)(stager ? sg : 0) * nsrc * MG + sr;
+  for (int r = threadIdx.x; r < NG * MG; r += 64 * FW) lexp[r] = 0;
+  __syncthreads();
+  {
+    constexpr int PER = 64 * FW / (NG * MG);  // threads per right-hand side
+    const int r = threadIdx.x % (NG * MG), nb = (nsrc + 255) / 256;
+    float m = 0.0f;
+    if (threadIdx.x < PER * NG * MG)
+      for (int b = threadIdx.x / (NG * MG); b < nb; b += PER) m = fmaxf(m, bmax[(int64_t)b * (NG * MG) + r]);
+    atomicMax(lexp + r, __float_as_int(m) >> 23);
+  }
+  __syncthreads();
+  // 2^(e - 127) is the unit of a right-hand side, 2^(127 - e) its inverse: both are normal
+  auto unit_exp = [&](int r) {
+    const int e = lexp[r];
+    return e < 1 ? 1 : (e > 253 ? 253 : e);
+  };
+  const T scale = __int_as_float((254 - unit_exp(stager ? sg * MG + sr : 0)) << 23);
   V2<T> next[SI];
   T nextg;  // and one value of the geometry
   static_assert(ST * 8 == 64 * FW, "");
@@ -537,8 +587,8 @@ __global__ void __launch_bounds__(64 * FW, 2)
       bf2 v[3][SI / 2];
 #pragma unroll
       for (int u = 0; u < SI; u += 2) {
-        T a = m == 0 ? next[u].x : next[u].y;
-        T b = m == 0 ? next[u + 1].x : next[u + 1].y;
+        T a = scale * (m == 0 ? next[u].x : next[u].y);
+        T b = scale * (m == 0 ? next[u + 1].x : next[u + 1].y);
 #pragma unroll
         for (int k = 0; k < 3; k++) v[k][u / 2] = next_term(a, b);
       }
@@ -644,10 +694,12 @@ __global__ void __launch_bounds__(64 * FW, 2)
     for (int g = 0; g < NG; g++) {
       const int r = g * MG + (lane & 15);
       if (r >= nrhs) continue;
+      const T unit = __int_as_float(unit_exp(r) << 23);
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const int it = t0 + 16 * t + 4 * ks + e;
-        if (it < ntarg) part[(int64_t)blockIdx.y * ldpart + (int64_t)r * ntarg + it] = {re[t][g][e], im[t][g][e]};
+        if (it < ntarg)
+          part[(int64_t)blockIdx.y * ldpart + (int64_t)r * ntarg + it] = {unit * re[t][g][e], unit * im[t][g][e]};
       }
     }
 }
@@ -1135,7 +1187,7 @@ static int ensure_ws(ApplyPlan* P, int nrhs) {
   apply_plan_free_ws(P);
   const size_t ns = (size_t)P->nptso * padded_rhs(nrhs);
   P->str64 = dal<double>(2 * ns);
-  P->str32 = dal<float>(2 * ns);
+  P->str32 = dal<float>(2 * ns + bmax_values(P->nptso, padded_rhs(nrhs)));
   P->sig64c = dal<double>(2 * (size_t)P->npts);
   P->pot64c = dal<double>(2 * (size_t)P->ntarg);
   // partial far sums: nsplit x nrhs x npts with nsplit x nrhs <= far_split_cap x 64
@@ -1286,10 +1338,12 @@ static int launch_far_split(ApplyPlan* P, int64_t wg_target, const V2<float>* st
                                        part_cap / ((int64_t)nrhs * P->ntarg), &chunk);
   const dim3 grid(g, (unsigned)nsplit);
   const int kind = far_kind<float>(P);
+  const float* bmax = (const float*)(str + P->nptso * padded_rhs(nrhs, MG));  // as in oversample
 #define FMM_FARS(KD, NG)                                                                                          \
-  k_farsum_split<KD, NG><<<grid, 64 * FW, 0, s>>>((int)P->ntarg, trg[0], trg[1], trg[2], (int)P->nptso, P->geo32, \
-                                                  P->ixyzso, str, P->row_ptr, P->near_sorted, far_par<float>(P),  \
-                                                  (int)chunk, nrhs, part, (int64_t)nrhs * P->ntarg)
+  k_farsum_split<KD, NG><<<grid, 64 * FW, 0, s>>>(                                                             \
+      (int)P->ntarg, trg[0], trg[1], trg[2], (int)P->nptso, P->geo32, P->ixyzso, str,                          \
+      bmax, P->row_ptr, P->near_sorted, far_par<float>(P), (int)chunk, nrhs, part,                              \
+      (int64_t)nrhs * P->ntarg)
 #define FMM_FARK(NG)                     \
   do {                                   \
     if (kind == 0) FMM_FARS(0, NG);      \
@@ -1324,7 +1378,11 @@ static int far_group(const ApplyPlan* P, int nrhs, int prec, int64_t str_cap, in
   const auto it = P->tuned.find(prec * 1000 + nrhs);
   *wg = it != P->tuned.end() ? it->second.second : P->far_wg_target;
   int grp = it != P->tuned.end() ? it->second.first : default_group(nrhs);
-  while (P->nptso * padded_rhs(nrhs, grp) > str_cap || grp > MG) {
+  auto need = [&](int g) {
+    const int nr = padded_rhs(nrhs, g);
+    return P->nptso * nr + (prec == 32 && g == MG ? (bmax_values(P->nptso, nr) + 1) / 2 : 0);
+  };
+  while (need(grp) > str_cap) {
     grp /= 2;
     while (nrhs % grp != 0) grp /= 2;
   }
@@ -1433,10 +1491,13 @@ static void oversample(ApplyPlan* P, const V2<T>* sigma, int nrhs, int grp, V2<T
   const T* wover;
   if constexpr (sizeof(T) == 8) wover = P->wover;
   else wover = P->wover32;
+  float* bmax = nullptr;
+  if constexpr (sizeof(T) == 4)
+    if (grp == MG) bmax = (float*)(str + NO * nr);  // for k_farsum_split, behind the strengths
 #define FMM_OVER(RB)                                                                                             \
   k_oversample<T, RB><<<dim3(nblk(NO, 256), (unsigned)(nr / RB)), 256, 0, s>>>(                                  \
       NO, P->opatch, P->ixyzs, P->ixyzso, P->ioff, P->np_of, P->imat, sigma, nrhs, P->npts, wover,               \
-      P->far_phase[0], P->far_phase[1], grp, str)
+      P->far_phase[0], P->far_phase[1], grp, str, bmax)
   if (grp % 4 == 0) FMM_OVER(4);
   else if (grp == 2) FMM_OVER(2);
   else FMM_OVER(1);
@@ -1488,9 +1549,10 @@ static int check_prec_nrhs(int prec, int nrhs) {
 }
 
 static ApplyWs plan_ws(const ApplyPlan* P, int prec) {
-  const int64_t cap = (int64_t)P->far_split_cap * 64 * P->ntarg, str = P->nptso * padded_rhs(P->ws_cap);
+  const int nr = padded_rhs(P->ws_cap);
+  const int64_t cap = (int64_t)P->far_split_cap * 64 * P->ntarg, str = P->nptso * nr;
   if (prec == 64) return {P->str64, P->part64, str, cap};
-  return {P->str32, P->part32, str, cap};
+  return {P->str32, P->part32, str + (bmax_values(P->nptso, nr) + 1) / 2, cap};
 }
 
 // sigma/pot: complex (interleaved) device arrays of length npts * nrhs, leading dim npts;
@@ -1567,9 +1629,9 @@ int apply_plan_tune(ApplyPlan* P, int prec, int nrhs, hipStream_t s, double* rep
   if (nrhs < 1 || nrhs > 64 || (prec != 32 && prec != 64)) return -6;
   if (ensure_ws(P, nrhs) != 0) return -2;
   if (P->ntarg == 0 || P->nptso == 0) return 0;
-  const int64_t nval = 2 * P->nptso * padded_rhs(nrhs);
+  const int64_t nval = 2 * P->nptso * padded_rhs(nrhs), nmax = bmax_values(P->nptso, padded_rhs(nrhs));
   if (prec == 64) k_fill<double><<<nblk(nval, 256), 256, 0, s>>>(nval, P->str64, 1.0);
-  else k_fill<float><<<nblk(nval, 256), 256, 0, s>>>(nval, P->str32, 1.0f);
+  else k_fill<float><<<nblk(nval + nmax, 256), 256, 0, s>>>(nval + nmax, P->str32, 1.0f);
   auto far = [&](int gsz, int64_t wg) {
     int64_t nsplit;
     const int64_t cap = (int64_t)P->far_split_cap * 64 * P->ntarg;

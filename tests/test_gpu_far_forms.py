@@ -92,9 +92,11 @@ def test_far_sum_forms_match_a_64_bit_sum(cuda, helm, pars, norder):
 
 
 # densities far down FP32's range at a long wavelength: the unit in which a plan stores its coordinates
-# must not enter the strengths (k / (2 pi) squared is 2.5e-10 here, which would leave them 1e-42)
-@pytest.mark.parametrize("nrhs", [1, 3, 8])
-def test_small_densities_at_a_long_wavelength(cuda, nrhs):
+# must not enter the strengths (k / (2 pi) squared is 2.5e-10 here, which would leave them 1e-42), nor
+# the smallest value of the terms of the split products (strengths of 2e-35 here); and far up
+@pytest.mark.parametrize("nrhs,size", [(1, 1e-31), (3, 1e-31), (8, 1e-31), (9, 1e-33), (16, 1e-33), (17, 1e-33),
+                                       (33, 1e-33), (64, 1e-33), (16, 1e36), (64, 1e36)])
+def test_densities_of_extreme_size_at_a_long_wavelength(cuda, nrhs, size):
     import torch
     from fmm3dbie_amd import geometry as G, layer, problem
     g = G.get_sphere_npat(1.0, 1, (0, 0, 0), 4)
@@ -104,12 +106,12 @@ def test_small_densities_at_a_long_wavelength(cuda, nrhs):
                            P["novers"], P["ixyzso"], P["srcover"], P["whtsover"])
     rng = np.random.default_rng(2)
     N = len(g["srcvals"])
-    S = 1e-31 * (rng.standard_normal((nrhs, N)) + 1j * rng.standard_normal((nrhs, N)))
-    ref, size, _ = _sum64(g, P, True, pars, S)
-    s = torch.as_tensor(S, device=cuda).to(torch.complex64)
-    out = np.atleast_2d(plan.apply(s[0].contiguous() if nrhs == 1 else s.contiguous(), 32, 1).cpu().numpy())
-    # (norms of values whose squares underflow in FP32: complex128 from here on)
-    err = np.linalg.norm((out.astype(complex) - ref) * 1e30) / np.linalg.norm(size * 1e30)
+    S = rng.standard_normal((nrhs, N)) + 1j * rng.standard_normal((nrhs, N))
+    ref, bound, _ = _sum64(g, P, True, pars, S)
+    s = torch.as_tensor(size * S, device=cuda).to(torch.complex64)
+    out = plan.apply(s[0].contiguous() if nrhs == 1 else s.contiguous(), 32, 1).cpu().numpy()
+    out = np.atleast_2d(out).astype(complex) / size
+    err = np.linalg.norm(out - ref) / np.linalg.norm(bound)
     assert err < 30 * 2.0 ** -24, err * 2.0 ** 24  # the bound above
     plan.close()
 
