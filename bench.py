@@ -533,7 +533,8 @@ def learned_mixed_solve(dev):
     # per-kernel times of each kernel alone (every kernel in order on one stream)
     layer.set_side_stream(False)
     nq.run()
-    q64 = {k: nq.stats[k] for k in ("ms_tree", "ms_adap", "ms_fixed", "ms_self")}
+    # (ms_select of the plain rule: bucketing its pairs by patch)
+    q64 = {k: nq.stats[k] for k in ("ms_select", "ms_tree", "ms_adap", "ms_fixed", "ms_self")}
     nq.run(selector=params, route_lmax=lmax)
     ql = {k: nq.stats[k] for k in ("ms_select", "ms_tree", "ms_tree_routed", "ms_adap", "ms_fixed", "ms_self",
                                    "nfallback", "ncls")}
@@ -555,7 +556,7 @@ def learned_mixed_solve(dev):
                               "rres": rrl, "quad_ms": ql, "field_err": el,
                               "err_vs_converged_fp64": _wrel(xl.cpu().numpy(), xc, P["wts"])},
             "speedup_solve": ts64 / tsl, "speedup_setup_plus_solve": tt64 / ttl,
-            "adaptive_part_ms": {"plain": q64["ms_tree"] + q64["ms_adap"],
+            "adaptive_part_ms": {"plain": q64["ms_select"] + q64["ms_tree"] + q64["ms_adap"],
                                  "learned": ql["ms_select"] + ql["ms_tree"] + ql["ms_tree_routed"] + ql["ms_adap"]},
             "selector": {"train_pairs": info["n_train"], "heldout_pairs": info["n_heldout"],
                          "acc_train": info["acc_train"], "acc_heldout": info["acc_heldout"],

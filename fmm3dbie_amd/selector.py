@@ -23,7 +23,8 @@ with it, and its tree cache holds no depth below that cap.
 
 Workflow: ``X, y, idx, info = collect(nq)``, ``params, tinfo = train(X, y)`` (GPU
 training, normalisation folded into the first layer), ``lmax = level_caps(y, info)``,
-then ``nq.run(selector=params, route_lmax=lmax)``.
+then ``nq.run(selector=params, route_lmax=lmax)``; where ``info["used"]`` holds the plain
+class alone, routing does not pay on this surface and ``nq.run()`` is the faster call.
 """
 import ctypes as C
 
@@ -107,8 +108,12 @@ def chunks(norder, kq):
     return -(-kq // cr), -(-4 * kq // cr)
 
 
-# Cost of a node step on the cached tree in chunks of the subtrees below it, measured on the
-# deformed sphere of order 6: 25 ps per pair and step, 2.2 ns per chunk.
+# Cost of a node step on the cached tree in chunks of the subtrees below it: 25 ps per pair and
+# step against 2.2 ns per chunk, measured on the deformed sphere of order 6.  Fitted by itself from
+# the six launches of a surface the ratio is ill-determined, the steps of a class being nearly a
+# cost per pair: 0 to 0.009 on tori, spheres and deformed spheres of orders 2 to 6, both kernels.
+# With this one the fitted launch times of orders 4 to 6 are within 10% of the measured ones (16%
+# for a Laplace torus), those of orders 2 and 3 within 31%.
 STEP_CHUNKS = 0.011
 
 
@@ -127,12 +132,14 @@ def collect(nq, stream=None):
     its lanes are all busy or not).  A pair's work is its steps on the cached tree, at
     STEP_CHUNKS chunks each, and its chunks below it (geometry evaluated); the measured times
     of the six launches are fitted by a cost per chunk and a cost per pair, and the label is
-    the class of least fitted cost among the classes worth their tree cache (open_classes).
+    the class of least fitted cost among the classes worth their tree cache and the selector
+    itself (open_classes).
     Returns (X (nadap, 8) float32, y (nadap,) int32, CSR entry index of each adaptive pair,
     info with the per-class fitted cost 'cost', kernel evaluations 'evals', deepest levels
     'lev' (6, nadap), launch times 'ms', the fitted unit costs 'unit' (ms per chunk, per
-    pair), node counts 'kq', the plain degree 'q0', the classes used 'used' and the plain
-    rule's tree-cache time for depths 0..2 'ms_tree')."""
+    pair), node counts 'kq', the plain degree 'q0', the classes used 'used', the plain
+    rule's tree-cache time for depths 0..2 'ms_tree' and the selector's own time (features,
+    inference, bucketing by class) beyond the plain bucketing 'ms_route')."""
     from scipy.optimize import nnls
     from . import layer
     torch = _torch()
@@ -154,6 +161,9 @@ def collect(nq, stream=None):
         ccomp = np.zeros((NCLASS, len(idx)))
         lev = np.zeros((NCLASS, len(idx)), np.int32)
         ms = np.zeros(NCLASS)
+        route = np.zeros(NCLASS)
+        nq.run(stream=stream)
+        ms_bucket = nq.stats["ms_select"]
         for c in range(NCLASS):
             sel = torch.as_tensor(forced(c), device=dev)
             for rep in range(2):  # the second run is timed (tables and caches built)
@@ -167,6 +177,7 @@ def collect(nq, stream=None):
             ccomp[c] = chunks(nq.norder, kq[c])[1] * unc
             lev[c] = st["lev"][idx]
             ms[c] = st["ms_adap"]
+            route[c] = st["ms_select"]
     finally:
         layer.set_side_stream(side)
     # a cost per pair (lists, test, weights: the same for every class) keeps the step costs from
@@ -176,9 +187,10 @@ def collect(nq, stream=None):
     cost = unit[0] * work
     tree = tree_cost(ms_tree, kq, q0)
     fill = np.where(tree > 0.0, fill_cost(nq.npatches, kq, STEP_CHUNKS * unit[0]), 0.0)
-    y, used = open_classes(cost, tree + fill)
+    ms_route = max(0.0, float(route.min() - ms_bucket))
+    y, used = open_classes(cost, tree + fill, ms_route)
     return X, y, idx, dict(cost=cost, evals=ncached + ncomp, lev=lev, ms=ms, unit=unit, kq=kq, q0=q0,
-                           used=used, ms_tree=ms_tree)
+                           used=used, ms_tree=ms_tree, ms_route=ms_route)
 
 
 def tree_cost(ms_tree, kq, q0):
@@ -201,17 +213,22 @@ def fill_cost(npatches, kq, step):
     return 8.0 * npatches * 25 * step * np.array([tile_steps(int(k)) for k in kq])
 
 
-def open_classes(cost, cache):
+def open_classes(cost, cache, route=0.0):
     """Which rule classes to use and each pair's label.  A class other than the plain one
     costs its tree cache and partly filled tiles once per generation (cache[c], same unit as cost);
     starting from the plain class alone, the class whose pairs would save the most
     (sum over pairs of the drop in their least cost, minus its cache) is added while that
-    saving is positive.  Returns (labels: the least-cost used class of every pair, used
+    saving is positive.  Routing itself costs route once per generation (the selector): where
+    all that is saved does not pay for it, the free classes alone are used.  (Uncharged, a
+    torus of 768 patches of order 4 opened a class that took the adaptive part from 0.77 to
+    0.94 ms, a sphere of 1728 patches of order 3 one from 0.93 to 1.22 ms.)  Returns (labels: the least-cost used class of every pair, used
     classes as a boolean array)."""
     ncls = cost.shape[0]
     used = np.zeros(ncls, bool)
     used[[c for c in range(ncls) if cache[c] == 0.0] or [PLAIN_CLASS]] = True
+    free = used.copy()
     best = cost[used].min(axis=0)
+    saved = 0.0
     while True:
         gain = np.array([np.maximum(best - cost[c], 0.0).sum() - cache[c] if not used[c] else -np.inf
                          for c in range(ncls)])
@@ -219,7 +236,10 @@ def open_classes(cost, cache):
         if not np.isfinite(gain[c]) or gain[c] <= 0.0:
             break
         used[c] = True
+        saved += gain[c]
         best = np.minimum(best, cost[c])
+    if saved <= route:
+        used = free
     masked = np.where(used[:, None], cost, np.inf)
     return np.argmin(masked, axis=0).astype(np.int32), used
 

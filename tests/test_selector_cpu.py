@@ -108,6 +108,12 @@ def test_open_classes_pays_for_each_tree_cache():
     cache[0], cache[5] = 200.0, 60.0
     y, used = S.open_classes(cost, cache)
     assert used.sum() == 1 and used[P] and np.all(y == P)
+    # classes that save 40 and 10 pay for a selector that costs 49, and not for one of 51
+    cache[0], cache[5] = 60.0, 30.0
+    y, used = S.open_classes(cost, cache, 49.0)
+    assert used[0] and used[5]
+    y, used = S.open_classes(cost, cache, 51.0)
+    assert used.sum() == 1 and used[P] and np.all(y == P)
     # the plain class's cache is free; classes of the plain degree too
     c = S.tree_cost(0.3, [33, 42, 55, 79, 112, 150], 16)
     assert c[P] == 0.0 and abs(c[5] - 0.3 * 150 / 55) < 1e-15
