@@ -254,7 +254,7 @@ __global__ void __launch_bounds__(64) k_farsum(int ntarg, const T* __restrict__ 
 #pragma unroll
   for (int r = 0; r < NRHS; r++) { accr[r] = 0; acci[r] = 0; }
   const int jbeg = blockIdx.y * chunk;
-  const int jend = jbeg + chunk < nsrc ? jbeg + chunk : nsrc;
+  const int jend = chunk < nsrc - jbeg ? jbeg + chunk : nsrc;
   // source j: r^2 and, unless skip, its contribution
   auto pair = [&](int j, auto test) -> T {
     const T* g = geo + (int64_t)j * GEO<T>;
@@ -375,7 +375,7 @@ __global__ void __launch_bounds__(64 * FW)
   T x[NT], y[NT], z[NT];
   dbl4 re[NT], im[NT];
   const int jbeg = blockIdx.y * chunk;
-  const int jend = jbeg + chunk < nsrc ? jbeg + chunk : nsrc;
+  const int jend = chunk < nsrc - jbeg ? jbeg + chunk : nsrc;
   NearCursor nc[NT];
   bool act[NT];
 #pragma unroll
@@ -522,7 +522,7 @@ __global__ void __launch_bounds__(64 * FW, 2)
   const int t0 = (blockIdx.x * FW + wv) * (16 * NT);
   const int ks = lane >> 4;  // this lane's sources: 8 ks .. 8 ks + 7 of a tile
   const int jbeg = blockIdx.y * chunk;
-  const int jend = jbeg + chunk < nsrc ? jbeg + chunk : nsrc;
+  const int jend = chunk < nsrc - jbeg ? jbeg + chunk : nsrc;
   T x[NT], y[NT], z[NT];
   NearCursor nc[NT];
   bool act[NT];
@@ -1029,6 +1029,13 @@ int apply_plan_build(ApplyPlan* P, const ApplyPlanInput& in, hipStream_t s) {
   const int64_t npat = in.npatches, N = P->ntarg, NO = in.nptso;
   const double* tsrc = in.targs ? in.targs : in.srcvals;  // target coordinates
   const int64_t tstride = in.targs ? in.ndtarg : 12;
+  // the far sum counts nodes and targets, rounded up to a tile, in 32 bits (more do not fit the
+  // card: 96 bytes of geometry records and strengths per node and 12 KB of partial sums per target)
+  if (NO > INT32_MAX - 4096 || N > INT32_MAX - 4096) {
+    fprintf(stderr, "fmm3dbie_amd: %lld oversampled nodes and %lld targets: at most 2^31 - 4097 of each\n",
+            (long long)NO, (long long)N);
+    return -2;
+  }
   // host-side tables: interpolation matrices per (norder, nover), patch of each
   // oversampled point, sorted near lists, uniform-p check
   std::vector<int64_t> ioff(npat);
