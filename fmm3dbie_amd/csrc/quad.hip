@@ -1448,8 +1448,9 @@ __global__ void k_features(int nadap, const int2* __restrict__ list, const int64
     for (int k = 0; k < 8; k++) feat_full[8 * (int64_t)jt.x + k] = f[k];
 }
 
-// Bucket key of an adaptive pair (MLP_OUT * npatches keys): place of its rule class (the 4 bits of
-// place from 4 c), then patch.  Without a prediction every pair is in class 0 (the plain rule),
+static_assert(MLP_OUT == MAX_RULES, "");
+// Bucket key of an adaptive pair (npatches keys, with a selector MAX_RULES * npatches): place of its
+// rule class (the 4 bits of place from 4 c), then patch.  Without a prediction every pair is in class 0 (the plain rule),
 // sorted by patch.
 __device__ __forceinline__ int64_t bucket_key(int c, int place, int64_t patch, int64_t npat) {
   return ((place >> (4 * c)) & 15) * npat + patch;
@@ -1703,9 +1704,9 @@ T* dalloc(size_t n) {
 // are serialised (g_quad_mutex) and every call synchronises its stream before returning,
 // so a buffer is never resized while a kernel of an earlier call uses it.
 enum WsSlot {
-  W_CMS, W_RADS, W_EPSP, W_AREA, W_CNT, W_OFF, W_FILL, W_CLS, W_COUNTS, W_ADAP, W_SELF, W_FIXED, W_NREF,
-  W_CACHE, W_STACK, W_X, W_PRED, W_BCNT, W_BOFF, W_SORTED, W_FB, W_PFULL, W_QCTR, W_LEV, W_SEG, W_UNC,
-  W_SLOTS, W_ITEMS, W_LIST1, W_LIST2, W_TCNT, W_FLAG,
+  W_CMS, W_RADS, W_EPSP, W_AREA, W_ZERO, W_OFF, W_CLS, W_ADAP, W_SELF, W_FIXED, W_NREF,
+  W_CACHE, W_STACK, W_X, W_PRED, W_BOFF, W_SORTED, W_FB, W_PFULL, W_LEV, W_SEG, W_UNC,
+  W_SLOTS, W_ITEMS, W_LIST1, W_LIST2, W_FLAG,
   W_RCACHE0,  // tree caches of the routed rule classes: W_RCACHE0 + class
   W_NSLOTS = W_RCACHE0 + MAX_RULES
 };
@@ -1980,21 +1981,23 @@ constexpr int SLOTS_ALL = 21;
 constexpr size_t SLOT_ALL_BYTES = (size_t)2 << 30;
 constexpr double SLOTS_PER_PAIR = 2.25;
 
+// Counters of a pass (run_tiles): slots and items, pairs refined at the root and at its children
+constexpr int64_t tile_counters(int64_t nbuckets) { return 16 + 5 * nbuckets; }
+
 // One pass over n adaptive pairs (T.sorted by bucket; classes R): batched levels, subtrees below,
-// weights.  cap: slots of the pool; T.flag and T.fb where pairs can be sent back.
+// weights.  cap: slots of the pool; T.flag and T.fb where pairs can be sent back.  qctr: queue
+// counters and behind them c, the pass's own; cleared: they are zero already.
 template <int N, bool HELM>
 int run_tiles(const NearQuadArgs& A, const AdapRules& R, AdapTiles T, int n, int nwaves, const KPar& kp, double* stack,
-              int* qctr, int* unc, int* over, hipStream_t s) {
+              int* qctr, bool cleared, int* unc, int* over, hipStream_t s) {
   constexpr int NP = (N + 1) * (N + 2) / 2;
   const int64_t nb = A.npatches * R.nrules;
-  int* c = wsalloc<int>(W_TCNT, 16 + 5 * nb);
-  if (!c) return -2;
+  int* c = qctr + 8 * QUEUE_STRIDE;
   T.nslot = c;
   T.nitem = c + 1;
   T.cnt1 = c + 16;
   T.cnt2 = c + 16 + nb;
-  HCHK(hipMemsetAsync(c, 0, sizeof(int) * (16 + 5 * nb), s));
-  HCHK(hipMemsetAsync(qctr, 0, sizeof(int) * 8 * QUEUE_STRIDE, s));
+  if (!cleared) HCHK(hipMemsetAsync(qctr, 0, sizeof(int) * (8 * QUEUE_STRIDE + tile_counters(nb)), s));
   // tiles of a patch's pairs at levels 0 and 1: about one per workgroup, two on large surfaces
   int64_t z = (n + 16 * nb - 1) / (16 * nb);
   if (A.npatches > 2048) z = (z + 1) / 2;
@@ -2038,20 +2041,24 @@ int run_order(const NearQuadArgs& A, NearQuadStats* st, hipStream_t s) {
   double *d_umat = TB.umat, *d_rvw = TB.rvw, *d_rvuv = TB.rvuv, *d_xg = TB.xg, *d_Pq = TB.Pq, *d_Bq = TB.Bq;
   double *d_cms = wsalloc<double>(W_CMS, 3 * npat), *d_rads = wsalloc<double>(W_RADS, npat),
          *d_epsp = wsalloc<double>(W_EPSP, npat), *d_area = wsalloc<double>(W_AREA, npat);
-  int *d_cnt = wsalloc<int>(W_CNT, npat), *d_off = wsalloc<int>(W_OFF, npat + 1),
-      *d_fill = wsalloc<int>(W_FILL, npat);
-  int *d_cls = wsalloc<int>(W_CLS, A.nnz), *d_counts = wsalloc<int>(W_COUNTS, 8);
+  // every counter that starts at zero, cleared at once (one by one the small kernels that clear them
+  // were seven of a small generation's launches): queue segments, the first pass of the adaptive
+  // pairs, list lengths, fixed-rule pairs per patch (counted, placed), adaptive pairs per bucket
+  const int nclass = A.mlp_params ? MAX_RULES : 1;
+  const int64_t nkey = nclass * npat, nzero = 8 * QUEUE_STRIDE + tile_counters(nkey) + 64 + 2 * npat + 2 * nkey;
+  int* d_zero = wsalloc<int>(W_ZERO, nzero);
+  int *d_qctr = d_zero, *d_counts = d_qctr + 8 * QUEUE_STRIDE + tile_counters(nkey), *d_cnt = d_counts + 64,
+      *d_fill = d_cnt + npat, *d_bcnt = d_fill + npat, *d_bfill = d_bcnt + nkey;
+  int *d_off = wsalloc<int>(W_OFF, npat + 1), *d_cls = wsalloc<int>(W_CLS, A.nnz);
   int2 *d_adap = wsalloc<int2>(W_ADAP, A.nnz), *d_self = wsalloc<int2>(W_SELF, A.nnz),
        *d_fixed = wsalloc<int2>(W_FIXED, A.nnz);
   int* d_nref = A.want_nref ? wsalloc<int>(W_NREF, A.nnz) : nullptr;
-  if (!d_cms || !d_rads || !d_epsp || !d_cnt || !d_off || !d_fill || !d_cls || !d_counts || !d_adap || !d_self ||
+  if (!d_cms || !d_rads || !d_epsp || !d_zero || !d_off || !d_cls || !d_adap || !d_self ||
       !d_fixed || !d_area || (A.want_nref && !d_nref)) {
     fprintf(stderr, "fmm3dbie_amd: device allocation failed in getnearquad\n");
     return -2;
   }
-  HCHK(hipMemsetAsync(d_cnt, 0, sizeof(int) * npat, s));
-  HCHK(hipMemsetAsync(d_fill, 0, sizeof(int) * npat, s));
-  HCHK(hipMemsetAsync(d_counts, 0, sizeof(int) * 8, s));
+  HCHK(hipMemsetAsync(d_zero, 0, sizeof(int) * nzero, s));
   KPar kp;
   kp.zkr = A.zk[0]; kp.zki = A.zk[1];
   kp.ar = A.alpha[0]; kp.ai = A.alpha[1];
@@ -2168,18 +2175,16 @@ int run_order(const NearQuadArgs& A, NearQuadStats* st, hipStream_t s) {
   const bool learned = A.mlp_params != nullptr && nadap > 0;
   const bool want_feat = (learned || A.feat_out) && nadap > 0;
   float* d_X = want_feat ? wsalloc<float>(W_X, (size_t)nadap * 8) : nullptr;
-  int *d_pred = nullptr, *d_boff = nullptr, *d_bcnt = nullptr, *d_pfull = nullptr, *d_qctr = nullptr;
+  int *d_pred = nullptr, *d_boff = nullptr, *d_pfull = nullptr;
   int *d_lev = nullptr, *d_seg = nullptr, *d_unc = nullptr;
   int2* d_sorted = nullptr;
   if (want_feat && !d_X) return -2;
   if (nadap > 0) {
-    d_bcnt = wsalloc<int>(W_BCNT, MLP_OUT * npat);
-    d_boff = wsalloc<int>(W_BOFF, MLP_OUT * npat + 1);
+    d_boff = wsalloc<int>(W_BOFF, nkey + 1);
     d_sorted = wsalloc<int2>(W_SORTED, 2 * (size_t)nadap);
-    d_qctr = wsalloc<int>(W_QCTR, 8 * QUEUE_STRIDE);
     if (A.lev_host) d_lev = wsalloc<int>(W_LEV, A.nnz);
     if (A.unc_host) d_unc = wsalloc<int>(W_UNC, A.nnz);
-    if (!d_bcnt || !d_boff || !d_sorted || !d_qctr || (A.lev_host && !d_lev) || (A.unc_host && !d_unc)) return -2;
+    if (!d_boff || !d_sorted || (A.lev_host && !d_lev) || (A.unc_host && !d_unc)) return -2;
   }
   if (learned) {
     d_pred = wsalloc<int>(W_PRED, nadap);
@@ -2216,12 +2221,10 @@ int run_order(const NearQuadArgs& A, NearQuadStats* st, hipStream_t s) {
     for (int c = 0; c < MAX_RULES; c++) place |= at[c] << (4 * c);
   }
   if (nadap > 0) {
-    HCHK(hipMemsetAsync(d_bcnt, 0, sizeof(int) * MLP_OUT * npat, s));
     k_bucket_count<<<(nadap + tb - 1) / tb, tb, 0, s>>>(nadap, nullptr, d_adap, d_pred, place, A.col_ind, npat, d_bcnt);
-    k_scan<<<1, 1024, 0, s>>>(MLP_OUT * npat, d_bcnt, d_boff);
-    HCHK(hipMemsetAsync(d_bcnt, 0, sizeof(int) * MLP_OUT * npat, s));
+    k_scan<<<1, 1024, 0, s>>>(nkey, d_bcnt, d_boff);
     k_bucket_scatter<<<(nadap + tb - 1) / tb, tb, 0, s>>>(nadap, nullptr, d_adap, d_pred, place, A.col_ind, npat,
-                                                          d_boff, d_bcnt, d_sorted, d_pfull);
+                                                          d_boff, d_bfill, d_sorted, d_pfull);
     HCHK(hipGetLastError());
   }
   // rules: the plain rule (P), and with a selector those of the other classes (R, class c: XG
@@ -2335,13 +2338,15 @@ int run_order(const NearQuadArgs& A, NearQuadStats* st, hipStream_t s) {
       if (!d_flag || !s2nd) return -2;
     }
     // back: counters of pairs sent back to T.fb (all, past the cap; null: none can be), zero before
+    bool cleared = true;  // the first pass's counters are
     auto pass = [&](const AdapRules& rules, int n, int2* fb, int* back) -> int {
       T.fb = fb;
       T.flag = back ? d_flag : nullptr;
       T.nfb = back;
       T.npast = back ? back + 1 : nullptr;
       if (back) HCHK(hipMemsetAsync(d_flag, 0, sizeof(int) * nadap, s));
-      const int rc = run_tiles<N, HELM>(A, rules, T, n, nwaves, kp, d_stack, d_qctr, d_unc, d_over, s);
+      const int rc = run_tiles<N, HELM>(A, rules, T, n, nwaves, kp, d_stack, d_qctr, cleared, d_unc, d_over, s);
+      cleared = false;
       if (!rc && back && (d_nref || d_lev || d_unc)) {
         k_adap_reset<<<(unsigned)((nadap + tb - 1) / tb), tb, 0, s>>>(back, fb, d_nref, d_lev, d_unc);
         HCHK(hipGetLastError());
