@@ -1254,6 +1254,29 @@ int fmm3dbie_sincos_red(int64_t n, const double* x, double* s, double* c) {
   return 0;
 }
 
+int fmm3dbie_sincos_pi(int64_t n, const double* x, double* s, double* c) {
+  for (int64_t i = 0; i < n; i++) {
+    if (!(std::fabs(x[i]) <= SINCOS_RED_MAX)) return -1;
+    sincos_pi(x[i], s[i], c[i]);
+  }
+  return 0;
+}
+
+int fmm3dbie_sincos_turns(double k, int64_t n, const double* r, double* s, double* c) {
+  double hi, lo;
+  half_turns(k, hi, lo);
+  for (int64_t i = 0; i < n; i++) {
+    if (!(std::fabs(k * r[i]) <= SINCOS_RED_MAX)) return -1;
+    bool neg;
+    sincos_turns(r[i], hi, lo, s[i], c[i], neg);
+    if (neg) {
+      s[i] = -s[i];
+      c[i] = -c[i];
+    }
+  }
+  return 0;
+}
+
 // ---------------------------------------------------------------- learned selector
 int fmm3dbie_mlp_nparam() { return MLP_NPARAM; }
 

@@ -104,20 +104,14 @@ __device__ __forceinline__ double rsqrt_halley(double x) {
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
-// sin x and cos x of the quadrature kernels, |x| <= SINCOS_RED_MAX: x = n pi + y (three-part
-// reduction as in sincos_red), then sincos_half_pi(y) and the sign of n's parity.  Near a
+// sin x and cos x of the quadrature kernels, |x| <= SINCOS_RED_MAX: sincos_pi.  Near a
 // patch k r is small: where it is within pi/2 in every lane of the wavefront, n is zero and
 // the reduction and the signs are jumped over (20 instructions instead of 34 with
 // sincos_red); the bits of a lane's result do not depend on the other lanes.
 __device__ __forceinline__ void sincos_near(double x, double& s, double& c) {
   const bool reduce = !__all(fabs(x) <= 1.5707963267948966);
   double y = x, n = 0.0;
-  if (reduce) {
-    n = rint(x * 0x1.45f306dc9c883p-2);  // 1/pi
-    y = fma(-n, 0x1.921fb54442d18p+1, x);
-    y = fma(-n, 0x1.1a62633145c07p-53, y);
-    y = fma(-n, -0x1.f1976b7ed8fbcp-109, y);
-  }
+  if (reduce) n = pi_reduce(x, y);
   sincos_half_pi(y, s, c);
   if (reduce) {
     const bool odd = (int)n & 1;

@@ -1,14 +1,15 @@
 // sin and cos of FP64 arguments of bounded size, for the Helmholtz kernel evaluations
-// (sincos_turns: far sums; sincos_half_pi: quadrature, with the reduction of sincos_near in
-// common.hpp) and for callers of the library on the host (sincos_red).
+// (sincos_turns: far sums; sincos_pi: quadrature, whose kernels take its two steps one by one in
+// sincos_near, common.hpp) and for callers of the library on the host (sincos_red, which no
+// kernel uses).
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include <cmath>
 #include <cstdint>
 
-// Largest |x| for sincos_red: n = rint(2x/pi) stays below 2^20, where the three-part
-// reduction below is accurate to rounding.  The host checks |k| times the largest
+// Largest |x| for each: n = rint(2x/pi) stays below 2^20, where the three-part reductions
+// below are accurate to rounding.  The host checks |k| times the largest
 // distance of a computation against it.
 constexpr double SINCOS_RED_MAX = 1.6e6;
 
@@ -64,8 +65,9 @@ inline void half_turns(double k, double& hi, double& lo) {
 // sin(pi y) / y and cos(pi y) are polynomials of degree 8 in y^2, minimax on [0, 1/4] (Remez
 // exchange in 300 bits; errors 1.6e-19 and 3.9e-18).  A reduction by pi needs neither the
 // swap of sine and cosine nor the quadrant signs of one by pi/2 at the same polynomial work.
-// Error against long double over k r up to 40: root mean square 1.0e-16, where sincos_red of
-// the rounded product k * r has 1.2e-15 (the product's rounding).
+// Error against 60-digit arithmetic over k r up to SINCOS_RED_MAX: at most 3.9e-16; over k r up to 40 in
+// root mean square 0.9e-16, where sincos_red of the rounded product k * r has 6.5e-16 (the product's
+// rounding).
 __host__ __device__ __forceinline__ void sincos_turns(double r, double khi, double klo, double& s, double& c,
                                                       bool& neg) {
   const double m = fma(r, khi, 0x1.8p52);
@@ -104,13 +106,13 @@ __host__ __device__ __forceinline__ void sincos_turns(double r, double khi, doub
 // 4.3e-18).
 // The coefficients are kept in scalar registers (scalar_const): as literals each costs two
 // vector moves at every use, as many instructions as the polynomials themselves.
-__device__ __forceinline__ double scalar_const(double x) {
+__host__ __device__ __forceinline__ double scalar_const(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
   asm("" : "+s"(x));
 #endif
   return x;
 }
-__device__ __forceinline__ void sincos_half_pi(double x, double& s, double& c) {
+__host__ __device__ __forceinline__ void sincos_half_pi(double x, double& s, double& c) {
   const double z = x * x;
   double ps = scalar_const(0x1.87cf34cb45316p-49);
   ps = fma(ps, z, scalar_const(-0x1.ae3f72f9ed52ap-41));
@@ -130,4 +132,23 @@ __device__ __forceinline__ void sincos_half_pi(double x, double& s, double& c) {
   pc = fma(pc, z, scalar_const(0x1.555555555541ep-5));
   pc = fma(pc, z, scalar_const(-0x1.ffffffffffffdp-2));
   c = fma(pc, z, 1.0);
+}
+
+// x = n pi + y, |y| <= pi/2 (the rounding of x / pi aside), |x| <= SINCOS_RED_MAX: returns n.  Three-part
+// reduction as in sincos_red.
+__host__ __device__ __forceinline__ double pi_reduce(double x, double& y) {
+  const double n = rint(x * 0x1.45f306dc9c883p-2);  // 1/pi
+  y = fma(-n, 0x1.921fb54442d18p+1, x);
+  y = fma(-n, 0x1.1a62633145c07p-53, y);
+  y = fma(-n, -0x1.f1976b7ed8fbcp-109, y);
+  return n;
+}
+
+// sin x and cos x for |x| <= SINCOS_RED_MAX: pi_reduce, sincos_half_pi and the sign of n's parity.
+__host__ __device__ __forceinline__ void sincos_pi(double x, double& s, double& c) {
+  double y;
+  const bool odd = (int)pi_reduce(x, y) & 1;
+  sincos_half_pi(y, s, c);
+  s = odd ? -s : s;
+  c = odd ? -c : c;
 }

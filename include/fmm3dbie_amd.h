@@ -215,9 +215,12 @@ int fmm3dbie_rv_umat(int norder, double *umat);
 void fmm3dbie_koorn_pols(double u, double v, int nmax, double *pols);
 /* src/tria_routs/triasymq.f:89-158  triasymq on the simplex: returns the node count */
 int fmm3dbie_xg_rule(int deg, double *uvs, double *wts);
-/* No reference counterpart: sine and cosine for |x| <= 1.6e6, the range of the Helmholtz
- * kernel evaluations, on the host; returns -1 beyond that. */
+/* No reference counterpart: sine and cosine for |x| <= 1.6e6 on the host; return -1 beyond that.
+ * _pi and _turns are the functions that the Helmholtz kernels evaluate: _pi in the quadrature,
+ * _turns (of k r[i], the product not rounded) in the far sums.  No kernel uses _red. */
 int fmm3dbie_sincos_red(int64_t n, const double *x, double *s, double *c);
+int fmm3dbie_sincos_pi(int64_t n, const double *x, double *s, double *c);
+int fmm3dbie_sincos_turns(double k, int64_t n, const double *r, double *s, double *c);
 
 /* ---- device-pointer interface (inputs resident in HBM, caller's stream) -------------- */
 /* No single reference counterpart: the same computations as the entries above with

@@ -119,8 +119,8 @@ def test_setup_passes_the_complex_wavenumber_to_the_far_order():
 
 
 def test_bounded_sincos_matches_libm():
-    """sin and cos of the Helmholtz kernel evaluations (three-part Cody-Waite reduction by
-    pi/2 and Taylor polynomials, evaluated on the host through the library): within 2.3e-16
+    """The library's bounded-range sin and cos for callers on the host (three-part Cody-Waite
+    reduction by pi/2 and Taylor polynomials; the kernels' own are tested below): within 2.3e-16
     of libm on random arguments up to the 1.6e6 bound and next to multiples of pi/2, where
     the reduction cancels; arguments beyond the bound are refused."""
     import math
@@ -141,3 +141,77 @@ def test_bounded_sincos_matches_libm():
     assert np.array_equal(sn, -s) and np.array_equal(cn, c)
     bad = np.array([2e6])
     assert L.fmm3dbie_sincos_red(1, p(bad), p(s), p(c)) == -1
+
+
+def test_quadrature_sincos_matches_libm():
+    """sin and cos of the quadrature kernels (reduction by pi, minimax polynomials, on the host
+    through the library) within 3e-16 of libm (libm half a unit, 1.1e-16; the last addition's rounding
+    the same, the polynomials' and the reduction's a quarter each) over +-1.6e6, next to multiples of
+    pi/2 and below pi/2, where the kernels skip the reduction."""
+    import math
+    from fmm3dbie_amd import lib
+    L = lib()
+    rng = np.random.default_rng(2)
+    k = np.arange(-3000, 3000) * (math.pi / 2)
+    x = np.concatenate([rng.uniform(-1.6, 1.6, 20000), rng.uniform(-1e3, 1e3, 20000), rng.uniform(-1.6e6, 1.6e6, 20000),
+                        k, np.nextafter(k, np.inf), np.nextafter(k, -np.inf), [0.0, -0.0, 1e-300, 1.6e6]])
+    s, c = np.zeros_like(x), np.zeros_like(x)
+    p = lambda a: C.c_void_p(a.ctypes.data)
+    assert L.fmm3dbie_sincos_pi(len(x), p(x), p(s), p(c)) == 0
+    assert np.abs(s - np.sin(x)).max() <= 3e-16 and np.abs(c - np.cos(x)).max() <= 3e-16
+    # relative accuracy where sin is small (its kernels divide by k r)
+    t = np.abs(x) < 1e-3
+    assert np.abs(s[t] - np.sin(x[t])).max() <= 3e-16 * 1e-3
+    xn, sn, cn = -x, np.zeros_like(x), np.zeros_like(x)
+    assert L.fmm3dbie_sincos_pi(len(x), p(xn), p(sn), p(cn)) == 0
+    assert np.array_equal(sn, -s) and np.array_equal(cn, c)
+    bad = np.array([2e6])
+    assert L.fmm3dbie_sincos_pi(1, p(bad), p(s), p(c)) == -1
+
+
+def _sincos_exact(k, r):
+    """sin(k r) and cos(k r) of the exact product, in 60-digit arithmetic, rounded to double."""
+    from decimal import Decimal, getcontext
+    getcontext().prec = 60
+    pi = Decimal("3.14159265358979323846264338327950288419716939937510582097494459230781640628620899")
+    out = []
+    for v in r:
+        x = Decimal(float(k)) * Decimal(float(v))
+        n = (x / pi).to_integral_value()
+        y = x - n * pi
+        s, c, ts, tc = Decimal(0), Decimal(0), y, Decimal(1)
+        for m in range(1, 25):
+            s, c = s + ts, c + tc
+            ts = -ts * y * y / (2 * m * (2 * m + 1))
+            tc = -tc * y * y / ((2 * m - 1) * (2 * m))
+        sign = -1 if int(n) % 2 else 1
+        out.append((float(sign * s), float(sign * c)))
+    return np.array(out).T
+
+
+def test_far_sum_sincos_matches_60_digits():
+    """sin and cos of k r in the far sums (reduction in half turns with k / pi as two doubles, minimax
+    polynomials, on the host through the library), of the exact product k r: within 4.5e-16 (four
+    roundings: of the reduced argument, the polynomial, the result and the reference) up to k r = 1.6e6, for k of either sign, at
+    products next to multiples of pi/2 and at r = 0."""
+    import math
+    from fmm3dbie_amd import lib
+    L = lib()
+    rng = np.random.default_rng(3)
+    p = lambda a: C.c_void_p(a.ctypes.data)
+    for k in (1.0, -4.0, 10.123, 0.037, 1234.5):
+        near = np.arange(-200, 4000, 7) * (math.pi / 2) / k
+        r = np.concatenate([rng.uniform(0, 40, 400), rng.uniform(0, 1e3, 400), rng.uniform(0, 1.6e6, 400)]) / abs(k)
+        r = np.concatenate([r, np.abs(near), np.nextafter(np.abs(near), 1e9), [0.0, 1e-300]])
+        s, c = np.zeros_like(r), np.zeros_like(r)
+        assert L.fmm3dbie_sincos_turns(k, len(r), p(r), p(s), p(c)) == 0
+        es, ec = _sincos_exact(k, r)
+        assert np.abs(s - es).max() <= 4.5e-16 and np.abs(c - ec).max() <= 4.5e-16
+        # relative to the sine where it is small
+        t = np.abs(k * r) < 1e-3
+        assert np.abs(s[t] - es[t]).max() <= 4e-16 * 1e-3
+        sn, cn = np.zeros_like(r), np.zeros_like(r)
+        assert L.fmm3dbie_sincos_turns(-k, len(r), p(r), p(sn), p(cn)) == 0
+        assert np.array_equal(sn, -s) and np.array_equal(cn, c)
+    bad = np.array([2e6])
+    assert L.fmm3dbie_sincos_turns(1.0, 1, p(bad), p(s), p(c)) == -1

@@ -11,15 +11,13 @@ pytestmark = pytest.mark.gpu
 def _over(g, P, sig):
     """sigma_over * w at the oversampled nodes, (nrhs, nptso)."""
     from fmm3dbie_amd import basis
-    no = int(g["norders"][0])
-    p = len(basis.rv_nodes(no)[1])
-    um = basis.rv_umat(no)
     over = np.zeros((len(sig), len(P["whtsover"])), complex)
     for ip, nv in enumerate(P["novers"]):
+        no = int(g["norders"][ip])
         uv, _ = basis.rv_nodes(int(nv))
-        im = np.stack([basis.koorn_pols(u, v, no) for u, v in uv]) @ um
+        im = np.stack([basis.koorn_pols(u, v, no) for u, v in uv]) @ basis.rv_umat(no)
         a, b = P["ixyzso"][ip] - 1, P["ixyzso"][ip + 1] - 1
-        over[:, a:b] = sig[:, ip * p:(ip + 1) * p] @ im.T
+        over[:, a:b] = sig[:, g["ixyzs"][ip] - 1:g["ixyzs"][ip + 1] - 1] @ im.T
     return over * P["whtsover"]
 
 
@@ -88,6 +86,64 @@ def test_far_sum_forms_match_a_64_bit_sum(cuda, helm, pars, norder):
             out = np.atleast_2d(plan.apply(sp.contiguous(), prec, mode).cpu().numpy())
             err = np.linalg.norm(out - ref[:nrhs]) / np.linalg.norm(size[:nrhs])
             assert err < 30 * unit, (nrhs, prec, mode, err / unit)
+    plan.close()
+
+
+def _mixed_sphere(na, orders):
+    """A sphere whose patches alternate between the orders."""
+    from fmm3dbie_amd import geometry as G
+    gs = [G.get_sphere_npat(1.0, na, (0, 0, 0), n) for n in orders]
+    npat = len(gs[0]["norders"])
+    pick = [gs[ip % len(gs)] for ip in range(npat)]
+    rows = [slice(q["ixyzs"][ip] - 1, q["ixyzs"][ip + 1] - 1) for ip, q in enumerate(pick)]
+    g = dict(gs[0])
+    g["norders"] = np.array([q["norders"][ip] for ip, q in enumerate(pick)])
+    g["iptype"] = np.array([q["iptype"][ip] for ip, q in enumerate(pick)])
+    g["ixyzs"] = np.cumsum([1] + [r.stop - r.start for r in rows])
+    for key in ("srcvals", "srccoefs"):
+        g[key] = np.concatenate([q[key][r] for q, r in zip(pick, rows)])
+    return g
+
+
+# patches of several orders: the general CSR kernel, the near subtraction as a kernel of its own, the
+# reduction over source splits on its own, interpolation matrices by patch
+@pytest.mark.parametrize("helm,pars,orders", [(True, (2.0, 2.0j, 1.0), (3, 4)), (False, (1.0, 0.5), (2, 5, 3)),
+                                              (True, (2.0 + 0.5j, 1.0, 1.0j), (4, 3))])
+def test_patches_of_several_orders(cuda, helm, pars, orders):
+    import torch
+    from fmm3dbie_amd import layer, problem
+    g = _mixed_sphere(2, orders)
+    pars = np.array(pars)
+    P = problem.setup(g, 1e-6, helm, pars, nover_fixed=5)
+    rng = np.random.default_rng(8)
+    # (of the size of quadrature weights)
+    w = 1e-3 * rng.standard_normal(P["nquad"])
+    if helm:
+        w = w + 1e-3j * rng.standard_normal(P["nquad"])
+    plan = layer.ApplyPlan(g, helm, pars, P["row_ptr"], P["col_ind"], P["iquad"], w, P["novers"], P["ixyzso"],
+                           P["srcover"], P["whtsover"])
+    assert plan.info()[3] == 0  # no uniform patch size
+    N = len(g["srcvals"])
+    S = rng.standard_normal((17, N)) + 1j * rng.standard_normal((17, N))
+    ref, size_far, size_all = _sum64(g, P, helm, pars, S)
+    near, size_near = np.zeros_like(ref), np.zeros(ref.shape)
+    for i in range(N):
+        for j in range(P["row_ptr"][i] - 1, P["row_ptr"][i + 1] - 1):
+            ip = P["col_ind"][j] - 1
+            wj = w[P["iquad"][j] - 1:P["iquad"][j + 1] - 1]
+            sj = S[:, g["ixyzs"][ip] - 1:g["ixyzs"][ip + 1] - 1]
+            near[:, i] += sj @ wj
+            size_near[:, i] += np.abs(sj) @ np.abs(wj)
+    ref = ref + near
+    for nrhs in (1, 3, 8, 17):
+        s = torch.as_tensor(S[:nrhs], device=cuda)
+        s = s[0] if nrhs == 1 else s
+        for prec, mode, unit, size in ((64, 1, 2.0 ** -53, size_far), (64, 0, 2.0 ** -53, size_all),
+                                       (32, 1, 2.0 ** -24, size_far)):
+            sp = s if prec == 64 else s.to(torch.complex64)
+            out = np.atleast_2d(plan.apply(sp.contiguous(), prec, mode).cpu().numpy())
+            err = np.linalg.norm(out - ref[:nrhs]) / np.linalg.norm(size[:nrhs] + size_near[:nrhs])
+            assert err < 30 * unit, (nrhs, prec, mode, err / unit)  # the bound above
     plan.close()
 
 
