@@ -148,9 +148,9 @@ def test_patches_of_several_orders(cuda, helm, pars, orders):
 
 
 # densities far down FP32's range at a long wavelength: the unit in which a plan stores its coordinates
-# must not enter the strengths (k / (2 pi) squared is 2.5e-10 here, which would leave them 1e-42), nor
+# must not enter the strengths or a product with them (k / (2 pi) is 1.6e-5 here, the strengths 2e-36), nor
 # the smallest value of the terms of the split products (strengths of 2e-35 here); and far up
-@pytest.mark.parametrize("nrhs,size", [(1, 1e-31), (3, 1e-31), (8, 1e-31), (9, 1e-33), (16, 1e-33), (17, 1e-33),
+@pytest.mark.parametrize("nrhs,size", [(1, 1e-34), (3, 1e-34), (8, 1e-34), (9, 1e-33), (16, 1e-33), (17, 1e-33),
                                        (33, 1e-33), (64, 1e-33), (16, 1e36), (64, 1e36)])
 def test_densities_of_extreme_size_at_a_long_wavelength(cuda, nrhs, size):
     import torch
