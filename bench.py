@@ -117,8 +117,8 @@ def main():
     ap.add_argument("--batched-sequential", type=int, default=8,
                     help="FP64 single-RHS solves timed for the batched comparison")
     ap.add_argument("--apply-only", action="store_true",
-                    help="only the near quadrature once, then 5 FP64 (add/subtract), 5 FP32 (masked) and 5 16-RHS FP32 applies "
-                         "of the workload (for the apply's rocprofv3 counters)")
+                    help="only the near quadrature once, then 5 applies each of one FP64 (add/subtract), one FP32 (masked), "
+                         "16 and 64 FP32 and 16 FP64 densities of the workload (for the apply's rocprofv3 counters)")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="only run a 1 GiB device read + 1 GiB write (torch.neg) for HBM counter scaling")
     args = ap.parse_args()
@@ -384,9 +384,9 @@ def _timed(fn):
 
 def apply_only(g, helm, pars, P, nq, dev):
     """5 FP64 applies in the reference's add/subtract algebra, 5 FP32 masked applies of a
-    random density and 5 FP32 masked applies of 16 random densities (the far sum on the
+    random density, 5 of 16 and of 64 in FP32 and 5 of 16 in FP64 (the far sum on the
     matrix cores), with the per-phase HIP-event times (ms): oversampling, far sum, split
-    sum + CSR correction, subtraction."""
+    sum + CSR correction (in the add/subtract form with the subtraction)."""
     import torch
     from fmm3dbie_amd import layer
     w = nq.run()
@@ -396,10 +396,11 @@ def apply_only(g, helm, pars, P, nq, dev):
     rng = np.random.default_rng(0)
     sig = torch.as_tensor(rng.standard_normal(npts) + 1j * rng.standard_normal(npts), device=dev)
     out = {"workload_points": npts, "oversampled_sources": nptso, "nnz": P["nnz"], "nquad": P["nquad"]}
-    sig16 = torch.as_tensor(rng.standard_normal((16, npts)) + 1j * rng.standard_normal((16, npts)),
-                            device=dev).to(torch.complex64)
+    sig64 = torch.as_tensor(rng.standard_normal((64, npts)) + 1j * rng.standard_normal((64, npts)), device=dev)
     for name, prec, mode, s in (("fp64_addsub", 64, 0, sig), ("fp32_masked", 32, 1, sig.to(torch.complex64)),
-                                ("fp32_masked_16rhs", 32, 1, sig16)):
+                                ("fp32_masked_16rhs", 32, 1, sig64[:16].to(torch.complex64)),
+                                ("fp32_masked_64rhs", 32, 1, sig64.to(torch.complex64)),
+                                ("fp64_masked_16rhs", 64, 1, sig64[:16].contiguous())):
         tm = np.zeros(4)
         acc = []
         plan.apply(s, prec, mode)
@@ -407,7 +408,7 @@ def apply_only(g, helm, pars, P, nq, dev):
             plan.apply(s, prec, mode, times=tm)
             acc.append(tm.copy())
         torch.cuda.synchronize()
-        out[name + "_ms"] = dict(zip(("oversample", "far", "csr", "subtract"), np.mean(acc, axis=0).tolist()))
+        out[name + "_ms"] = dict(zip(("oversample", "far", "csr"), np.mean(acc, axis=0).tolist()))
     plan.close()
     return out
 

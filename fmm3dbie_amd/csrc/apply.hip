@@ -227,12 +227,12 @@ struct NearCursor {
 // Every lane works on the same source, whose geometry and strengths are wave-uniform: they
 // come by scalar loads into scalar registers, and one operand of each vector instruction
 // may be one of those, so that no LDS, barrier or vector register is spent on them.
-// Bound by vector instruction issue: a pair takes 58 instructions in FP64 with a real
-// wavenumber (76 with a charge and a dipole strength per source, sincos_red and a Newton
-// step more; 262 against 330 cycles of a SIMD per 64 pairs; the add/subtract apply of 344064
-// points 412 -> 337 ms, of 25920 points 4.44 -> 3.55 ms), 20 for Laplace (which ran the
-// Helmholtz kernel with k = 0: 106 against 330 cycles) and 26 in FP32 (91 against 103
-// cycles: 1.95 -> 1.85 ms for 43008 points), three of them hardware functions of 10 cycles.
+// Bound by vector instruction issue: a pair takes 61 instructions in the add/subtract form of FP64
+// with a real wavenumber (counted; 76 with a charge and a dipole strength per source, sincos_red
+// and a Newton step more; 266 cycles of a SIMD per 64 pairs, before 330; the apply of 344064
+// points 412 -> 337 ms, of 25920 points 4.44 -> 3.55 ms) and 27.5 in FP32 (93 cycles, before 103:
+// 1.95 -> 1.85 ms for 43008 points), three of them hardware functions of 10 cycles.  Laplace,
+// which ran the Helmholtz kernel with k = 0, takes 117 cycles in FP64 and 65 in FP32.
 // MASK: sources of the target's near patches are skipped; tiles of STILE sources that hold
 // none for any lane of the wavefront (nearly all) run without a test.
 // !MASK: sources within thresh of the target are skipped: each pair is compared, and only
@@ -295,7 +295,8 @@ __global__ void __launch_bounds__(64) k_farsum(int ntarg, const T* __restrict__ 
     return r2;
   };
   if constexpr (MASK) {
-    constexpr int UN = sizeof(T) == 8 ? 2 : 1;  // FP64: 262 against 295 cycles per 64 pairs; FP32: 98 against 95
+    // unrolled by 2 against rolled, cycles per 64 pairs: FP64 262 and 295, FP32 98 and 95
+    constexpr int UN = sizeof(T) == 8 ? 2 : 1;
     NearCursor nc{near_sorted, ixyzso};
     if (act && jbeg < jend) {
       nc.ptr = row_ptr[i] - 1;
@@ -473,7 +474,9 @@ __global__ void __launch_bounds__(64 * FW)
 // computed once for all groups, and the products run in bfloat16, where the matrix cores have
 // sixteen times their FP32 rate, exact products and FP32 sums: each value is split into three
 // bfloat16 terms (hi + mid + lo, rounded to nearest, is the FP32 value to its last bit), and six
-// products of terms take the place of one (those left out are below 2^-26 of it).
+// products of terms take the place of one (those left out are below 2^-26 of it), as in Henry, Tang
+// and Heinecke, Leveraging the bfloat16 artificial intelligence datatype for higher-precision
+// computations, ARITH 2019.
 // A wavefront takes MT tiles of 16 targets; in a tile of ST = 32 sources lane l evaluates the pairs
 // (target l % 16, sources 8 (l / 16) ..) on the vector units, which are the operand of the 16x16x32
 // products as they stand.  The workgroup stages the sources' geometry and the split strengths in
@@ -488,10 +491,10 @@ __global__ void __launch_bounds__(64 * FW)
 // of a chain downwards, which over all sources would add up (error of the 64-density apply below
 // against the FP64 one 3.1e-6; 3.8e-7 in this way).  Re K Re s and Im K Im s have a sum each,
 // which costs less than to negate an operand.
-// Bound by issue: per 64 pairs and group 48 x 4.5 cycles of products, 35 instructions of kernel
-// values and splits per pair, and the staging, which MT = 2 tiles share.  The apply of 86016
-// points (139206 sources): 16 densities 15.1 ms, 32 21.8, 48 28.9, 64 33.0; in FP32 products, a group
-// at a time, 19.3 ms for each 16.
+// Bound by issue: per 64 pairs 3 matrix and 39 vector instructions with one group, 12 and 52 with
+// four (kernel values and splits, sums, and the staging, which MT = 2 tiles share): 184 and 381
+// cycles of a SIMD.  The apply of 86016 points (139206 sources): 16 densities 15.4 ms, 32 22.8, 48
+// 30.6, 64 34.8; in FP32 products, a group at a time, 19.3 ms for each 16.
 typedef float flt2 __attribute__((ext_vector_type(2)));
 typedef float flt4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
@@ -1388,8 +1391,11 @@ static int default_group(int nrhs) {
 }
 
 // Right-hand sides per far-sum group, tuned or default; a last group is padded with zeros.  Measured
-// in cycles of a SIMD per 64 pairs (43008 x 70000 pairs, Helmholtz): FP64 262 / 280 / 316 for
-// 1, 2 and 4 densities and 466 for 16; FP32 98 / 110 / 140 and 217.  str_cap: strengths
+// in cycles of a SIMD per 64 pairs (43008 x 69120 pairs, Helmholtz): FP64 268 / 289 / 325 / 409
+// for 1, 2, 4 and 8 densities and 528 for each 16 (a group of 8 is the cheaper one for 5 to 8
+// densities, and two of them, 818, the dearer for 9 to 16); FP32 93 / 107 / 140 / 208 and 190 for 16,
+// 401 for 64.  Laplace: FP64 117 / 118 / 145 / 203 and 257; FP32 65 / 71 / 82 / 121 and 114, 262.
+// str_cap: strengths
 // (complex values) that fit the buffer of the call; a padded block that does not falls back
 // to a group that divides nrhs.
 static int far_group(const ApplyPlan* P, int nrhs, int prec, int64_t str_cap, int64_t* wg) {
